@@ -28,6 +28,7 @@
 
 #include "radio_device.hpp"
 #include "radio_launch.hpp"
+#include "radio_pair_fast.hpp"
 #include "../runtime.hpp"
 
 namespace c8mi::radio {
@@ -82,49 +83,18 @@ __device__ __forceinline__ double doppler(double index, V3 beta, V3 emit) {
   return (1. - product) - perr;
 }
 
-// ---- arithmetic of the two precision modes --------------------------------
+// ---- exact arithmetic ---------------------------------------------------------
 //
-// Exact: the reference's FP64 expressions in its operation order (correctly
-// rounded IEEE division and square root, no contraction): the fixed-point
-// waveforms equal the FP64 restatement's bit for bit.
-// Fast: FP64 throughout, but every division and square root of the pair loop
-// becomes a hardware reciprocal / reciprocal square root refined by two Newton
-// steps (about one ulp), and the inverse distance is shared by the emission
-// direction and the amplitudes. Arrival times must stay at FP64 accuracy: an
-// endpoint sample is a spike in one bin, and a delay error of even 1e-15 s at
-// 15 km (an FP32 refractivity ratio) moves a few samples per million across a
-// bin edge, which shows up as per-bin errors of order 1e-3.
-
-__device__ __forceinline__ double recip_fast(double b) {
-  double const r0 = __builtin_amdgcn_rcp(b);
-  double e = fma(-b, r0, 1.);
-  double r = fma(r0, e, r0);
-  e = fma(-b, r, 1.);
-  r = fma(r, e, r);
-  // 0 and +-inf: keep the hardware result (+-inf, +-0) instead of NaN.
-  return isfinite(r0) && r0 != 0. ? r : r0;
-}
-
-// Returns sqrt(x) and 1/sqrt(x) for x > 0 (NaN propagates).
-__device__ __forceinline__ double rsqrt_fast(double x, double& root) {
-  double y = __builtin_amdgcn_rsq(x);
-  double h = x * y;
-  double e = fma(-h, y, 1.);
-  y = fma(0.5 * y, e, y);
-  h = x * y;
-  e = fma(-h, y, 1.);
-  y = fma(0.5 * y, e, y);
-  root = x * y;
-  return y;
-}
+// The reference's FP64 expressions in its operation order (correctly rounded
+// IEEE division and square root, no contraction): the fixed-point waveforms
+// equal the FP64 restatement's bit for bit. The fast form of the same updates
+// is in radio_pair_fast.hpp.
 
 struct Track {
   V3 start, end, disp, beta;
   double t0, t1, duration, length, beta_module, constant;
-  double inv_beta_module;  // fast mode only
 };
 
-template <bool Exact>
 __device__ __forceinline__ bool load_track(double const* __restrict__ tracks,
                                            std::uint64_t stride, std::uint64_t i, Track& t) {
   t.start = {tracks[i], tracks[stride + i], tracks[2 * stride + i]};
@@ -134,21 +104,10 @@ __device__ __forceinline__ bool load_track(double const* __restrict__ tracks,
   double const signed_weight = tracks[8 * stride + i];
   t.duration = t.t1 - t.t0;
   t.disp = vsub(t.end, t.start);
-  if constexpr (Exact) {
-    t.length = sqrt(vdot(t.disp, t.disp));
-    if (!(t.duration > 0.) || !(t.length > 0.)) return false;
-    t.beta = vdiv(t.disp, kC * t.duration);
-    t.beta_module = t.length / (kC * t.duration);
-  } else {
-    double const l2 = fma(t.disp.x, t.disp.x, fma(t.disp.y, t.disp.y, t.disp.z * t.disp.z));
-    if (!(t.duration > 0.) || !(l2 > 0.)) return false;
-    double const inv_length = rsqrt_fast(l2, t.length);
-    double const c_duration = kC * t.duration;
-    double const inv_c_duration = recip_fast(c_duration);
-    t.beta = vmul(t.disp, inv_c_duration);
-    t.beta_module = t.length * inv_c_duration;
-    t.inv_beta_module = c_duration * inv_length;
-  }
+  t.length = sqrt(vdot(t.disp, t.disp));
+  if (!(t.duration > 0.) || !(t.length > 0.)) return false;
+  t.beta = vdiv(t.disp, kC * t.duration);
+  t.beta_module = t.length / (kC * t.duration);
   t.constant = kChargeEm * signed_weight;
   return true;
 }
@@ -157,7 +116,7 @@ __device__ __forceinline__ bool load_track(double const* __restrict__ tracks,
 // thread with the same expressions propagate() and add_sample() use.
 struct Obs {
   V3 position;
-  double start, duration, rate, grid, wavelength, two_pi_over_wavelength;
+  double start, duration, rate, grid, wavelength;
   double nbins_d;
   std::int32_t nbins;
   std::uint64_t offset;
@@ -168,27 +127,18 @@ struct Obs {
 
 struct Path {
   double time, n_source, n_destination, distance;
-  double inv_distance;  // fast mode only
   V3 emit;
 };
 
-template <bool Exact>
 __device__ __forceinline__ Path propagate(PropagationDev const& p, V3 source, Obs const& o) {
   Path r;
   V3 const disp = vsub(o.position, source);
-  if constexpr (Exact) {
-    r.distance = sqrt(vdot(disp, disp));
-    r.emit = vdiv(disp, r.distance);
-  } else {
-    double const r2 = fma(disp.x, disp.x, fma(disp.y, disp.y, disp.z * disp.z));
-    r.inv_distance = rsqrt_fast(r2, r.distance);
-    r.emit = vmul(disp, r.inv_distance);
-  }
+  r.distance = sqrt(vdot(disp, disp));
+  r.emit = vdiv(disp, r.distance);
   double const distance = r.distance;
   if (p.homogeneous_index > 0.) {
     double const index = p.homogeneous_index;
-    if constexpr (Exact) r.time = index * distance / kC;
-    else r.time = index * distance * (1. / kC);
+    r.time = index * distance / kC;
     r.n_source = index;
     r.n_destination = index;
     return r;
@@ -226,12 +176,7 @@ __device__ __forceinline__ Path propagate(PropagationDev const& p, V3 source, Ob
     n_destination = 1.;
     height = destination_height - fabs(source_height);
   }
-  if constexpr (Exact) {
-    r.time = (1. + (integrated_source - o.integrated_destination) / height) * distance / kC;
-  } else {
-    double const ratio = (integrated_source - o.integrated_destination) * recip_fast(height);
-    r.time = (1. + ratio) * (distance * (1. / kC));
-  }
+  r.time = (1. + (integrated_source - o.integrated_destination) / height) * distance / kC;
   r.n_source = n_source;
   r.n_destination = n_destination;
   return r;
@@ -379,19 +324,11 @@ __device__ __forceinline__ void add_potential_sample(Obs const& o, double scale,
   tally.overflow += valid ? 0ull : n;
 }
 
-// separate_same_bin_endpoints (RadioProjection.inl:303-336); `to_bins` is the
-// reference's division by the grid (exact) or the product with the rate (fast).
-template <bool Exact>
-__device__ __forceinline__ double to_bins(double time, Obs const& o) {
-  if constexpr (Exact) return time / o.grid;
-  else return time * o.rate;
-}
-
-template <bool Exact>
+// separate_same_bin_endpoints (RadioProjection.inl:303-336).
 __device__ __forceinline__ void separate_same_bin(double& start_time, double& end_time,
                                                   Obs const& o, bool signed_order) {
-  double const s = to_bins<Exact>(start_time, o);
-  double const e = to_bins<Exact>(end_time, o);
+  double const s = start_time / o.grid;
+  double const e = end_time / o.grid;
   if (static_cast<long long>(nearest_bin(s)) != static_cast<long long>(nearest_bin(e))) return;
   double const grid = o.grid;
   double const sf = s - floor(s);
@@ -411,18 +348,16 @@ __device__ __forceinline__ void separate_same_bin(double& start_time, double& en
 }
 
 // t.constant * rate / (doppler * R)
-template <bool Exact>
 __device__ __forceinline__ double field_scale(Track const& t, Obs const& o, double doppler_factor,
                                               Path const& path) {
-  if constexpr (Exact) return t.constant * o.rate / (doppler_factor * path.distance);
-  else return (t.constant * o.rate) * path.inv_distance * recip_fast(doppler_factor);
+  return t.constant * o.rate / (doppler_factor * path.distance);
 }
 
-template <bool Exact, bool Fixed>
+template <bool Fixed>
 __device__ __forceinline__ void coreas_pair(Track const& t, PropagationDev const& p, Obs const& o,
                             double scale, Tile<Fixed> const& tile, Tally& tally) {
-  Path const ps = propagate<Exact>(p, t.start, o);
-  Path const pe = propagate<Exact>(p, t.end, o);
+  Path const ps = propagate(p, t.start, o);
+  Path const pe = propagate(p, t.end, o);
   double const pre = doppler(ps.n_source, t.beta, ps.emit);
   double const post = doppler(pe.n_source, t.beta, pe.emit);
   double start_receive = t.t0 + ps.time;
@@ -431,15 +366,14 @@ __device__ __forceinline__ void coreas_pair(Track const& t, PropagationDev const
       (fabs(pre) < kCoreasThreshold || fabs(post) < kCoreasThreshold)) {
     V3 const midpoint = vmul(vadd(t.start, t.end), 0.5);
     double const middle_time = (t.t0 + t.t1) * 0.5;
-    Path const pm = propagate<Exact>(p, midpoint, o);
+    Path const pm = propagate(p, midpoint, o);
     double const middle_receive = middle_time + pm.time;
     double const md = doppler(pm.n_source, t.beta, pm.emit);
     V3 field_start =
-        vmul(vcross(pm.emit, vcross(pm.emit, t.beta)), field_scale<Exact>(t, o, md, pm));
+        vmul(vcross(pm.emit, vcross(pm.emit, t.beta)), field_scale(t, o, md, pm));
     V3 field_end = vmul(field_start, -1.);
     double delta;
-    if constexpr (Exact) delta = t.length / (kC * t.beta_module) * fabs(md);
-    else delta = t.duration * fabs(md);  // length / (c beta) is the duration
+    delta = t.length / (kC * t.beta_module) * fabs(md);
     if (start_receive < end_receive) {
       start_receive = middle_receive - 0.5 * delta;
       end_receive = middle_receive + 0.5 * delta;
@@ -449,33 +383,33 @@ __device__ __forceinline__ void coreas_pair(Track const& t, PropagationDev const
     }
     delta = end_receive - start_receive;
     if (fabs(delta) < o.grid) {
-      double const shrink = fabs(to_bins<Exact>(delta, o));
+      double const shrink = fabs(delta / o.grid);
       field_start = vmul(field_start, shrink);
       field_end = vmul(field_end, shrink);
-      separate_same_bin<Exact>(start_receive, end_receive, o, true);
+      separate_same_bin(start_receive, end_receive, o, true);
     }
     add_field_sample(o, scale, tile, start_receive, field_start, tally);
     add_field_sample(o, scale, tile, end_receive, field_end, tally);
     return;
   }
   V3 field_start =
-      vmul(vcross(ps.emit, vcross(ps.emit, t.beta)), field_scale<Exact>(t, o, pre, ps));
+      vmul(vcross(ps.emit, vcross(ps.emit, t.beta)), field_scale(t, o, pre, ps));
   V3 field_end =
-      vmul(vcross(pe.emit, vcross(pe.emit, t.beta)), -field_scale<Exact>(t, o, post, pe));
+      vmul(vcross(pe.emit, vcross(pe.emit, t.beta)), -field_scale(t, o, post, pe));
   if (pre < 1.e-9 || post < 1.e-9) {
     double const delta = end_receive - start_receive;
     if (fabs(delta) < o.grid) {
-      double const shrink = fabs(to_bins<Exact>(delta, o));
+      double const shrink = fabs(delta / o.grid);
       field_start = vmul(field_start, shrink);
       field_end = vmul(field_end, shrink);
-      separate_same_bin<Exact>(start_receive, end_receive, o, false);
+      separate_same_bin(start_receive, end_receive, o, false);
     }
   }
   add_field_sample(o, scale, tile, start_receive, field_start, tally);
   add_field_sample(o, scale, tile, end_receive, field_end, tally);
 }
 
-template <bool Exact, bool Fixed>
+template <bool Fixed>
 __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double time2, Track const& t,
                             PropagationDev const& p, Obs const& o, double scale,
                             Tile<Fixed> const& tile, Tally& tally, bool subdivided,
@@ -483,7 +417,7 @@ __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double t
   // The cached path travels by value: a pointer to the caller's local would
   // pin it to scratch memory.
   Path const path = use_cached ? cached_midpoint_path
-                               : propagate<Exact>(p, vmul(vadd(p1, p2), 0.5), o);
+                               : propagate(p, vmul(vadd(p1, p2), 0.5), o);
   double const n_source = path.n_source;
   double const bk = vdot(t.beta, path.emit);
   double const middle_time = (time1 + time2) * 0.5;
@@ -500,24 +434,14 @@ __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double t
   double const end_bin = floor((d2 - o.start) * o.rate + 0.5);
   V3 const bperp = vcross(path.emit, vcross(t.beta, path.emit));
   double const den = 1. - n_source * bk;
-  // constant / (den * R)
-  double k;
-  if constexpr (Exact) k = 0.;  // divisions below keep the reference's form
-  else k = t.constant * path.inv_distance * recip_fast(den);
   if (start_bin == end_bin) {
     V3 potential;
     if (fabs(den) > 1.e-15) {
       double const fraction = fabs(d2 * o.rate - d1 * o.rate);
-      if constexpr (Exact)
-        potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
-      else
-        potential = vmul(bperp, sign * k * fraction);
+      potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
     } else {
       double const fraction = (time2 - time1) * o.rate;
-      if constexpr (Exact)
-        potential = vmul(bperp, sign * t.constant * fraction / path.distance);
-      else
-        potential = vmul(bperp, sign * t.constant * fraction * path.inv_distance);
+      potential = vmul(bperp, sign * t.constant * fraction / path.distance);
     }
     add_potential_sample(o, scale, tile, d2, potential, tally);
     return;
@@ -525,27 +449,14 @@ __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double t
   int const nb = static_cast<int>(end_bin - start_bin);
   double fraction = fabs(start_bin + 0.5 - x1);
   V3 potential;
-  if constexpr (Exact)
-    potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
-  else
-    potential = vmul(bperp, sign * k * fraction);
+  potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
   add_potential_sample(o, scale, tile, d1, potential, tally);
   if (nb > 1) {
-    V3 middle;
-    if constexpr (Exact)
-      middle = vmul(bperp, (subdivided ? 1. : sign) * t.constant / (den * path.distance));
-    else
-      middle = vmul(bperp, (subdivided ? 1. : sign) * k);
+    V3 const middle = vmul(bperp, (subdivided ? 1. : sign) * t.constant / (den * path.distance));
     // Bins of the first and last middle sample, exactly as the per-bin loop
     // computes them; in between the bins are consecutive.
-    double b_first, b_last;
-    if constexpr (Exact) {
-      b_first = nearest_bin((d1 + 1. / o.rate - o.start) * o.rate);
-      b_last = nearest_bin((d1 + static_cast<double>(nb - 1) / o.rate - o.start) * o.rate);
-    } else {
-      b_first = nearest_bin(x1 + 1.);
-      b_last = nearest_bin(x1 + static_cast<double>(nb - 1));
-    }
+    double const b_first = nearest_bin((d1 + 1. / o.rate - o.start) * o.rate);
+    double const b_last = nearest_bin((d1 + static_cast<double>(nb - 1) / o.rate - o.start) * o.rate);
     if (b_last - b_first == static_cast<double>(nb - 2)) {
       double const lo = b_first < 0. ? 0. : b_first;
       double const hi = b_last < o.nbins_d - 1. ? b_last : o.nbins_d - 1.;
@@ -565,29 +476,19 @@ __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double t
     }
   }
   fraction = fabs((d2 - o.start) * o.rate + 0.5 - end_bin);
-  if constexpr (Exact)
-    potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
-  else
-    potential = vmul(bperp, sign * k * fraction);
+  potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
   add_potential_sample(o, scale, tile, d2, potential, tally);
 }
 
-template <bool Exact, bool Fixed>
+template <bool Fixed>
 __device__ __forceinline__ void zhs_pair(Track const& t, PropagationDev const& p, std::uint32_t refinement_u,
                          Obs const& o, double scale, Tile<Fixed> const& tile, Tally& tally,
                          bool count_subtracks) {
   V3 const midpoint = vmul(vadd(t.start, t.end), 0.5);
-  Path const mp = propagate<Exact>(p, midpoint, o);
-  double u_k, fraunhofer;
-  if constexpr (Exact) {
-    u_k = vdot(t.beta, mp.emit) / t.beta_module;
-    double const sin2 = 1. - u_k * u_k;
-    fraunhofer = sin2 * t.length * t.length / mp.distance / o.wavelength * 2. * kPi;
-  } else {
-    u_k = vdot(t.beta, mp.emit) * t.inv_beta_module;
-    double const sin2 = 1. - u_k * u_k;
-    fraunhofer = sin2 * t.length * t.length * mp.inv_distance * o.two_pi_over_wavelength;
-  }
+  Path const mp = propagate(p, midpoint, o);
+  double const u_k = vdot(t.beta, mp.emit) / t.beta_module;
+  double const sin2 = 1. - u_k * u_k;
+  double const fraunhofer = sin2 * t.length * t.length / mp.distance / o.wavelength * 2. * kPi;
   double divisor = 1.;
   int nsub = 1;
   if (fraunhofer > 1.) {
@@ -626,7 +527,7 @@ __device__ __forceinline__ void zhs_pair(Track const& t, PropagationDev const& p
   for (int i = 0; i < segments; ++i) {
     V3 const p2 = vadd(p1, rs);
     double const time2 = time1 + rt;
-    zhs_segment<Exact>(p1, p2, time1, time2, t, p, o, scale, tile, tally, subdivided, use_cached,
+    zhs_segment(p1, p2, time1, time2, t, p, o, scale, tile, tally, subdivided, use_cached,
                        mp);
     p1 = p2;
     time1 = time2;
@@ -641,7 +542,6 @@ __device__ __forceinline__ Obs make_obs(ObserverDev const& d, PropagationDev con
   o.rate = d.sample_rate;
   o.grid = 1. / d.sample_rate;
   o.wavelength = kC / d.sample_rate;
-  o.two_pi_over_wavelength = 2. * kPi / o.wavelength;
   o.nbins = static_cast<std::int32_t>(d.number_of_bins);
   o.nbins_d = static_cast<double>(d.number_of_bins);
   o.offset = d.waveform_offset;
@@ -700,6 +600,101 @@ __device__ void block_inclusive_scan(T* row, std::uint32_t count, T* wave_totals
   __syncthreads();
 }
 
+template <class T>
+__device__ __forceinline__ T wave_sum(T x) {
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
+  return x;
+}
+
+// A value every lane of the wave holds, kept in scalar registers.
+__device__ __forceinline__ double uniform(double x) {
+  long long const bits = __double_as_longlong(x);
+  std::uint32_t const lo = __builtin_amdgcn_readfirstlane(static_cast<int>(bits));
+  std::uint32_t const hi = __builtin_amdgcn_readfirstlane(static_cast<int>(bits >> 32));
+  return __longlong_as_double(static_cast<long long>((static_cast<std::uint64_t>(hi) << 32) | lo));
+}
+
+__device__ __forceinline__ fast::View make_view(ObserverDev const& d, PropagationDev const& p,
+                                                std::uint64_t tile_begin, std::uint32_t tile_bins,
+                                                double coreas_scale, double zhs_scale) {
+  Obs const o = make_obs(d, p);
+  fast::View v;
+  v.position = {uniform(o.position.x), uniform(o.position.y), uniform(o.position.z)};
+  v.start = uniform(o.start);
+  v.end = uniform(o.start + o.duration);
+  v.rate = uniform(o.rate);
+  v.grid = uniform(o.grid);
+  v.two_pi_over_wavelength = uniform(2. * kPi / o.wavelength);
+  v.tile_begin = uniform(static_cast<double>(tile_begin));
+  v.tile_end = uniform(static_cast<double>(tile_begin + tile_bins));
+  v.table_last = uniform(static_cast<double>(p.table_size - 1));
+  v.destination_height = uniform(o.destination_height);
+  v.destination_index = uniform(static_cast<double>(o.destination_index));
+  v.n_destination = uniform(o.n_destination_table);
+  v.integrated_destination = uniform(o.integrated_destination);
+  v.coreas_scale = uniform(coreas_scale);
+  v.zhs_scale = uniform(zhs_scale);
+  return v;
+}
+
+// Tracks of one wave whose CoREAS update takes the Cherenkov form. About one
+// track-antenna pair in ten does in air (2^20 tracks x 160 antennas: 10%), so
+// nearly every wave would run both forms; a wave lists them (LDS, its own
+// entries) and runs the second form on 64 of them at a time.
+inline constexpr std::uint32_t kNearEntries = 128;  // up to 63 left over + 64 new
+inline constexpr std::uint32_t kForwardBit = 1u << 31;
+
+// The fast updates of the tracks [chunk_begin, chunk_end) by a workgroup.
+template <bool Coreas, bool Zhs, bool Homogeneous, int Block>
+__device__ __forceinline__ void fast_chunk(ProjectionLaunch const& L, PropagationDev const& prop,
+                                           fast::View const& view, std::uint64_t chunk_begin,
+                                           std::uint64_t chunk_end, long long* coreas_tile,
+                                           std::uint32_t coreas_stride, long long* zhs_tile,
+                                           std::uint32_t zhs_stride, bool count_valid, bool count_subtracks,
+                                           std::uint32_t* near_entries, fast::Tally& tally) {
+  std::uint32_t const lane = threadIdx.x % 64;
+  double const* const chunk = L.tracks + chunk_begin;
+  std::uint32_t const count = static_cast<std::uint32_t>(chunk_end - chunk_begin);
+  std::uint32_t pending = 0;  // this wave's listed tracks
+  auto run_near = [&](std::uint32_t entry) {
+    fast::Track t;
+    (void)fast::load_track(chunk, L.stride, entry & ~kForwardBit, t);
+    fast::coreas_near<Homogeneous>(t, prop, view, coreas_tile, coreas_stride, tally, (entry & kForwardBit) != 0);
+  };
+  for (std::uint32_t i = 0; i < count; i += Block) {
+    bool near = false, forward = false;
+    if (i + threadIdx.x < count) {
+      fast::Track t;
+      if (fast::load_track(chunk + i, L.stride, threadIdx.x, t)) {
+        if (count_valid) ++tally.valid;
+        if constexpr (Coreas)
+          near = fast::coreas_far<Homogeneous>(t, prop, view, coreas_tile, coreas_stride, tally, forward);
+        if constexpr (Zhs)
+          fast::zhs_update<Homogeneous>(t, prop, L.zhs_refinement, view, zhs_tile, zhs_stride, tally,
+                                        count_subtracks);
+      }
+    }
+    if constexpr (Coreas) {
+      unsigned long long const mask = __ballot(near);
+      if (mask == 0) continue;
+      std::uint32_t const below = __builtin_amdgcn_mbcnt_hi(
+          static_cast<std::uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<std::uint32_t>(mask), 0u));
+      if (near) near_entries[pending + below] = (i + threadIdx.x) | (forward ? kForwardBit : 0u);
+      pending += static_cast<std::uint32_t>(__popcll(mask));
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own entries, in order
+      if (pending >= 64) {
+        pending -= 64;
+        run_near(near_entries[pending + lane]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      }
+    }
+  }
+  if constexpr (Coreas) {
+    if (lane < pending) run_near(near_entries[lane]);
+  }
+}
+
 template <bool Coreas, bool Zhs, bool Fixed, bool Exact, int Block>
 __global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunch L) {
   using Acc = std::conditional_t<Fixed, long long, double>;
@@ -707,6 +702,7 @@ __global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunc
   __shared__ Acc scan_scratch[Zhs ? Block / 64 : 1];
   __shared__ unsigned long long block_counts[5];
   __shared__ double block_abs[2];
+  __shared__ std::uint32_t near_lists[Coreas && !Exact ? Block / 64 : 1][Coreas && !Exact ? kNearEntries : 1];
 
   std::uint32_t observer, bin_tile;
   std::uint64_t chunk_begin, chunk_end;
@@ -766,39 +762,74 @@ __global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunc
   // A fused launch has identical CoREAS and ZHS observers (position, window,
   // rate, bins and hence offsets); only their fixed-point scales differ.
   ObserverDev const& view = Coreas ? L.coreas_observers[observer] : L.zhs_observers[observer];
-  Obs const o = make_obs(view, prop);
+  std::uint64_t const offset = view.waveform_offset;
   double const coreas_scale = Coreas ? L.coreas_observers[observer].fixed_scale : 0.;
   double const zhs_scale = Zhs ? L.zhs_observers[observer].fixed_scale : 0.;
-  std::uint64_t const nbins = static_cast<std::uint64_t>(o.nbins);
+  std::uint64_t const nbins = view.number_of_bins;
   std::uint32_t const tile_bins =
       tile_begin < nbins ? static_cast<std::uint32_t>(nbins - tile_begin < W ? nbins - tile_begin : W)
                          : 0u;
-  Tile<Fixed> const ctile{coreas_lds, W, static_cast<std::int32_t>(tile_begin),
-                          static_cast<std::int32_t>(tile_bins)};
-  Tile<Fixed> const ztile{zhs_lds, W + 1, static_cast<std::int32_t>(tile_begin),
-                          static_cast<std::int32_t>(tile_bins)};
 
-  Tally ctally, ztally;
-  for (std::uint64_t i = chunk_begin + threadIdx.x; i < chunk_end; i += blockDim.x) {
-    Track t;
-    if (!load_track<Exact>(L.tracks, L.stride, i, t)) continue;
-    if (first_observer_tile) ++ctally.valid;
-    if constexpr (Coreas) {
-      if (tile_bins) coreas_pair<Exact>(t, prop, o, coreas_scale, ctile, ctally);
+  unsigned long long counts[5];
+  double abs_sums[2];
+  if constexpr (Exact) {
+    Obs const o = make_obs(view, prop);
+    Tile<Fixed> const ctile{coreas_lds, W, static_cast<std::int32_t>(tile_begin),
+                            static_cast<std::int32_t>(tile_bins)};
+    Tile<Fixed> const ztile{zhs_lds, W + 1, static_cast<std::int32_t>(tile_begin),
+                            static_cast<std::int32_t>(tile_bins)};
+    Tally ctally, ztally;
+    for (std::uint64_t i = chunk_begin + threadIdx.x; i < chunk_end; i += blockDim.x) {
+      Track t;
+      if (!load_track(L.tracks, L.stride, i, t)) continue;
+      if (first_observer_tile) ++ctally.valid;
+      if constexpr (Coreas) {
+        if (tile_bins) coreas_pair(t, prop, o, coreas_scale, ctile, ctally);
+      }
+      if constexpr (Zhs) {
+        zhs_pair(t, prop, L.zhs_refinement, o, zhs_scale, ztile, ztally, bin_tile == 0);
+      }
     }
-    if constexpr (Zhs) {
-      zhs_pair<Exact>(t, prop, L.zhs_refinement, o, zhs_scale, ztile, ztally, bin_tile == 0);
-    }
+    counts[0] = ctally.coreas;
+    counts[1] = ztally.zhs;
+    counts[2] = ztally.subtracks;
+    counts[3] = ctally.valid;
+    counts[4] = ctally.overflow + ztally.overflow;
+    abs_sums[0] = ctally.abs_sum;
+    abs_sums[1] = ztally.abs_sum;
+  } else {
+    fast::View const v = make_view(view, prop, tile_begin, tile_bins, coreas_scale, zhs_scale);
+    fast::Tally tally;
+    std::uint32_t* const near = near_lists[Coreas ? threadIdx.x / 64 : 0];
+    if (prop.homogeneous_index > 0.)
+      fast_chunk<Coreas, Zhs, true, Block>(L, prop, v, chunk_begin, chunk_end, coreas_lds, W, zhs_lds, W + 1,
+                                           first_observer_tile, bin_tile == 0, near, tally);
+    else
+      fast_chunk<Coreas, Zhs, false, Block>(L, prop, v, chunk_begin, chunk_end, coreas_lds, W, zhs_lds, W + 1,
+                                            first_observer_tile, bin_tile == 0, near, tally);
+    counts[0] = tally.coreas;
+    counts[1] = tally.zhs;
+    counts[2] = tally.subtracks + tally.single_subtracks;
+    counts[3] = tally.valid;
+    counts[4] = tally.overflow;
+    abs_sums[0] = tally.coreas_abs;
+    abs_sums[1] = tally.zhs_abs;
   }
 
-  atomicAdd(&block_counts[0], ctally.coreas);
-  atomicAdd(&block_counts[1], ztally.zhs);
-  atomicAdd(&block_counts[2], ztally.subtracks);
-  atomicAdd(&block_counts[3], ctally.valid);
-  atomicAdd(&block_counts[4], ctally.overflow + ztally.overflow);
+  // one LDS add per wave and tally
+#pragma unroll
+  for (int k = 0; k < 5; ++k) {
+    if ((k == 0 && !Coreas) || ((k == 1 || k == 2) && !Zhs)) continue;
+    unsigned long long const sum = wave_sum(counts[k]);
+    if (threadIdx.x % 64 == 0 && sum) atomicAdd(&block_counts[k], sum);
+  }
   if constexpr (Fixed) {
-    atomicAdd(&block_abs[0], ctally.abs_sum);
-    atomicAdd(&block_abs[1], ztally.abs_sum);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      if ((k == 0 && !Coreas) || (k == 1 && !Zhs)) continue;
+      double const sum = wave_sum(abs_sums[k]);
+      if (threadIdx.x % 64 == 0) atomicAdd(&block_abs[k], sum);
+    }
   }
   __syncthreads();
 
@@ -812,21 +843,21 @@ __global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunc
   auto flush = [&](Acc const* lds, std::uint32_t row, std::uint32_t bins, void* global,
                    std::uint64_t total_bins) {
     Acc* const g = static_cast<Acc*>(global);
-    for (std::uint32_t idx = threadIdx.x; idx < 3 * bins; idx += blockDim.x) {
-      std::uint32_t const c = idx / bins;
-      std::uint32_t const b = idx % bins;
-      Acc const v = lds[c * row + b];
-      if (v == 0) continue;
-      std::uint64_t const at = c * total_bins + o.offset + tile_begin + b;
-      if constexpr (Fixed) {
-        long long const previous = static_cast<long long>(
-            atomicAdd(reinterpret_cast<unsigned long long*>(g + at),
-                      static_cast<unsigned long long>(v)));
-        if ((v > 0 && previous > 0x7fffffffffffffffLL - v) ||
-            (v < 0 && previous < (-0x7fffffffffffffffLL - 1) - v))
-          ++flush_overflows;
-      } else {
-        atomicAdd(g + at, v);
+    for (std::uint32_t c = 0; c < 3; ++c) {
+      for (std::uint32_t b = threadIdx.x; b < bins; b += blockDim.x) {
+        Acc const v = lds[c * row + b];
+        if (v == 0) continue;
+        std::uint64_t const at = c * total_bins + offset + tile_begin + b;
+        if constexpr (Fixed) {
+          long long const previous = static_cast<long long>(
+              atomicAdd(reinterpret_cast<unsigned long long*>(g + at),
+                        static_cast<unsigned long long>(v)));
+          if ((v > 0 && previous > 0x7fffffffffffffffLL - v) ||
+              (v < 0 && previous < (-0x7fffffffffffffffLL - 1) - v))
+            ++flush_overflows;
+        } else {
+          atomicAdd(g + at, v);
+        }
       }
     }
   };

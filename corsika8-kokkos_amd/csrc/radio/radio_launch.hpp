@@ -23,8 +23,12 @@ inline constexpr std::size_t kMaxDynamicLdsBytes = 144 * 1024;
 // ZHS window keep one tile.
 inline constexpr std::size_t kPreferredWorkgroupLdsBytes = 53 * 1024;
 // Upper bound of the projection kernel's static LDS: the wave totals of the ZHS
-// scan (16 x 8 B for 1024 threads), block counters and |increment| sums.
+// scan (16 x 8 B for 1024 threads), block counters and |increment| sums; with
+// CoREAS also the Cherenkov lists of 512 threads' waves (8 x 512 B).
 inline constexpr std::size_t kProjectionStaticLdsBytes = 256;
+inline constexpr std::size_t kCoreasStaticLdsBytes = 4096;
+// Most tracks a workgroup takes (its tallies and lists use 32-bit words).
+inline constexpr std::uint64_t kMaxChunkTracks = std::uint64_t{1} << 30;
 // Tracks per workgroup the default chunking gives a batch large enough for
 // eight such chunks, at least (a smaller batch is cut into eight chunks).
 inline constexpr std::uint64_t kMinimumDefaultChunk = 32768;

@@ -159,6 +159,7 @@ void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, std::uint32_t 
     std::uint64_t const block = tuning.block_threads;
     chunk = std::max<std::uint64_t>(block, (chunk + block - 1) / block * block);
   }
+  chunk = std::min(chunk, kMaxChunkTracks);
   L.chunk_size = chunk;
   std::uint64_t const chunks = (count + chunk - 1) / chunk;
   if (chunks > std::numeric_limits<std::uint32_t>::max())

@@ -1,0 +1,100 @@
+"""The fast radio projection at the edges of its workgroups, waves, tiles and lists
+against the FP64 oracle.
+
+Track counts around a wave (64), a workgroup (512) and their remainders; tracks that all
+take CoREAS's Cherenkov form (a wave lists them and runs 64 at a time), none, or a mix;
+window tiles that cut segments of several bins; sources above, below and on the ends of
+the propagation table; groups of observers and their remainders. The bar is the fast
+form's: per observer a relative L2 error of 1e-6 (FP64 rounding of about ten operations per
+sample is 1e-14 relative, 1e-11 near the Cherenkov angle, where 1 - n b.e >= 1e-9 cancels),
+with a field limit of 1e-6 V/m, so that the int64 quantum (2^-62 of the limit per sample)
+is below 1e-9 of the smallest field here. Counters equal the oracle's.
+"""
+import numpy as np
+import pytest
+
+import c8mi
+import oracle_lib
+from radio_cases import C, random_tracks, uniform_table, window_observers
+from test_radio_gpu import POSITIONS, exponential_table, gpu_project
+
+pytestmark = pytest.mark.gpu
+
+
+LIMIT = 1.0e-6
+
+
+def assert_close(tracks, obs, prop, refinement=1, tuning=None):
+    ref = oracle_lib.radio_project(prop, obs, tracks, refinement=refinement, limit=LIMIT, threads=4)
+    got = gpu_project(tracks, obs, prop, refinement=refinement, exact=False, limit=LIMIT, tuning=tuning)
+    offsets = np.concatenate([[0], np.cumsum(obs["number_of_bins"].astype(np.int64))])
+    for fixed, name in ((got[0], "coreas"), (got[1], "zhs")):
+        field = oracle_lib.radio_decode(fixed, obs, limit=LIMIT, potential=name == "zhs")
+        for k in range(obs.size):
+            want = ref[name + "_float"][:, offsets[k]:offsets[k + 1]]
+            error = np.linalg.norm(field[:, offsets[k]:offsets[k + 1]] - want)
+            assert error <= 1e-6 * np.linalg.norm(want), (name, k)
+    assert got[2] == ref["counters"]
+    return ref["counters"]
+
+
+def near_tracks(count, seed):
+    """Tracks whose direction points at the antennas at beta ~ 1: small Doppler factors."""
+    rng = np.random.default_rng(seed)
+    tracks = random_tracks(count, seed, box=1.0, height=(900.0, 1400.0))
+    length = rng.uniform(0.5, 3.0, count)
+    tracks[3:6] = tracks[0:3] + np.stack([np.zeros(count), np.zeros(count), -length])
+    tracks[7] = tracks[6] + length / (C * rng.uniform(0.9995, 1.0, count))
+    return tracks
+
+
+def mixed(count, seed, share):
+    tracks = random_tracks(count, seed)
+    near = np.random.default_rng(seed + 1).random(count) < share
+    tracks[:, near] = near_tracks(count, seed + 2)[:, near]
+    return tracks
+
+
+@pytest.mark.parametrize("count", [1, 63, 64, 65, 511, 512, 513, 1300])
+@pytest.mark.parametrize("share", [0.0, 0.4, 1.0])
+def test_counts_and_cherenkov_lists(count, share):
+    tracks = mixed(count, 11 + count, share)
+    obs = window_observers(tracks, POSITIONS[:5], 2.0e9, 1024)
+    for prop in (exponential_table(), c8mi.Propagation(homogeneous_index=1.0003)):
+        assert_close(tracks, obs, prop)
+
+
+@pytest.mark.parametrize("tile", [0, 5, 64, 333])
+@pytest.mark.parametrize("refinement", [1, 3])
+def test_segments_across_window_tiles(tile, refinement):
+    tracks = mixed(700, 5, 0.2)
+    tracks[3:6] += 3.0 * (tracks[3:6] - tracks[0:3])  # segments of several bins
+    tracks[7] += 3.0 * (tracks[7] - tracks[6])
+    obs = window_observers(tracks, POSITIONS[:4], 1.0e9, 120)
+    prop = uniform_table(1.0003, upper=4000.0)
+    tuning = dict(tile_bins=tile, chunk_tracks=512, block_threads=512) if tile else None
+    counters = assert_close(tracks, obs, prop, refinement, tuning)
+    assert counters["zhs_contributions"] > 1.5 * counters["zhs_subtracks"]
+
+
+def test_sources_outside_the_table():
+    tracks = random_tracks(600, 21, height=(-40.0, 300.0))
+    tracks[2, :5] = tracks[5, :5] = 200.0  # the last table height
+    tracks[2, 5:10] = 0.0  # the first
+    obs = window_observers(tracks, ((3., 4., 50.), (-20., 60., 120.)), 2.0e9, 2048)
+    prop = uniform_table(1.0003, lower=0.0, upper=200.0)
+    assert_close(tracks, obs, prop)
+
+
+def test_large_increments():
+    """Components beyond 2^51 in fixed point take the rounding form."""
+    tracks = mixed(200, 3, 0.3)
+    obs = window_observers(tracks, POSITIONS[:3], 2.0e9, 512)
+    prop = exponential_table()
+    limit = 1.0e-9
+    ref = oracle_lib.radio_project(prop, obs, tracks, limit=limit, threads=4)
+    got = gpu_project(tracks, obs, prop, exact=False, limit=limit)
+    for k, name in enumerate(("coreas", "zhs")):
+        want = ref[name + "_fixed"].astype(np.float64)
+        assert np.abs(want).max() > 2.0 ** 52
+        assert np.linalg.norm(got[k] - want) <= 1e-6 * np.linalg.norm(want)
