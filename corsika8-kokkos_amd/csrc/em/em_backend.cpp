@@ -796,7 +796,15 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
   f.first_interactions = first_interactions_.data();
   f.first_candidates = first_candidates_.data();
   int const track_buffer = track_parity_;
-  if ((radio_ || slot_radio_) && !photon) {
+  // An attached accumulator alone gathers the fronts' tracks into its own
+  // batches (a front's 1e2 to 1e5 tracks leave the projection's workgroups with a
+  // window to clear and flush for few tracks each, and its launches hold up the
+  // next front's kernels: 10 TeV with 160 antennas 0.36 -> 0.30 s, whose groups of
+  // observers launched front by front took 0.31 where one observer a workgroup took 0.28).
+  bool const batched = radio_ && !slot_radio_ && !photon;
+  if (batched) {
+    f.tracks = radio_->reserve_tracks(m, f.track_stride, stream_);
+  } else if ((radio_ || slot_radio_) && !photon) {
     // tracks [9][n]; the buffer's previous projections must be done first
     std::uint64_t& capacity = track_capacity_[track_buffer];
     if (capacity < m) {
@@ -814,6 +822,11 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
   // Projects this front's tracks on the accumulators' streams once the step kernel is done.
   auto project_tracks = [&] {
     if (!f.tracks) return;
+    if (batched) {
+      C8MI_HIP(hipEventRecord(track_ready_[0], stream_));
+      radio_->commit_tracks(m, track_ready_[0]);
+      return;
+    }
     std::uint64_t const chunk = slot_radio_ ? slot_radio_->chunk_for(m) : 0;
     if (slot_radio_) {
       std::size_t const keys = static_cast<std::size_t>(slots_) * kMaxRuns;

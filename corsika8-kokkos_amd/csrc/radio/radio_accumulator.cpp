@@ -39,13 +39,13 @@ RadioAccumulator::RadioAccumulator(c8mi_radio_config const& config, hipStream_t 
       coreas_snapshots_.assign(config.coreas_observers,
                                config.coreas_observers + config.coreas_observer_count);
       coreas_host_ = make_observers(config.coreas_observers, config.coreas_observer_count,
-                                    limit, false, coreas_bins_, coreas_max_bins_);
+                                    limit, false, config.propagation, coreas_bins_, coreas_max_bins_);
     }
     if (config.zhs_enabled) {
       zhs_snapshots_.assign(config.zhs_observers,
                             config.zhs_observers + config.zhs_observer_count);
       zhs_host_ = make_observers(config.zhs_observers, config.zhs_observer_count, limit, true,
-                                 zhs_bins_, zhs_max_bins_);
+                                 config.propagation, zhs_bins_, zhs_max_bins_);
     }
     // The config keeps borrowed pointers only for validation; the snapshots
     // above own the observer data from here on.
@@ -90,12 +90,15 @@ RadioAccumulator::~RadioAccumulator() {
     (void)hipEventDestroy(e.first);
     (void)hipEventDestroy(e.second);
   }
+  for (auto& b : batches_)
+    if (b.projected) (void)hipEventDestroy(b.projected);
   if (owns_stream_) (void)hipStreamDestroy(stream_);
 }
 
 void RadioAccumulator::reset() {
   if (host_count_ != 0)
     throw std::logic_error("cannot reset radio with uncommitted host tracks");
+  for (auto& b : batches_) b.count = 0;  // their waveforms would be cleared here
   if (coreas_fixed_.size())
     C8MI_HIP(hipMemsetAsync(coreas_fixed_.data(), 0, coreas_fixed_.bytes(), stream_));
   if (zhs_fixed_.size())
@@ -170,6 +173,41 @@ void RadioAccumulator::accumulate_tracks(double const* device_tracks, std::uint6
   project(device_tracks, stride, count);
 }
 
+double* RadioAccumulator::reserve_tracks(std::uint64_t count, std::uint64_t& stride, hipStream_t producer) {
+  if (sealed_) throw std::logic_error("radio endpoint already committed; reset before new tracks");
+  if (batches_[batch_].count + count > batches_[batch_].capacity) {
+    project_batch();
+    batch_ ^= 1;
+  }
+  TrackBatch& b = batches_[batch_];
+  if (b.capacity < count) {
+    if (b.recorded) C8MI_HIP(hipEventSynchronize(b.projected));
+    b.capacity = 0;
+    b.tracks.allocate(C8MI_RADIO_TRACK_FIELDS * std::max(count, kBatchTracks));
+    b.capacity = std::max(count, kBatchTracks);
+  }
+  if (!b.projected) C8MI_HIP(hipEventCreateWithFlags(&b.projected, hipEventDisableTiming));
+  if (b.recorded) C8MI_HIP(hipStreamWaitEvent(producer, b.projected, 0));
+  stride = b.capacity;
+  return b.tracks.data() + b.count;
+}
+
+void RadioAccumulator::commit_tracks(std::uint64_t count, hipEvent_t written) {
+  C8MI_HIP(hipStreamWaitEvent(stream_, written, 0));
+  batches_[batch_].count += count;
+  downloaded_ = false;
+}
+
+void RadioAccumulator::project_batch() {
+  TrackBatch& b = batches_[batch_];
+  if (b.count == 0) return;
+  std::uint64_t const count = b.count;
+  b.count = 0;
+  project(b.tracks.data(), b.capacity, count);
+  C8MI_HIP(hipEventRecord(b.projected, stream_));
+  b.recorded = true;
+}
+
 void RadioAccumulator::check_accumulate(std::uint64_t count) const {
   if (count == 0) return;
   if (sealed_) throw std::logic_error("radio endpoint already committed; reset before new tracks");
@@ -198,7 +236,7 @@ ProjectionLaunch RadioAccumulator::base_launch(bool coreas, bool zhs, std::uint3
   tuning.tile_bins_limit = tile_bins_limit_;
   tuning.target_workgroups = target_workgroups_;
   tuning.block_threads = block_threads_;
-  shape_projection(L, coreas, zhs, observers, max_bins, count, tuning);
+  shape_projection(L, coreas, zhs, config_.deterministic && !config_.exact_fp64, observers, max_bins, count, tuning);
   return L;
 }
 
@@ -233,7 +271,7 @@ void RadioAccumulator::project(double const* tracks, std::uint64_t stride, std::
       }
       C8MI_HIP(hipEventRecord(events.first, stream_));
     }
-    launch_projection(L, coreas, zhs, fixed, config_.exact_fp64 != 0, block_threads_, stream_);
+    launch_projection(L, coreas, zhs, fixed, config_.exact_fp64 != 0, stream_);
     if (timing_) {
       C8MI_HIP(hipEventRecord(events.second, stream_));
       pending_events_.push_back({events.first, events.second, coreas && zhs ? 0 : coreas ? 1 : 2});
@@ -272,6 +310,7 @@ void RadioAccumulator::copy_counters(c8mi_radio_counters* out) {
 void RadioAccumulator::download(double* coreas, double* zhs, c8mi_radio_counters* counters) {
   if (downloaded_ || sealed_) throw std::logic_error("radio waveforms downloaded twice");
   flush_host_lepton_tracks();
+  project_batch();
   c8mi_radio_counters c{};
   copy_counters(&c);
   if (counters) *counters = c;
@@ -319,6 +358,7 @@ void RadioAccumulator::download_fixed(std::int64_t* coreas, std::int64_t* zhs,
   if (!config_.deterministic) throw std::logic_error("fixed radio snapshot needs deterministic mode");
   if (downloaded_ || sealed_) throw std::logic_error("fixed radio snapshot already committed");
   flush_host_lepton_tracks();
+  project_batch();
   sealed_ = true;
   copy_counters(counters);
   if (coreas && coreas_fixed_.size())
@@ -348,6 +388,7 @@ void RadioAccumulator::set_tuning(std::uint64_t chunk_tracks, std::uint32_t tile
 }
 
 void RadioAccumulator::enable_kernel_timing(bool enable) {
+  project_batch();  // timed or not as it was committed
   timing_ = enable;
   for (int k = 0; k < 3; ++k) {
     timed_ms_[k] = 0.;
@@ -356,6 +397,7 @@ void RadioAccumulator::enable_kernel_timing(bool enable) {
 }
 
 void RadioAccumulator::kernel_time_ms(double ms[3], std::uint64_t launches[3]) {
+  project_batch();
   C8MI_HIP(hipStreamSynchronize(stream_));
   for (auto& e : pending_events_) {
     float elapsed = 0.f;

@@ -56,6 +56,14 @@ class RadioAccumulator {
   // Throws what accumulate_tracks of `count` valid tracks would throw, without
   // launching anything (callers check before work that cannot be undone).
   void check_accumulate(std::uint64_t count) const;
+  // Tracks of a producer on another stream, gathered into batches large enough to
+  // fill the chip: room for `count` tracks in the accumulator's own buffer
+  // ([9][stride], valid until the next reserve or download), which `producer`
+  // then writes and commits with an event recorded behind its writes. A full
+  // batch is projected at once, the last by download, download_fixed or
+  // kernel_time_ms.
+  double* reserve_tracks(std::uint64_t count, std::uint64_t& stride, hipStream_t producer);
+  void commit_tracks(std::uint64_t count, hipEvent_t written);
 
   // Decoded waveforms, [3][total_bins] per algorithm (x, y, z blocks). Either
   // output may be null. Throws OverflowError when the fixed-point range was
@@ -83,6 +91,7 @@ class RadioAccumulator {
 
  private:
   void project(double const* tracks, std::uint64_t stride, std::uint64_t count);
+  void project_batch();
   void ensure_track_capacity(std::uint64_t count);
   ProjectionLaunch base_launch(bool coreas, bool zhs, std::uint32_t observers,
                                std::uint64_t max_bins, std::uint64_t count) const;
@@ -116,6 +125,17 @@ class RadioAccumulator {
   DeviceBuffer<CountersDev> counters_;
   DeviceBuffer<double> tracks_;
   std::uint64_t track_capacity_ = 0;
+  // Batches of committed tracks: one fills while the other is projected. 2^20
+  // tracks (75 MB) unless a single reserve asks for more.
+  static constexpr std::uint64_t kBatchTracks = std::uint64_t{1} << 20;
+  struct TrackBatch {
+    DeviceBuffer<double> tracks;
+    std::uint64_t capacity = 0, count = 0;
+    hipEvent_t projected = nullptr;
+    bool recorded = false;
+  };
+  TrackBatch batches_[2];
+  int batch_ = 0;
   DeviceBuffer<c8mi_lepton_transport_record> host_batch_device_;
   PinnedBuffer<c8mi_lepton_transport_record> host_batch_;
   std::size_t host_count_ = 0;
@@ -126,7 +146,7 @@ class RadioAccumulator {
   // separate CoREAS and ZHS launches (48 KiB LDS each, three workgroups per
   // CU), 512 threads, about 8192 workgroups per launch.
   std::uint32_t target_workgroups_ = 8192;
-  std::uint32_t block_threads_ = 512;
+  std::uint32_t block_threads_ = 0;  // 0: by the launch's shape
   bool split_ = true;
 
   bool timing_ = false;

@@ -18,6 +18,13 @@ struct ObserverDev {
   double fixed_scale;  // 2^62 * (ZHS ? sample_rate : 1) / field limit
   std::uint64_t number_of_bins;
   std::uint64_t waveform_offset;
+  // derived once on the host for the fast kernels
+  double end_time;                // start_time + duration
+  double grid;                    // 1 / sample_rate
+  double two_pi_over_wavelength;  // at the sample rate
+  double destination_height, destination_index;  // the observer in the propagation table
+  double n_destination, integrated_destination;  // and the table there
+  double pad;
 };
 
 // Straight-ray propagation table (RadioPropagationView,
@@ -77,7 +84,7 @@ struct ProjectionLaunch {
   std::uint32_t bin_tiles;   // window tiles per observer
   std::uint32_t tile_bins;   // bins held in LDS per mode
   std::uint32_t count_valid; // tally valid tracks in this launch (once per batch)
-  std::uint32_t pad;
+  std::uint32_t group;       // observers per workgroup (fast form; 1 in the exact form)
   // Pooled showers (segments non-null): workgroup b < *item_count is an item of
   // the segment holding it; the segment's slot selects the observers
   // [slot * slot_observers, + slot_observer_counts[slot]) and counters[slot].
@@ -86,7 +93,7 @@ struct ProjectionLaunch {
   unsigned long long const* item_count;
   std::uint32_t const* slot_observer_counts;
   std::uint32_t slot_observers;
-  std::uint32_t pad2;
+  std::uint32_t block_threads;  // threads per workgroup
 };
 
 }  // namespace c8mi::radio

@@ -26,9 +26,9 @@
 #include <stdexcept>
 #include <type_traits>
 
+#include "radio_block.hpp"
 #include "radio_device.hpp"
 #include "radio_launch.hpp"
-#include "radio_pair_fast.hpp"
 #include "../runtime.hpp"
 
 namespace c8mi::radio {
@@ -42,8 +42,6 @@ constexpr double kEmConstant = 1. / (4. * kPi * kEps0 * kC);
 constexpr double kChargeEm = kE * kEmConstant;
 constexpr double kCoreasThreshold = 1.e-3;
 constexpr double kIntLimit = 9223372036854775808.;  // 2^63
-
-constexpr int kXcds = 8;
 
 struct V3 {
   double x, y, z;
@@ -559,193 +557,36 @@ __device__ __forceinline__ Obs make_obs(ObserverDev const& d, PropagationDev con
   return o;
 }
 
-// Inclusive prefix sum over `count` entries of an LDS row, whole block: each
-// thread sums a contiguous run, the run totals are scanned within each wave by
-// shuffles and across waves by the first wave (wave_totals: one entry per wave).
-template <class T>
-__device__ __forceinline__ T wave_inclusive_sum(T x, std::uint32_t lane) {
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    T const y = __shfl_up(x, d, 64);
-    if (static_cast<int>(lane) >= d) x += y;
-  }
-  return x;
-}
-
-template <class T>
-__device__ void block_inclusive_scan(T* row, std::uint32_t count, T* wave_totals) {
-  std::uint32_t const tid = threadIdx.x;
-  std::uint32_t const threads = blockDim.x;
-  std::uint32_t const lane = tid & 63u, wave = tid >> 6;
-  std::uint32_t const waves = (threads + 63u) >> 6;
-  std::uint32_t const per = (count + threads - 1) / threads;
-  std::uint32_t const begin = tid * per < count ? tid * per : count;
-  std::uint32_t const end = begin + per < count ? begin + per : count;
-  T running = 0;
-  for (std::uint32_t i = begin; i < end; ++i) {
-    running += row[i];
-    row[i] = running;
-  }
-  T const inclusive = wave_inclusive_sum(running, lane);
-  if (lane == 63u) wave_totals[wave] = inclusive;
-  __syncthreads();
-  if (wave == 0) {
-    T const total = lane < waves ? wave_totals[lane] : T(0);
-    T const before = wave_inclusive_sum(total, lane) - total;
-    if (lane < waves) wave_totals[lane] = before;
-  }
-  __syncthreads();
-  T const offset = wave_totals[wave] + (inclusive - running);
-  for (std::uint32_t i = begin; i < end; ++i) row[i] += offset;
-  __syncthreads();
-}
-
-template <class T>
-__device__ __forceinline__ T wave_sum(T x) {
-#pragma unroll
-  for (int d = 32; d > 0; d >>= 1) x += __shfl_xor(x, d, 64);
-  return x;
-}
-
-// A value every lane of the wave holds, kept in scalar registers.
-__device__ __forceinline__ double uniform(double x) {
-  long long const bits = __double_as_longlong(x);
-  std::uint32_t const lo = __builtin_amdgcn_readfirstlane(static_cast<int>(bits));
-  std::uint32_t const hi = __builtin_amdgcn_readfirstlane(static_cast<int>(bits >> 32));
-  return __longlong_as_double(static_cast<long long>((static_cast<std::uint64_t>(hi) << 32) | lo));
-}
-
-__device__ __forceinline__ fast::View make_view(ObserverDev const& d, PropagationDev const& p,
-                                                std::uint64_t tile_begin, std::uint32_t tile_bins,
-                                                double coreas_scale, double zhs_scale) {
-  Obs const o = make_obs(d, p);
-  fast::View v;
-  v.position = {uniform(o.position.x), uniform(o.position.y), uniform(o.position.z)};
-  v.start = uniform(o.start);
-  v.end = uniform(o.start + o.duration);
-  v.rate = uniform(o.rate);
-  v.grid = uniform(o.grid);
-  v.two_pi_over_wavelength = uniform(2. * kPi / o.wavelength);
-  v.tile_begin = uniform(static_cast<double>(tile_begin));
-  v.tile_end = uniform(static_cast<double>(tile_begin + tile_bins));
-  v.table_last = uniform(static_cast<double>(p.table_size - 1));
-  v.destination_height = uniform(o.destination_height);
-  v.destination_index = uniform(static_cast<double>(o.destination_index));
-  v.n_destination = uniform(o.n_destination_table);
-  v.integrated_destination = uniform(o.integrated_destination);
-  v.coreas_scale = uniform(coreas_scale);
-  v.zhs_scale = uniform(zhs_scale);
-  return v;
-}
-
-// Tracks of one wave whose CoREAS update takes the Cherenkov form. About one
-// track-antenna pair in ten does in air (2^20 tracks x 160 antennas: 10%), so
-// nearly every wave would run both forms; a wave lists them (LDS, its own
-// entries) and runs the second form on 64 of them at a time.
-inline constexpr std::uint32_t kNearEntries = 128;  // up to 63 left over + 64 new
-inline constexpr std::uint32_t kForwardBit = 1u << 31;
-
-// The fast updates of the tracks [chunk_begin, chunk_end) by a workgroup.
-template <bool Coreas, bool Zhs, bool Homogeneous, int Block>
-__device__ __forceinline__ void fast_chunk(ProjectionLaunch const& L, PropagationDev const& prop,
-                                           fast::View const& view, std::uint64_t chunk_begin,
-                                           std::uint64_t chunk_end, long long* coreas_tile,
-                                           std::uint32_t coreas_stride, long long* zhs_tile,
-                                           std::uint32_t zhs_stride, bool count_valid, bool count_subtracks,
-                                           std::uint32_t* near_entries, fast::Tally& tally) {
-  std::uint32_t const lane = threadIdx.x % 64;
-  double const* const chunk = L.tracks + chunk_begin;
-  std::uint32_t const count = static_cast<std::uint32_t>(chunk_end - chunk_begin);
-  std::uint32_t pending = 0;  // this wave's listed tracks
-  auto run_near = [&](std::uint32_t entry) {
-    fast::Track t;
-    (void)fast::load_track(chunk, L.stride, entry & ~kForwardBit, t);
-    fast::coreas_near<Homogeneous>(t, prop, view, coreas_tile, coreas_stride, tally, (entry & kForwardBit) != 0);
-  };
-  for (std::uint32_t i = 0; i < count; i += Block) {
-    bool near = false, forward = false;
-    if (i + threadIdx.x < count) {
-      fast::Track t;
-      if (fast::load_track(chunk + i, L.stride, threadIdx.x, t)) {
-        if (count_valid) ++tally.valid;
-        if constexpr (Coreas)
-          near = fast::coreas_far<Homogeneous>(t, prop, view, coreas_tile, coreas_stride, tally, forward);
-        if constexpr (Zhs)
-          fast::zhs_update<Homogeneous>(t, prop, L.zhs_refinement, view, zhs_tile, zhs_stride, tally,
-                                        count_subtracks);
-      }
-    }
-    if constexpr (Coreas) {
-      unsigned long long const mask = __ballot(near);
-      if (mask == 0) continue;
-      std::uint32_t const below = __builtin_amdgcn_mbcnt_hi(
-          static_cast<std::uint32_t>(mask >> 32), __builtin_amdgcn_mbcnt_lo(static_cast<std::uint32_t>(mask), 0u));
-      if (near) near_entries[pending + below] = (i + threadIdx.x) | (forward ? kForwardBit : 0u);
-      pending += static_cast<std::uint32_t>(__popcll(mask));
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the wave's own entries, in order
-      if (pending >= 64) {
-        pending -= 64;
-        run_near(near_entries[pending + lane]);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      }
-    }
-  }
-  if constexpr (Coreas) {
-    if (lane < pending) run_near(near_entries[lane]);
-  }
-}
-
-template <bool Coreas, bool Zhs, bool Fixed, bool Exact, int Block>
-__global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunch L) {
+template <bool Coreas, bool Zhs, bool Fixed, int Block>
+__global__ void __launch_bounds__(Block, 4) radio_exact_kernel(ProjectionLaunch L) {
   using Acc = std::conditional_t<Fixed, long long, double>;
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ Acc scan_scratch[Zhs ? Block / 64 : 1];
-  __shared__ unsigned long long block_counts[5];
-  __shared__ double block_abs[2];
-  __shared__ std::uint32_t near_lists[Coreas && !Exact ? Block / 64 : 1][Coreas && !Exact ? kNearEntries : 1];
+  __shared__ BlockTallies block;
 
-  std::uint32_t observer, bin_tile;
+  std::uint32_t observer, bin_tile, within;
   std::uint64_t chunk_begin, chunk_end;
   CountersDev* counters = L.counters;
   bool first_observer_tile;
   if (L.segments == nullptr) {
-    // XCD-aware decode of blockIdx.x into (chunk, observer, window tile).
-    std::uint32_t const linear = blockIdx.x;
-    std::uint32_t const xcd = linear % kXcds;
-    std::uint32_t const sequence = linear / kXcds;
-    std::uint32_t const per_chunk = L.observer_count * L.bin_tiles;
-    std::uint32_t const chunk = (sequence / per_chunk) * kXcds + xcd;
-    if (chunk >= L.chunks) return;
-    std::uint32_t const within = sequence % per_chunk;
+    if (!decode_chunk(L, L.observer_count * L.bin_tiles, within, chunk_begin, chunk_end)) return;
     observer = within / L.bin_tiles;
     bin_tile = within % L.bin_tiles;
-    chunk_begin = static_cast<std::uint64_t>(chunk) * L.chunk_size;
-    chunk_end = chunk_begin + L.chunk_size < L.track_count ? chunk_begin + L.chunk_size : L.track_count;
-    first_observer_tile = L.count_valid && observer == 0 && bin_tile == 0;
+    first_observer_tile = L.count_valid && within == 0;
   } else {
-    // Pooled showers: the segment whose items hold blockIdx.x (binary search
-    // over item_begin), then (chunk, observer of the slot, window tile).
-    unsigned long long const item = blockIdx.x;
-    if (item >= *L.item_count) return;
-    std::uint32_t lo = 0, hi = *L.segment_count;  // segments[lo].item_begin <= item
-    while (hi - lo > 1) {
-      std::uint32_t const mid = (lo + hi) / 2;
-      if (L.segments[mid].item_begin <= item) lo = mid;
-      else hi = mid;
-    }
-    SegmentDev const seg = L.segments[lo];
-    std::uint64_t const local = item - seg.item_begin;
+    SegmentDev seg;
+    std::uint64_t local;
+    if (!decode_segment(L, seg, local)) return;
     std::uint64_t const per_chunk =
         static_cast<std::uint64_t>(L.slot_observer_counts[seg.slot]) * L.bin_tiles;
     std::uint64_t const chunk = local / per_chunk;
-    std::uint32_t const within = static_cast<std::uint32_t>(local % per_chunk);
-    std::uint32_t const slot_observer = within / L.bin_tiles;
-    observer = seg.slot * L.slot_observers + slot_observer;
+    within = static_cast<std::uint32_t>(local % per_chunk);
+    observer = seg.slot * L.slot_observers + within / L.bin_tiles;
     bin_tile = within % L.bin_tiles;
     chunk_begin = seg.begin + chunk * L.chunk_size;
     chunk_end = chunk_begin + L.chunk_size < seg.end ? chunk_begin + L.chunk_size : seg.end;
     counters = L.counters + seg.slot;
-    first_observer_tile = slot_observer == 0 && bin_tile == 0;
+    first_observer_tile = within == 0;
   }
 
   std::uint32_t const W = L.tile_bins;
@@ -753,8 +594,7 @@ __global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunc
   Acc* const zhs_lds = coreas_lds + (Coreas ? 3 * W : 0);
   std::uint32_t const lds_count = (Coreas ? 3 * W : 0) + (Zhs ? 3 * (W + 1) : 0);
   for (std::uint32_t i = threadIdx.x; i < lds_count; i += blockDim.x) coreas_lds[i] = 0;
-  if (threadIdx.x < 5) block_counts[threadIdx.x] = 0;
-  if (threadIdx.x < 2) block_abs[threadIdx.x] = 0.;
+  clear_tallies(block);
   __syncthreads();
 
   PropagationDev const prop = L.propagation;
@@ -762,124 +602,47 @@ __global__ void __launch_bounds__(Block, 4) radio_project_kernel(ProjectionLaunc
   // A fused launch has identical CoREAS and ZHS observers (position, window,
   // rate, bins and hence offsets); only their fixed-point scales differ.
   ObserverDev const& view = Coreas ? L.coreas_observers[observer] : L.zhs_observers[observer];
-  std::uint64_t const offset = view.waveform_offset;
+  Obs const o = make_obs(view, prop);
   double const coreas_scale = Coreas ? L.coreas_observers[observer].fixed_scale : 0.;
   double const zhs_scale = Zhs ? L.zhs_observers[observer].fixed_scale : 0.;
-  std::uint64_t const nbins = view.number_of_bins;
+  std::uint64_t const nbins = static_cast<std::uint64_t>(o.nbins);
   std::uint32_t const tile_bins =
       tile_begin < nbins ? static_cast<std::uint32_t>(nbins - tile_begin < W ? nbins - tile_begin : W)
                          : 0u;
+  Tile<Fixed> const ctile{coreas_lds, W, static_cast<std::int32_t>(tile_begin),
+                          static_cast<std::int32_t>(tile_bins)};
+  Tile<Fixed> const ztile{zhs_lds, W + 1, static_cast<std::int32_t>(tile_begin),
+                          static_cast<std::int32_t>(tile_bins)};
 
-  unsigned long long counts[5];
-  double abs_sums[2];
-  if constexpr (Exact) {
-    Obs const o = make_obs(view, prop);
-    Tile<Fixed> const ctile{coreas_lds, W, static_cast<std::int32_t>(tile_begin),
-                            static_cast<std::int32_t>(tile_bins)};
-    Tile<Fixed> const ztile{zhs_lds, W + 1, static_cast<std::int32_t>(tile_begin),
-                            static_cast<std::int32_t>(tile_bins)};
-    Tally ctally, ztally;
-    for (std::uint64_t i = chunk_begin + threadIdx.x; i < chunk_end; i += blockDim.x) {
-      Track t;
-      if (!load_track(L.tracks, L.stride, i, t)) continue;
-      if (first_observer_tile) ++ctally.valid;
-      if constexpr (Coreas) {
-        if (tile_bins) coreas_pair(t, prop, o, coreas_scale, ctile, ctally);
-      }
-      if constexpr (Zhs) {
-        zhs_pair(t, prop, L.zhs_refinement, o, zhs_scale, ztile, ztally, bin_tile == 0);
-      }
+  Tally ctally, ztally;
+  for (std::uint64_t i = chunk_begin + threadIdx.x; i < chunk_end; i += blockDim.x) {
+    Track t;
+    if (!load_track(L.tracks, L.stride, i, t)) continue;
+    if (first_observer_tile) ++ctally.valid;
+    if constexpr (Coreas) {
+      if (tile_bins) coreas_pair(t, prop, o, coreas_scale, ctile, ctally);
     }
-    counts[0] = ctally.coreas;
-    counts[1] = ztally.zhs;
-    counts[2] = ztally.subtracks;
-    counts[3] = ctally.valid;
-    counts[4] = ctally.overflow + ztally.overflow;
-    abs_sums[0] = ctally.abs_sum;
-    abs_sums[1] = ztally.abs_sum;
-  } else {
-    fast::View const v = make_view(view, prop, tile_begin, tile_bins, coreas_scale, zhs_scale);
-    fast::Tally tally;
-    std::uint32_t* const near = near_lists[Coreas ? threadIdx.x / 64 : 0];
-    if (prop.homogeneous_index > 0.)
-      fast_chunk<Coreas, Zhs, true, Block>(L, prop, v, chunk_begin, chunk_end, coreas_lds, W, zhs_lds, W + 1,
-                                           first_observer_tile, bin_tile == 0, near, tally);
-    else
-      fast_chunk<Coreas, Zhs, false, Block>(L, prop, v, chunk_begin, chunk_end, coreas_lds, W, zhs_lds, W + 1,
-                                            first_observer_tile, bin_tile == 0, near, tally);
-    counts[0] = tally.coreas;
-    counts[1] = tally.zhs;
-    counts[2] = tally.subtracks + tally.single_subtracks;
-    counts[3] = tally.valid;
-    counts[4] = tally.overflow;
-    abs_sums[0] = tally.coreas_abs;
-    abs_sums[1] = tally.zhs_abs;
-  }
-
-  // one LDS add per wave and tally
-#pragma unroll
-  for (int k = 0; k < 5; ++k) {
-    if ((k == 0 && !Coreas) || ((k == 1 || k == 2) && !Zhs)) continue;
-    unsigned long long const sum = wave_sum(counts[k]);
-    if (threadIdx.x % 64 == 0 && sum) atomicAdd(&block_counts[k], sum);
-  }
-  if constexpr (Fixed) {
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if ((k == 0 && !Coreas) || (k == 1 && !Zhs)) continue;
-      double const sum = wave_sum(abs_sums[k]);
-      if (threadIdx.x % 64 == 0) atomicAdd(&block_abs[k], sum);
+    if constexpr (Zhs) {
+      zhs_pair(t, prop, L.zhs_refinement, o, zhs_scale, ztile, ztally, bin_tile == 0);
     }
   }
+  unsigned long long const counts[5] = {ctally.coreas, ztally.zhs, ztally.subtracks, ctally.valid,
+                                        ctally.overflow + ztally.overflow};
+  double const abs_sums[2] = {ctally.abs_sum, ztally.abs_sum};
+  add_tallies<Coreas, Zhs>(block, counts, abs_sums);
   __syncthreads();
 
   if constexpr (Zhs) {
     for (int c = 0; c < 3; ++c) block_inclusive_scan(zhs_lds + c * (W + 1), W, scan_scratch);
   }
-
-  // Flush the tile into the global waveforms (checked int64 atomics, as
-  // checked_radio_atomic_add; or FP64 atomics in floating mode).
-  unsigned long long flush_overflows = 0;
-  auto flush = [&](Acc const* lds, std::uint32_t row, std::uint32_t bins, void* global,
-                   std::uint64_t total_bins) {
-    Acc* const g = static_cast<Acc*>(global);
-    for (std::uint32_t c = 0; c < 3; ++c) {
-      for (std::uint32_t b = threadIdx.x; b < bins; b += blockDim.x) {
-        Acc const v = lds[c * row + b];
-        if (v == 0) continue;
-        std::uint64_t const at = c * total_bins + offset + tile_begin + b;
-        if constexpr (Fixed) {
-          long long const previous = static_cast<long long>(
-              atomicAdd(reinterpret_cast<unsigned long long*>(g + at),
-                        static_cast<unsigned long long>(v)));
-          if ((v > 0 && previous > 0x7fffffffffffffffLL - v) ||
-              (v < 0 && previous < (-0x7fffffffffffffffLL - 1) - v))
-            ++flush_overflows;
-        } else {
-          atomicAdd(g + at, v);
-        }
-      }
-    }
-  };
-  if constexpr (Coreas) flush(coreas_lds, W, tile_bins, L.coreas_waves, L.coreas_total_bins);
-  if constexpr (Zhs) flush(zhs_lds, W + 1, tile_bins, L.zhs_waves, L.zhs_total_bins);
-  if (flush_overflows) atomicAdd(&block_counts[4], flush_overflows);
+  unsigned long long overflows = 0;
+  std::uint64_t const first = o.offset + tile_begin;
+  if constexpr (Coreas)
+    overflows += flush_tile<Fixed>(coreas_lds, W, tile_bins, L.coreas_waves, L.coreas_total_bins, first);
+  if constexpr (Zhs) overflows += flush_tile<Fixed>(zhs_lds, W + 1, tile_bins, L.zhs_waves, L.zhs_total_bins, first);
+  if (overflows) atomicAdd(&block.counts[4], overflows);
   __syncthreads();
-
-  if (threadIdx.x == 0) {
-    unsigned long long overflow = block_counts[4];
-    // Integer sums are exact modulo 2^64; every LDS partial is bounded by the
-    // sum of |increments|, so a block whose bound reaches 2^63 may have lost
-    // its result and is reported as an overflow (conservatively).
-    if constexpr (Fixed) {
-      if (block_abs[0] >= kIntLimit || block_abs[1] >= kIntLimit) ++overflow;
-    }
-    if (block_counts[0]) atomicAdd(&counters->coreas_contributions, block_counts[0]);
-    if (block_counts[1]) atomicAdd(&counters->zhs_contributions, block_counts[1]);
-    if (block_counts[2]) atomicAdd(&counters->zhs_subtracks, block_counts[2]);
-    if (block_counts[3]) atomicAdd(&counters->valid_tracks, block_counts[3]);
-    if (overflow) atomicAdd(&counters->fixed_point_overflows, overflow);
-  }
+  publish_tallies(block, counters);
 }
 
 // LeptonTransportRecord -> compact track (make_radio_track_kinematics input
@@ -906,10 +669,10 @@ __global__ void __launch_bounds__(256)
   tracks[8 * stride + i] = pid == C8MI_PID_ELECTRON ? -w : w;
 }
 
-template <bool Coreas, bool Zhs, bool Fixed, bool Exact, int Block>
+template <bool Coreas, bool Zhs, bool Fixed, int Block>
 void launch_typed(ProjectionLaunch const& launch, hipStream_t stream, std::size_t lds_bytes,
                   std::uint32_t grid) {
-  auto kernel = radio_project_kernel<Coreas, Zhs, Fixed, Exact, Block>;
+  auto kernel = radio_exact_kernel<Coreas, Zhs, Fixed, Block>;
   static bool attribute_set = false;
   if (!attribute_set) {
     C8MI_HIP(hipFuncSetAttribute(reinterpret_cast<void const*>(kernel),
@@ -921,15 +684,24 @@ void launch_typed(ProjectionLaunch const& launch, hipStream_t stream, std::size_
   C8MI_HIP(hipGetLastError());
 }
 
-template <bool Coreas, bool Zhs, bool Fixed, bool Exact>
+template <bool Coreas, bool Zhs, bool Fixed>
 void launch_block(ProjectionLaunch const& launch, std::uint32_t block, hipStream_t stream,
                   std::size_t lds_bytes, std::uint32_t grid) {
   switch (block) {
-    case 256: launch_typed<Coreas, Zhs, Fixed, Exact, 256>(launch, stream, lds_bytes, grid); break;
-    case 512: launch_typed<Coreas, Zhs, Fixed, Exact, 512>(launch, stream, lds_bytes, grid); break;
-    case 1024: launch_typed<Coreas, Zhs, Fixed, Exact, 1024>(launch, stream, lds_bytes, grid); break;
+    case 256: launch_typed<Coreas, Zhs, Fixed, 256>(launch, stream, lds_bytes, grid); break;
+    case 512: launch_typed<Coreas, Zhs, Fixed, 512>(launch, stream, lds_bytes, grid); break;
+    case 1024: launch_typed<Coreas, Zhs, Fixed, 1024>(launch, stream, lds_bytes, grid); break;
     default: throw std::invalid_argument("radio workgroup size must be 256, 512 or 1024");
   }
+}
+
+template <bool Coreas, bool Zhs>
+void launch_modes(ProjectionLaunch const& launch, bool fixed, bool exact, std::uint32_t block,
+                  hipStream_t stream, std::size_t lds, std::uint32_t grid) {
+  // FP64 (non-deterministic) accumulation is offered in the exact form only.
+  if (!fixed) launch_block<Coreas, Zhs, false>(launch, block, stream, lds, grid);
+  else if (exact) launch_block<Coreas, Zhs, true>(launch, block, stream, lds, grid);
+  else launch_fast(launch, Coreas, Zhs, block, grid, stream);
 }
 
 }  // namespace
@@ -940,23 +712,14 @@ std::size_t projection_lds_bytes(bool coreas, bool zhs, std::uint32_t tile_bins)
 }
 
 std::uint32_t projection_grid(ProjectionLaunch const& launch) {
-  std::uint64_t const per_chunk =
-      static_cast<std::uint64_t>(launch.observer_count) * launch.bin_tiles;
+  std::uint64_t const groups = (launch.observer_count + launch.group - 1) / launch.group;
   std::uint64_t const chunk_rounds = (launch.chunks + kXcds - 1) / kXcds;
-  return static_cast<std::uint32_t>(chunk_rounds * kXcds * per_chunk);
-}
-
-template <bool Coreas, bool Zhs>
-void launch_modes(ProjectionLaunch const& launch, bool fixed, bool exact, std::uint32_t block,
-                  hipStream_t stream, std::size_t lds, std::uint32_t grid) {
-  // FP64 (non-deterministic) accumulation is offered in the exact form only.
-  if (!fixed) launch_block<Coreas, Zhs, false, true>(launch, block, stream, lds, grid);
-  else if (exact) launch_block<Coreas, Zhs, true, true>(launch, block, stream, lds, grid);
-  else launch_block<Coreas, Zhs, true, false>(launch, block, stream, lds, grid);
+  return static_cast<std::uint32_t>(chunk_rounds * kXcds * groups * launch.bin_tiles);
 }
 
 void launch_projection(ProjectionLaunch const& launch, bool coreas, bool zhs, bool fixed,
-                       bool exact, std::uint32_t block, hipStream_t stream) {
+                       bool exact, hipStream_t stream) {
+  std::uint32_t const block = launch.block_threads;
   if (launch.track_count == 0 || launch.observer_count == 0) return;
   std::size_t const lds = projection_lds_bytes(coreas, zhs, launch.tile_bins);
   std::uint32_t const grid = projection_grid(launch);
@@ -966,7 +729,8 @@ void launch_projection(ProjectionLaunch const& launch, bool coreas, bool zhs, bo
 }
 
 void launch_pooled_projection(ProjectionLaunch const& launch, bool coreas, bool zhs, bool exact,
-                              std::uint32_t block, std::uint32_t grid, hipStream_t stream) {
+                              std::uint32_t grid, hipStream_t stream) {
+  std::uint32_t const block = launch.block_threads;
   if (launch.track_count == 0 || grid == 0) return;
   std::size_t const lds = projection_lds_bytes(coreas, zhs, launch.tile_bins);
   if (coreas && zhs) launch_modes<true, true>(launch, true, exact, block, stream, lds, grid);

@@ -22,13 +22,24 @@ inline constexpr std::size_t kMaxDynamicLdsBytes = 144 * 1024;
 // 2048-bin tiles; a 1024-bin CoREAS+ZHS window (48 KiB of bins) and a 2048-bin
 // ZHS window keep one tile.
 inline constexpr std::size_t kPreferredWorkgroupLdsBytes = 53 * 1024;
-// Upper bound of the projection kernel's static LDS: the wave totals of the ZHS
-// scan (16 x 8 B for 1024 threads), block counters and |increment| sums; with
-// CoREAS also the Cherenkov lists of 512 threads' waves (8 x 512 B).
+// Upper bound of a projection kernel's static LDS beside the pair lists: the
+// wave totals of the ZHS scan (16 x 8 B for 1024 threads), counters and sums.
 inline constexpr std::size_t kProjectionStaticLdsBytes = 256;
-inline constexpr std::size_t kCoreasStaticLdsBytes = 4096;
+// Pair lists of the fast CoREAS kernels, bytes per thread (512 per wave).
+inline constexpr std::size_t kPairListBytesPerThread = 8;
+// LDS of a CU; what a fast workgroup holds beside its window tiles, and the most
+// its tiles may take.
+inline constexpr std::size_t kCuLdsBytes = 160 * 1024;
+inline constexpr std::size_t fast_static_lds(bool coreas, std::uint32_t threads) {
+  return kProjectionStaticLdsBytes + (coreas ? kPairListBytesPerThread * threads : 0u);
+}
+inline constexpr std::size_t fast_dynamic_lds_limit(bool coreas, std::uint32_t threads) {
+  return kCuLdsBytes - fast_static_lds(coreas, threads);
+}
+// Most observers of a group.
+inline constexpr std::uint32_t kMaxGroup = 8;
 // Most tracks a workgroup takes (its tallies and lists use 32-bit words).
-inline constexpr std::uint64_t kMaxChunkTracks = std::uint64_t{1} << 30;
+inline constexpr std::uint64_t kMaxChunkTracks = std::uint64_t{1} << 27;
 // Tracks per workgroup the default chunking gives a batch large enough for
 // eight such chunks, at least (a smaller batch is cut into eight chunks).
 inline constexpr std::uint64_t kMinimumDefaultChunk = 32768;
@@ -51,13 +62,14 @@ struct LaunchTuning {
   std::uint64_t chunk_tracks = 0;
   std::uint32_t tile_bins_limit = 0;
   std::uint32_t target_workgroups = 8192;
-  std::uint32_t block_threads = 512;
+  std::uint32_t block_threads = 0;  // 0: by the launch's shape
 };
 
-// Fills the tile and chunk fields of `L` (tile_bins, bin_tiles, chunk_size,
-// chunks) for `count` tracks on `observers` observers whose longest window has
-// `max_bins` bins. Throws length_error when the grid exceeds 2^32 workgroups.
-void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, std::uint32_t observers,
+// Fills the shape fields of `L` (tile_bins, bin_tiles, chunk_size, chunks, group,
+// block_threads) for `count` tracks on `observers` observers whose longest window
+// has `max_bins` bins; `fast`: the fast kernels (groups of observers). Throws
+// length_error when the grid exceeds 2^32 workgroups.
+void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std::uint32_t observers,
                       std::uint64_t max_bins, std::uint64_t count, LaunchTuning const& tuning);
 
 // LDS bytes for one workgroup holding `tile_bins` bins of each enabled mode.
@@ -68,12 +80,16 @@ std::uint32_t projection_grid(ProjectionLaunch const& launch);
 // exact: the reference's FP64 operation order (bit-identical fixed-point
 // sums); otherwise the fast FP64 form. Floating accumulation is always exact.
 void launch_projection(ProjectionLaunch const& launch, bool coreas, bool zhs, bool fixed,
-                       bool exact, std::uint32_t block, hipStream_t stream);
+                       bool exact, hipStream_t stream);
 
 // Pooled showers (launch.segments set): `grid` workgroups, an upper bound on
 // the items (*launch.item_count); int64 fixed point.
 void launch_pooled_projection(ProjectionLaunch const& launch, bool coreas, bool zhs, bool exact,
-                              std::uint32_t block, std::uint32_t grid, hipStream_t stream);
+                              std::uint32_t grid, hipStream_t stream);
+
+// The fast kernels (int64 fixed point), launch.group observers per workgroup.
+void launch_fast(ProjectionLaunch const& launch, bool coreas, bool zhs, std::uint32_t block, std::uint32_t grid,
+                 hipStream_t stream);
 
 void launch_records_to_tracks(c8mi_lepton_transport_record const* records,
                               std::uint64_t count, double* tracks, std::uint64_t stride,

@@ -106,10 +106,10 @@ void project_fixed_noalloc(c8mi_radio_config const& config, double const* device
   std::vector<ObserverDev> coreas_host, zhs_host;
   if (coreas)
     coreas_host = make_observers(config.coreas_observers, config.coreas_observer_count, limit,
-                                 false, coreas_bins, coreas_max);
+                                 false, p, coreas_bins, coreas_max);
   if (zhs)
     zhs_host = make_observers(config.zhs_observers, config.zhs_observer_count, limit, true,
-                              zhs_bins, zhs_max);
+                              p, zhs_bins, zhs_max);
 
   unsigned char* const base = scratch_address();
   auto* const device_counters = reinterpret_cast<CountersDev*>(base);
@@ -147,7 +147,7 @@ void project_fixed_noalloc(c8mi_radio_config const& config, double const* device
     L.zhs_refinement = config.zhs_subtrack_refinement;
     L.propagation = propagation_view(p, refractivity, integrated);
     L.counters = device_counters;
-    shape_projection(L, c, z, observers, c ? coreas_max : zhs_max, count, tuning);
+    shape_projection(L, c, z, !config.exact_fp64, observers, c ? coreas_max : zhs_max, count, tuning);
     L.tracks = device_tracks;
     L.stride = stride;
     L.track_count = count;
@@ -159,7 +159,7 @@ void project_fixed_noalloc(c8mi_radio_config const& config, double const* device
     L.zhs_total_bins = zhs_bins;
     L.count_valid = first ? 1u : 0u;
     first = false;
-    launch_projection(L, c, z, true, config.exact_fp64 != 0, tuning.block_threads, stream);
+    launch_projection(L, c, z, true, config.exact_fp64 != 0, stream);
   };
   if (count != 0) {
     if (coreas) run(true, false);

@@ -56,21 +56,68 @@ __device__ __forceinline__ double reciprocal_sqrt(double x) {
   return fma(y, e * fma(0.375, e, 0.5), y);
 }
 
-// What a workgroup knows of its observer and window tile (uniform).
+// One observer and window tile. Workgroups hold the same observers in every
+// wave, so the fields of a uniform view come from scalar loads.
 struct View {
   V3 position;
   double start, end, rate, grid, two_pi_over_wavelength;
   double tile_begin, tile_end;  // bins of the tile, [begin, end)
-  double table_last;            // last propagation-table entry
   double destination_height, destination_index;
   double n_destination, integrated_destination;
-  double coreas_scale, zhs_scale;
+  double scale;  // fixed-point scale of the algorithm
 };
+
+// A point of a track and what the propagation table says at it, shared by all
+// observers of the workgroup (the two table gathers of a point cost more than
+// the rest of its propagation: one L2 line per lane each).
+struct Source {
+  V3 at;
+  double index, integrated;
+  double height;  // table cell, or the height of a point off the table
+};
+enum SourceKind : std::uint32_t { kInside = 0, kAbove = 1, kAtZero = 2, kBelow = 3 };
+
+template <bool Homogeneous>
+__device__ __forceinline__ Source make_source(PropagationDev const& p, V3 at, std::uint32_t& kind) {
+  Source s;
+  s.at = at;
+  kind = kInside;
+  if constexpr (Homogeneous) {
+    s.index = p.homogeneous_index;
+    s.integrated = s.height = 0.;
+    return s;
+  }
+  double const height = (at.z - p.minimum_height) * p.inverse_step;
+  std::uint64_t const last = p.table_size - 1;
+  if (height > 0. && height + 0.5 < static_cast<double>(last)) {
+    // the table has fewer than 2^32 entries (checked on the host)
+    std::uint32_t const cell = static_cast<std::uint32_t>(height + 0.5);
+    s.index = p.refractivity[cell] + 1.;
+    s.integrated = p.integrated[cell];
+    s.height = static_cast<double>(cell);
+  } else if (height + 0.5 >= static_cast<double>(last)) {
+    kind = kAbove;
+    s.index = p.refractivity[last] + p.slope_n_upper * fabs((at.z - p.maximum_height) * p.inverse_step) + 1.;
+    s.integrated = p.integrated[last] + p.slope_i_upper * fabs(p.maximum_height - at.z);
+    s.height = height;
+  } else if (height == 0.) {
+    kind = kAtZero;
+    s.index = 1.;
+    s.integrated = p.integrated[0];
+    s.height = height;
+  } else {
+    kind = kBelow;
+    s.index = p.refractivity[0] + p.slope_n_lower * fabs(height) + 1.;
+    s.integrated = p.integrated[0] + p.slope_i_lower * fabs(height);
+    s.height = fabs(height);
+  }
+  return s;
+}
 
 struct Track {
   V3 start, end, beta;
   double t0, t1, duration;
-  double constant;  // charge x weight / (4 pi eps0 c)
+  double amplitude;  // charge x weight / (4 pi eps0 c)
 };
 
 // `base`: the batch's tracks from the workgroup's current position on, `lane`
@@ -81,7 +128,7 @@ __device__ __forceinline__ bool load_track(double const* __restrict__ base, std:
   t.end = {(base + 3 * stride)[lane], (base + 4 * stride)[lane], (base + 5 * stride)[lane]};
   t.t0 = (base + 6 * stride)[lane];
   t.t1 = (base + 7 * stride)[lane];
-  t.constant = kChargeEm * (base + 8 * stride)[lane];
+  t.amplitude = kChargeEm * (base + 8 * stride)[lane];
   t.duration = t.t1 - t.t0;
   V3 const d{t.end.x - t.start.x, t.end.y - t.start.y, t.end.z - t.start.z};
   if (!(t.duration > 0.) || !(dot(d, d) > 0.)) return false;
@@ -93,66 +140,48 @@ __device__ __forceinline__ bool load_track(double const* __restrict__ base, std:
   t.beta = {d.x * r, d.y * r, d.z * r};
   return true;
 }
+__device__ __forceinline__ V3 midpoint(Track const& t) {
+  return {(t.start.x + t.end.x) * 0.5, (t.start.y + t.end.y) * 0.5, (t.start.z + t.end.z) * 0.5};
+}
 
 struct Path {
-  double time, n_source, n_destination, inv_distance;
+  double time, inv_distance;
   V3 emit;
 };
 
-// Sources above, at or below the ends of the propagation table (the
-// reference's edge branches; RadioProjection.inl:170-238).
-__device__ __forceinline__ double edge_mean_index(PropagationDev const& p, View const& o, double source_z,
-                                                  double source_height, double& n_source,
-                                                  double& n_destination) {
-  std::uint64_t const last = p.table_size - 1;
-  double integrated, height;
-  if (source_height + 0.5 >= o.table_last) {
-    n_source = p.refractivity[last] + p.slope_n_upper * fabs((source_z - p.maximum_height) * p.inverse_step) + 1.;
-    integrated = p.integrated[last] + p.slope_i_upper * fabs(p.maximum_height - source_z);
-    height = source_height - o.destination_height;
-  } else if (source_height == 0.) {
-    n_source = 1.;
-    n_destination = 1.;
-    integrated = p.integrated[0];
-    height = o.destination_height - source_height;
-  } else {
-    n_source = p.refractivity[0] + p.slope_n_lower * fabs(source_height) + 1.;
-    integrated = p.integrated[0] + p.slope_i_lower * fabs(source_height);
-    n_destination = 1.;
-    height = o.destination_height - fabs(source_height);
-  }
-  return 1. + (integrated - o.integrated_destination) / height;
+// The reference's edge branches (RadioProjection.inl:170-238).
+__device__ __forceinline__ double edge_mean_index(View const& o, Source const& s, std::uint32_t kind) {
+  double const span = kind == kAbove ? s.height - o.destination_height : o.destination_height - s.height;
+  return 1. + (s.integrated - o.integrated_destination) / span;
 }
 
 template <bool Homogeneous>
-__device__ __forceinline__ Path propagate(PropagationDev const& p, View const& o, V3 source) {
+__device__ __forceinline__ Path propagate(PropagationDev const& p, View const& o, Source const& s,
+                                          std::uint32_t kind) {
   Path r;
-  V3 const d{o.position.x - source.x, o.position.y - source.y, o.position.z - source.z};
+  V3 const d{o.position.x - s.at.x, o.position.y - s.at.y, o.position.z - s.at.z};
   double const r2 = dot(d, d);
   r.inv_distance = reciprocal_sqrt(r2);
   r.emit = {d.x * r.inv_distance, d.y * r.inv_distance, d.z * r.inv_distance};
   double const flight = (r2 * r.inv_distance) * kInvC;
   if constexpr (Homogeneous) {
-    r.n_source = r.n_destination = p.homogeneous_index;
-    r.time = p.homogeneous_index * flight;
+    r.time = s.index * flight;
     return r;
   }
-  double const height = (source.z - p.minimum_height) * p.inverse_step;
-  double mean;
-  r.n_destination = o.n_destination;
-  if (height > 0. && height + 0.5 < o.table_last) {
-    // the table has fewer than 2^32 entries (checked on the host)
-    std::uint32_t const at = static_cast<std::uint32_t>(height + 0.5);
-    r.n_source = p.refractivity[at] + 1.;
-    double const difference = p.integrated[at] - o.integrated_destination;
-    double const cells = static_cast<double>(at) - o.destination_index;
-    double const span = cells == 0. ? 1. : cells * p.step;
-    mean = fma(difference, reciprocal(span), 1.);
-  } else {
-    mean = edge_mean_index(p, o, source.z, height, r.n_source, r.n_destination);
-  }
+  double const cells = s.height - o.destination_index;
+  double const span = cells == 0. ? 1. : cells * p.step;
+  double mean = fma(s.integrated - o.integrated_destination, reciprocal(span), 1.);
+  if (kind != kInside) mean = edge_mean_index(o, s, kind);
   r.time = mean * flight;
   return r;
+}
+
+// Index at the observer as the reference's propagation gives it: 1 for sources
+// at or below the table's lower end.
+template <bool Homogeneous>
+__device__ __forceinline__ double index_at_destination(PropagationDev const& p, View const& o, std::uint32_t kind) {
+  if constexpr (Homogeneous) return p.homogeneous_index;
+  return kind >= kAtZero ? 1. : o.n_destination;
 }
 
 // 1 - n b.e, with error-free products and sums where it cancels to zero.
@@ -271,20 +300,23 @@ __device__ __forceinline__ V3 transverse(V3 emit, V3 beta, double beta_emit, dou
 // returns true without adding anything where one does (`forward`: the start
 // arrives before the end), for coreas_near.
 template <bool Homogeneous>
-__device__ __forceinline__ bool coreas_far(Track const& t, PropagationDev const& p, View const& o,
-                                           long long* tile, std::uint32_t stride, Tally& tally, bool& forward) {
-  Path const ps = propagate<Homogeneous>(p, o, t.start);
-  Path const pe = propagate<Homogeneous>(p, o, t.end);
+__device__ __forceinline__ bool coreas_far(Track const& t, Source const& start, std::uint32_t start_kind,
+                                           Source const& end, std::uint32_t end_kind, PropagationDev const& p,
+                                           View const& o, long long* tile, std::uint32_t stride, Tally& tally,
+                                           bool& forward) {
+  Path const ps = propagate<Homogeneous>(p, o, start, start_kind);
+  Path const pe = propagate<Homogeneous>(p, o, end, end_kind);
   double const bs = dot(t.beta, ps.emit), be = dot(t.beta, pe.emit);
-  double const pre = doppler(ps.n_source, t.beta, ps.emit, bs);
-  double const post = doppler(pe.n_source, t.beta, pe.emit, be);
+  double const pre = doppler(start.index, t.beta, ps.emit, bs);
+  double const post = doppler(end.index, t.beta, pe.emit, be);
   double start_receive = t.t0 + ps.time;
   double end_receive = t.t1 + pe.time;
-  if (ps.n_destination > 1. && (fabs(pre) < kCoreasThreshold || fabs(post) < kCoreasThreshold)) {
+  if (index_at_destination<Homogeneous>(p, o, start_kind) > 1. &&
+      (fabs(pre) < kCoreasThreshold || fabs(post) < kCoreasThreshold)) {
     forward = start_receive < end_receive;
     return true;
   }
-  double const q = t.constant * o.rate * o.coreas_scale;
+  double const q = t.amplitude * o.rate * o.scale;
   V3 fs = transverse(ps.emit, t.beta, bs, q * ps.inv_distance * reciprocal(pre));
   V3 fe = transverse(pe.emit, t.beta, be, -(q * pe.inv_distance * reciprocal(post)));
   if (pre < 1.e-9 || post < 1.e-9) {
@@ -305,15 +337,16 @@ __device__ __forceinline__ bool coreas_far(Track const& t, PropagationDev const&
 template <bool Homogeneous>
 __device__ __forceinline__ void coreas_near(Track const& t, PropagationDev const& p, View const& o,
                                             long long* tile, std::uint32_t stride, Tally& tally, bool forward) {
-  V3 const midpoint{(t.start.x + t.end.x) * 0.5, (t.start.y + t.end.y) * 0.5, (t.start.z + t.end.z) * 0.5};
-  Path const pm = propagate<Homogeneous>(p, o, midpoint);
-  double const middle = (t.t0 + t.t1) * 0.5 + pm.time;
+  std::uint32_t kind;
+  Source const middle = make_source<Homogeneous>(p, midpoint(t), kind);
+  Path const pm = propagate<Homogeneous>(p, o, middle, kind);
+  double const middle_receive = (t.t0 + t.t1) * 0.5 + pm.time;
   double const bm = dot(t.beta, pm.emit);
-  double const md = doppler(pm.n_source, t.beta, pm.emit, bm);
-  V3 f = transverse(pm.emit, t.beta, bm, t.constant * o.rate * o.coreas_scale * pm.inv_distance * reciprocal(md));
+  double const md = doppler(middle.index, t.beta, pm.emit, bm);
+  V3 f = transverse(pm.emit, t.beta, bm, t.amplitude * o.rate * o.scale * pm.inv_distance * reciprocal(md));
   double const half = 0.5 * (t.duration * fabs(md));
-  double start_receive = forward ? middle - half : middle + half;
-  double end_receive = forward ? middle + half : middle - half;
+  double start_receive = forward ? middle_receive - half : middle_receive + half;
+  double end_receive = forward ? middle_receive + half : middle_receive - half;
   double const delta = end_receive - start_receive;
   if (fabs(delta) < o.grid) {
     f = scaled(f, fabs(delta * o.rate));
@@ -345,61 +378,106 @@ __device__ __forceinline__ void add_segment_row(long long* row, std::int32_t bin
   add(l2 + 1, 0ull - l);
 }
 
-// One ZHS segment from its midpoint's path: half_duration either side of
-// middle_time. `subdivided` keeps the reference's sign of the middle bins.
-__device__ __forceinline__ void zhs_segment(Path const& path, double beta_emit, double middle_time,
+// Arrival of a ZHS segment in bins of the observer: centre -+ spread.
+struct Arrival {
+  double x1, x2, b1, b2, den;
+};
+__device__ __forceinline__ Arrival segment_arrival(Path const& path, double index, double beta_emit,
+                                                   double middle_time, double half_duration, View const& o) {
+  Arrival a;
+  a.den = fma(-index, beta_emit, 1.);
+  double const spread = half_duration * fabs(a.den);
+  double const centre = middle_time + path.time;
+  a.x1 = ((centre - spread) - o.start) * o.rate;
+  a.x2 = ((centre + spread) - o.start) * o.rate;
+  a.b1 = nearest_bin(a.x1);
+  a.b2 = nearest_bin(a.x2);
+  return a;
+}
+
+// A segment over one bin or two neighbouring ones, as the difference array's
+// entries at the first bin and the two after it. u: e x (b x e) times the
+// amplitude over the distance; in one bin the denominator cancels and the
+// potential is u times the duration.
+__device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival const& a, View const& o,
+                                                  long long* tile, std::uint32_t stride, Tally& tally) {
+  bool const two = a.b1 != a.b2;
+  double const k = reciprocal(fabs(a.den));
+  std::int32_t const bins = static_cast<std::int32_t>(o.tile_end - o.tile_begin);
+  std::int32_t const at = static_cast<std::int32_t>(a.b1 - o.tile_begin);  // -1 .. bins - 1
+  bool const has_first = at >= 0, has_last = two && at + 1 < bins;
+  // a part without its bin in this tile takes no part in the sums
+  double const first = !has_first ? 0. : two ? (a.b1 + 0.5 - a.x1) * k : duration * o.rate;
+  double const last = has_last ? (a.x2 + 0.5 - a.b2) * k : 0.;
+  double const bound = (fabs(u.x) + fabs(u.y) + fabs(u.z)) * (fabs(first) + fabs(last));
+  std::uint32_t const base = at > 0 ? static_cast<std::uint32_t>(at) : 0u;
+  std::uint32_t const n = (has_first ? 1u : 0u) + (has_last ? 1u : 0u);
+  if (bound < kShiftLimit) {
+    tally.zhs_abs += bound;
+    double const us[3] = {u.x, u.y, u.z};
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      long long* const row = tile + c * stride + base;
+      long long const f = increment(us[c] * first), l = increment(us[c] * last);
+      if (has_first) {
+        lds_add(row, f);
+        lds_add(row + 1, l - f);
+        if (has_last) lds_add(row + 2, -l);
+      } else {
+        lds_add(row, l);
+        lds_add(row + 1, -l);
+      }
+    }
+    tally.zhs += n;
+    return;
+  }
+  double const us[3] = {u.x, u.y, u.z};
+  bool vf = true, vl = true;
+  for (int c = 0; c < 3; ++c) {
+    long long* const row = tile + c * stride;
+    long long f = 0, l = 0;
+    if (has_first) {
+      bool const ok = checked_increment(us[c] * first, f, tally.zhs_abs);
+      vf = vf && ok;
+      if (ok) {
+        lds_add(row + at, f);
+        lds_add(row + at + 1, -f);
+      }
+    }
+    if (has_last) {
+      bool const ok = checked_increment(us[c] * last, l, tally.zhs_abs);
+      vl = vl && ok;
+      if (ok) {
+        lds_add(row + at + 1, l);
+        lds_add(row + at + 2, -l);
+      }
+    }
+  }
+  unsigned long long const nf = has_first ? 1ull : 0ull, nl = has_last ? 1ull : 0ull;
+  tally.zhs += (vf ? nf : 0ull) + (vl ? nl : 0ull);
+  tally.overflow += (vf ? 0ull : nf) + (vl ? 0ull : nl);
+}
+
+// One ZHS segment of any length. `subdivided` keeps the reference's sign of the
+// middle bins.
+__device__ __forceinline__ void zhs_segment(Path const& path, double index, double beta_emit, double middle_time,
                                             double half_duration, Track const& t, View const& o,
                                             long long* tile, std::uint32_t stride, Tally& tally,
                                             bool subdivided) {
-  double const den = fma(-path.n_source, beta_emit, 1.);
-  double const spread = half_duration * fabs(den);
-  double const centre = middle_time + path.time;
-  double const x1 = ((centre - spread) - o.start) * o.rate;
-  double const x2 = ((centre + spread) - o.start) * o.rate;
-  double const b1 = nearest_bin(x1), b2 = nearest_bin(x2);
-  if (!(b2 >= o.tile_begin && b1 < o.tile_end)) return;
-  double const base = t.constant * path.inv_distance * o.zhs_scale;
-  // e x (b x e)
-  V3 const u = transverse(path.emit, t.beta, beta_emit, -base);
-  if (b1 == b2) {
-    V3 const c = scaled(u, 2. * half_duration * o.rate);
-    std::uint32_t const at = static_cast<std::uint32_t>(b2 - o.tile_begin);
-    double const magnitude = fabs(c.x) + fabs(c.y) + fabs(c.z);
-    if (magnitude < kShiftLimit) {
-      tally.zhs_abs += magnitude;
-      long long const ix = increment(c.x), iy = increment(c.y), iz = increment(c.z);
-      lds_add(tile + at, ix);
-      lds_add(tile + at + 1, -ix);
-      lds_add(tile + stride + at, iy);
-      lds_add(tile + stride + at + 1, -iy);
-      lds_add(tile + 2 * stride + at, iz);
-      lds_add(tile + 2 * stride + at + 1, -iz);
-      ++tally.zhs;
-      return;
-    }
-    double const cs[3] = {c.x, c.y, c.z};
-    bool valid = true;
-    for (int k = 0; k < 3; ++k) {
-      long long inc = 0;
-      if (checked_increment(cs[k], inc, tally.zhs_abs)) {
-        lds_add(tile + k * stride + at, inc);
-        lds_add(tile + k * stride + at + 1, -inc);
-      } else {
-        valid = false;
-      }
-    }
-    tally.zhs += valid ? 1ull : 0ull;
-    tally.overflow += valid ? 0ull : 1ull;
+  Arrival const a = segment_arrival(path, index, beta_emit, middle_time, half_duration, o);
+  if (!(a.b2 >= o.tile_begin && a.b1 < o.tile_end)) return;
+  V3 const u = transverse(path.emit, t.beta, beta_emit, -(t.amplitude * path.inv_distance * o.scale));
+  if (a.b2 - a.b1 <= 1.) {
+    add_short_segment(u, 2. * half_duration, a, o, tile, stride, tally);
     return;
   }
   std::int32_t const bins = static_cast<std::int32_t>(o.tile_end - o.tile_begin);
   // two bins either side of the tile tell everything the clipping needs
-  std::int32_t const l1 = static_cast<std::int32_t>(fmax(b1 - o.tile_begin, -2.));
-  std::int32_t const l2 = static_cast<std::int32_t>(fmin(b2 - o.tile_begin, static_cast<double>(bins) + 1.));
-  double const k = reciprocal(fabs(den));
-  V3 const edge = scaled(u, k);
-  double const first = fabs(b1 + 0.5 - x1), last = fabs(x2 + 0.5 - b2);
-  double const sign = subdivided && den < 0. ? -1. : 1.;
+  std::int32_t const l1 = static_cast<std::int32_t>(fmax(a.b1 - o.tile_begin, -2.));
+  std::int32_t const l2 = static_cast<std::int32_t>(fmin(a.b2 - o.tile_begin, static_cast<double>(bins) + 1.));
+  V3 const edge = scaled(u, reciprocal(fabs(a.den)));
+  double const first = fabs(a.b1 + 0.5 - a.x1), last = fabs(a.x2 + 0.5 - a.b2);
+  double const sign = subdivided && a.den < 0. ? -1. : 1.;
   bool const has_first = l1 >= 0, has_last = l2 < bins;
   std::int32_t const middle_bins = (l2 < bins ? l2 : bins) - (l1 + 1 > 0 ? l1 + 1 : 0);
   bool const has_middle = l2 - l1 > 1 && middle_bins > 0;
@@ -420,25 +498,32 @@ __device__ __forceinline__ void zhs_segment(Path const& path, double beta_emit, 
   tally.overflow += (vf ? 0ull : nf) + (vm ? 0ull : nm) + (vl ? 0ull : nl);
 }
 
+// The Fraunhofer measure of a track (RadioProjection.inl:482-529): above one it
+// is subdivided. sin^2 L^2 = L^2 - (d.e)^2 with d = beta c duration.
+__device__ __forceinline__ double fraunhofer(Path const& path, double beta_emit, double duration, double length2,
+                                             View const& o) {
+  double const along = beta_emit * (kC * duration);
+  return fma(-along, along, length2) * path.inv_distance * o.two_pi_over_wavelength;
+}
+
+// The ZHS update of a track from its midpoint (`length2`: its squared length).
 template <bool Homogeneous>
-__device__ __forceinline__ void zhs_update(Track const& t, PropagationDev const& p, std::uint32_t refinement,
-                                           View const& o, long long* tile, std::uint32_t stride, Tally& tally,
+__device__ __forceinline__ void zhs_update(Track const& t, Source const& middle, std::uint32_t kind, double length2,
+                                           PropagationDev const& p, std::uint32_t refinement, View const& o,
+                                           long long* tile, std::uint32_t stride, Tally& tally,
                                            bool count_subtracks) {
-  V3 const midpoint{(t.start.x + t.end.x) * 0.5, (t.start.y + t.end.y) * 0.5, (t.start.z + t.end.z) * 0.5};
-  Path const mp = propagate<Homogeneous>(p, o, midpoint);
-  V3 const d{t.end.x - t.start.x, t.end.y - t.start.y, t.end.z - t.start.z};
-  // sin^2 L^2 from the direction of the displacement: L^2 - (d.e)^2
-  double const along = dot(d, mp.emit);
-  double const fraunhofer = fma(-along, along, dot(d, d)) * mp.inv_distance * o.two_pi_over_wavelength;
-  if (!(fraunhofer > 1.) && refinement <= 1u) {
+  Path const mp = propagate<Homogeneous>(p, o, middle, kind);
+  double const bm = dot(t.beta, mp.emit);
+  double const measure = fraunhofer(mp, bm, t.duration, length2, o);
+  if (!(measure > 1.) && refinement <= 1u) {
     if (count_subtracks) ++tally.single_subtracks;
-    zhs_segment(mp, dot(t.beta, mp.emit), (t.t0 + t.t1) * 0.5, t.duration * 0.5, t, o, tile, stride, tally, false);
+    zhs_segment(mp, middle.index, bm, (t.t0 + t.t1) * 0.5, t.duration * 0.5, t, o, tile, stride, tally, false);
     return;
   }
   double divisor = 1.;
   int nsub = 1;
-  if (fraunhofer > 1.) {
-    divisor = sqrt(fraunhofer) + 1.;
+  if (measure > 1.) {
+    divisor = sqrt(measure) + 1.;
     nsub = static_cast<int>(ceil(divisor));
   }
   int const refine = static_cast<int>(refinement);
@@ -448,16 +533,19 @@ __device__ __forceinline__ void zhs_update(Track const& t, PropagationDev const&
   }
   int const segments = nsub * refine;
   double const parts = divisor * static_cast<double>(refine);
-  V3 const step{d.x / parts, d.y / parts, d.z / parts};
+  V3 const step{(t.end.x - t.start.x) / parts, (t.end.y - t.start.y) / parts, (t.end.z - t.start.z) / parts};
   double const dt = t.duration / parts;
   V3 p1 = t.start;
   double time1 = t.t0;
   for (int i = 0; i < segments; ++i) {
     V3 const p2{p1.x + step.x, p1.y + step.y, p1.z + step.z};
     double const time2 = time1 + dt;
-    Path const path = propagate<Homogeneous>(p, o, {(p1.x + p2.x) * 0.5, (p1.y + p2.y) * 0.5, (p1.z + p2.z) * 0.5});
-    zhs_segment(path, dot(t.beta, path.emit), (time1 + time2) * 0.5, (time2 - time1) * 0.5, t, o, tile, stride,
-                tally, true);
+    std::uint32_t part_kind;
+    Source const part =
+        make_source<Homogeneous>(p, {(p1.x + p2.x) * 0.5, (p1.y + p2.y) * 0.5, (p1.z + p2.z) * 0.5}, part_kind);
+    Path const path = propagate<Homogeneous>(p, o, part, part_kind);
+    zhs_segment(path, part.index, dot(t.beta, path.emit), (time1 + time2) * 0.5, (time2 - time1) * 0.5, t, o, tile,
+                stride, tally, true);
     p1 = p2;
     time1 = time2;
   }

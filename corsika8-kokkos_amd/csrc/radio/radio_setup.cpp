@@ -64,7 +64,7 @@ void validate_radio_config(c8mi_radio_config const& config) {
 
 // RadioAccumulator::makeObservers (RadioAccumulator.inl:591-617).
 std::vector<ObserverDev> make_observers(c8mi_radio_observer const* input, std::uint64_t count,
-                                        double limit, bool zhs_potential,
+                                        double limit, bool zhs_potential, c8mi_radio_propagation const& p,
                                         std::uint64_t& total_bins, std::uint64_t& max_bins) {
   std::vector<ObserverDev> result;
   result.reserve(count);
@@ -81,6 +81,17 @@ std::vector<ObserverDev> make_observers(c8mi_radio_observer const* input, std::u
     d.fixed_scale = kHeadroom * potential_factor / limit;
     d.number_of_bins = o.number_of_bins;
     d.waveform_offset = total_bins;
+    d.end_time = d.start_time + d.duration;
+    d.grid = 1. / d.sample_rate;
+    d.two_pi_over_wavelength = 2. * 3.141592653589793238462643383279502884 / (299792458. / d.sample_rate);
+    d.n_destination = 1.;
+    if (!(p.homogeneous_refractive_index > 0.)) {  // positions inside the table were checked
+      d.destination_height = (d.position[2] - p.minimum_height_m) * p.inverse_step_per_m;
+      auto const cell = static_cast<std::uint64_t>(d.destination_height + 0.5);
+      d.destination_index = static_cast<double>(cell);
+      d.n_destination = p.refractivity[cell] + 1.;
+      d.integrated_destination = p.integrated_refractivity[cell];
+    }
     if (o.number_of_bins > std::numeric_limits<std::uint64_t>::max() - total_bins)
       throw std::overflow_error("radio waveform bin overflow");
     total_bins += o.number_of_bins;
@@ -122,50 +133,125 @@ PropagationDev propagation_view(c8mi_radio_propagation const& p, double const* r
   return d;
 }
 
-void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, std::uint32_t observers,
+namespace {
+
+// The launch shape of a fast projection: window tiles of an observer, observers
+// of a workgroup (its tiles share the CU's LDS: one workgroup of 1024 threads, or
+// two of 512 with one tile each) and track chunks (a multiple of eight: chunk c
+// runs on XCD c % 8). A workgroup's time is its tracks times the cost of an
+// update, plus clearing and flushing its tiles; the launch takes as many rounds
+// as 256 CUs need for its workgroups, so a shape that just fills its rounds wins
+// over one that leaves the last round empty.
+//
+// Costs, measured with 2^20 tracks on 160 antennas and 1024 and 2048 bins at 0.2
+// ns: nanoseconds of a CU per track and observer with one observer a workgroup,
+// and the share of it left with g (the track's loads, table gathers and velocity
+// are paid once per workgroup). The estimate ordered the measured times of 26
+// shapes of 40000 to 2^20 tracks, 40 to 160 antennas and 333 to 4096 bins except
+// where two lay within 5%.
+constexpr double kCoreasNs = 5.0, kZhsNs = 2.75;
+constexpr double kCoreasShare[kMaxGroup] = {1., .59, .51, .475, .46, .445, .435, .43};
+constexpr double kZhsShare[kMaxGroup] = {1., .84, .755, .71, .685, .66, .65, .64};
+constexpr double kRoundNs = 6000., kFlushNsPerBin = 4.;
+constexpr std::uint64_t kCus = 256;
+constexpr std::uint64_t kMaxRounds = 16;  // chunk counts tried: up to so many workgroups a CU
+
+void shape_fast(ProjectionLaunch& L, bool coreas, bool zhs, std::uint64_t observers, std::uint64_t bins,
+                std::uint64_t count) {
+  auto const tile_bytes = [&](std::uint64_t tile) { return projection_lds_bytes(coreas, zhs, static_cast<std::uint32_t>(tile)); };
+  std::size_t const per_bin = (coreas ? 3u : 0u) + (zhs ? 3u : 0u);
+  std::size_t const most_lds = fast_dynamic_lds_limit(coreas, 1024);
+  std::uint64_t const capacity = (most_lds / sizeof(long long) - (zhs ? 3u : 0u)) / per_bin;
+  std::uint64_t const preferred = default_tile_capacity(per_bin, zhs);
+  std::uint64_t const last_tiles = (bins + preferred - 1) / preferred;
+  // every tile of an observer computes the track's update again, so the fewest
+  // that fit are tried too (windows of many tiles take the usual size)
+  std::uint64_t const first_tiles = last_tiles <= 8 ? (bins + capacity - 1) / capacity : last_tiles;
+  double best = std::numeric_limits<double>::infinity();
+  for (std::uint64_t tiles = first_tiles; tiles <= last_tiles; ++tiles) {
+    std::uint64_t const tile = (bins + tiles - 1) / tiles;
+    std::uint64_t const used = (bins + tile - 1) / tile;  // tiles that hold bins
+    for (std::uint32_t group = 1; group <= kMaxGroup && group <= observers; ++group) {
+      if (group * tile_bytes(tile) > most_lds) break;
+      std::uint64_t const per_chunk = (observers + group - 1) / group * used;
+      double const update = (coreas ? kCoreasNs * kCoreasShare[group - 1] : 0.) + (zhs ? kZhsNs * kZhsShare[group - 1] : 0.);
+      double const round = kRoundNs + kFlushNsPerBin * static_cast<double>(group * tile * ((coreas ? 1u : 0u) + (zhs ? 1u : 0u)));
+      for (std::uint64_t chunks = kXcdCount;; chunks += kXcdCount) {
+        std::uint64_t const chunk = (count + chunks - 1) / chunks;
+        std::uint64_t const rounds = (per_chunk * chunks + kCus - 1) / kCus;
+        if (chunk <= kMaxChunkTracks) {
+          double const time = static_cast<double>(rounds) * (static_cast<double>(chunk * group) * update + round);
+          if (time < best) {
+            best = time;
+            L.tile_bins = static_cast<std::uint32_t>(tile);
+            L.bin_tiles = static_cast<std::uint32_t>(used);
+            L.group = group;
+            // two workgroups of one tile each share a CU; a large tile or a group takes it alone
+            L.block_threads = group == 1 && 2 * (tile_bytes(tile) + fast_static_lds(coreas, 512)) <= kCuLdsBytes ? 512u : 1024u;
+            L.chunk_size = chunk;
+          }
+        }
+        if (chunk <= kMaxChunkTracks && (chunk <= 1024 || rounds >= kMaxRounds)) break;
+      }
+    }
+  }
+}
+
+}  // namespace
+
+void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std::uint32_t observers,
                       std::uint64_t max_bins, std::uint64_t count, LaunchTuning const& tuning) {
   // Window tile: the whole waveform when it fits the preferred LDS size, else
   // equal tiles of at most that size (a tuning limit may ask for others up to
   // the LDS budget).
-  std::size_t const words = kMaxDynamicLdsBytes / sizeof(long long);
-  std::size_t const per_bin = (coreas ? 3u : 0u) + (zhs ? 3u : 0u);
-  std::uint64_t capacity = default_tile_capacity(per_bin, zhs);
-  if (tuning.tile_bins_limit != 0)
-    capacity = std::min<std::uint64_t>((words - 3) / per_bin, tuning.tile_bins_limit);
-  std::uint64_t const want = std::max<std::uint64_t>(max_bins, 1);
-  std::uint64_t tile = std::min<std::uint64_t>(want, capacity);
-  if (tuning.tile_bins_limit == 0) {  // equal tiles: a 4096-bin window as two 2048-bin tiles
-    std::uint64_t const tiles = (want + capacity - 1) / capacity;
-    tile = (want + tiles - 1) / tiles;
+  L.block_threads = tuning.block_threads ? tuning.block_threads : 512;
+  L.group = 1;
+  if (fast && tuning.block_threads == 0 && tuning.chunk_tracks == 0 && tuning.tile_bins_limit == 0 && observers != 0 &&
+      max_bins != 0 && count != 0) {
+    shape_fast(L, coreas, zhs, observers, max_bins, count);
+  } else {
+    std::size_t const words = (fast ? std::min(kMaxDynamicLdsBytes, fast_dynamic_lds_limit(coreas, L.block_threads))
+                                    : kMaxDynamicLdsBytes) / sizeof(long long);
+    std::size_t const per_bin = (coreas ? 3u : 0u) + (zhs ? 3u : 0u);
+    std::uint64_t capacity = default_tile_capacity(per_bin, zhs);
+    if (tuning.tile_bins_limit != 0)
+      capacity = std::min<std::uint64_t>((words - 3) / per_bin, tuning.tile_bins_limit);
+    std::uint64_t const want = std::max<std::uint64_t>(max_bins, 1);
+    std::uint64_t tile = std::min<std::uint64_t>(want, capacity);
+    if (tuning.tile_bins_limit == 0) {  // equal tiles: a 4096-bin window as two 2048-bin tiles
+      std::uint64_t const tiles = (want + capacity - 1) / capacity;
+      tile = (want + tiles - 1) / tiles;
+    }
+    L.tile_bins = static_cast<std::uint32_t>(tile);
+    L.bin_tiles = static_cast<std::uint32_t>((max_bins + tile - 1) / tile);
+    if (L.bin_tiles == 0) L.bin_tiles = 1;
+    std::uint64_t chunk = tuning.chunk_tracks;
+    if (chunk == 0) {
+      std::uint64_t const per_chunk = std::max<std::uint64_t>(1, std::uint64_t(observers) * L.bin_tiles);
+      std::uint64_t const chunks_wanted = std::max<std::uint64_t>(1, tuning.target_workgroups / per_chunk);
+      // a workgroup clears and flushes a whole window tile, so chunks of tens
+      // of thousands of tracks pay (2^20 tracks on 160 antennas: 32768-track
+      // chunks 1.2x faster than 16384, as fast as 65536)
+      std::uint64_t chunks = std::min<std::uint64_t>(chunks_wanted, count / kMinimumDefaultChunk);
+      // chunk c runs on XCD c % 8: a multiple of eight chunks keeps the XCDs
+      // evenly loaded (50 chunks measured 12% slower than 48 or 64); a small
+      // batch (a lepton front's tracks) still gets eight chunks, so every XCD
+      // works on it (the EM + radio shower measured 10% faster than with
+      // chunks of at least 8192 tracks)
+      chunks = chunks >= kXcdCount ? chunks / kXcdCount * kXcdCount : kXcdCount;
+      chunk = (count + chunks - 1) / chunks;
+      std::uint64_t const block = L.block_threads;
+      chunk = std::max<std::uint64_t>(block, (chunk + block - 1) / block * block);
+    }
+    chunk = std::min(chunk, kMaxChunkTracks);
+    L.chunk_size = chunk;
   }
-  L.tile_bins = static_cast<std::uint32_t>(tile);
-  L.bin_tiles = static_cast<std::uint32_t>((max_bins + tile - 1) / tile);
-  if (L.bin_tiles == 0) L.bin_tiles = 1;
-  std::uint64_t chunk = tuning.chunk_tracks;
-  if (chunk == 0) {
-    std::uint64_t const per_chunk = std::max<std::uint64_t>(1, std::uint64_t(observers) * L.bin_tiles);
-    std::uint64_t const chunks_wanted = std::max<std::uint64_t>(1, tuning.target_workgroups / per_chunk);
-    // a workgroup clears and flushes a whole window tile, so chunks of tens
-    // of thousands of tracks pay (2^20 tracks on 160 antennas: 32768-track
-    // chunks 1.2x faster than 16384, as fast as 65536)
-    std::uint64_t chunks = std::min<std::uint64_t>(chunks_wanted, count / kMinimumDefaultChunk);
-    // chunk c runs on XCD c % 8: a multiple of eight chunks keeps the XCDs
-    // evenly loaded (50 chunks measured 12% slower than 48 or 64); a small
-    // batch (a lepton front's tracks) still gets eight chunks, so every XCD
-    // works on it (the EM + radio shower measured 10% faster than with
-    // chunks of at least 8192 tracks)
-    chunks = chunks >= kXcdCount ? chunks / kXcdCount * kXcdCount : kXcdCount;
-    chunk = (count + chunks - 1) / chunks;
-    std::uint64_t const block = tuning.block_threads;
-    chunk = std::max<std::uint64_t>(block, (chunk + block - 1) / block * block);
-  }
-  chunk = std::min(chunk, kMaxChunkTracks);
-  L.chunk_size = chunk;
-  std::uint64_t const chunks = (count + chunk - 1) / chunk;
+  std::uint64_t const chunks = (count + L.chunk_size - 1) / L.chunk_size;
   if (chunks > std::numeric_limits<std::uint32_t>::max())
     throw std::length_error("radio track batch too large for one launch");
   L.chunks = static_cast<std::uint32_t>(chunks);
-  std::uint64_t const grid = (chunks + 7) / 8 * 8 * std::uint64_t(observers) * L.bin_tiles;
+  std::uint64_t const groups = (std::uint64_t(observers) + L.group - 1) / L.group;
+  std::uint64_t const grid = (chunks + 7) / 8 * 8 * groups * L.bin_tiles;
   if (grid > std::numeric_limits<std::uint32_t>::max())
     throw std::length_error("radio projection grid too large");
 }

@@ -18,9 +18,11 @@ void validate_radio_config(c8mi_radio_config const& config);
 void validate_observers(c8mi_radio_observer const* observers, std::uint64_t count,
                         c8mi_radio_propagation const& p);
 // RadioAccumulator::makeObservers (RadioAccumulator.inl:591-617): device
-// observers with consecutive waveform offsets from 0.
+// observers with consecutive waveform offsets from 0. `p`: validated, with its
+// host tables.
 std::vector<ObserverDev> make_observers(c8mi_radio_observer const* input, std::uint64_t count, double limit,
-                                        bool zhs_potential, std::uint64_t& total_bins, std::uint64_t& max_bins);
+                                        bool zhs_potential, c8mi_radio_propagation const& p,
+                                        std::uint64_t& total_bins, std::uint64_t& max_bins);
 // observersCanShareTrackKinematics (RadioAccumulator.inl:619-632).
 bool can_fuse(std::vector<ObserverDev> const& a, std::vector<ObserverDev> const& b);
 // The propagation snapshot with device table pointers.

@@ -50,7 +50,13 @@ SlotRadio::SlotRadio(c8mi_radio_config const& config, std::uint32_t slots, std::
                          hipMemcpyHostToDevice));
     }
     propagation_ = propagation_view(p, refractivity_.data(), integrated_.data());
-    config_.propagation.refractivity = config_.propagation.integrated_refractivity = nullptr;
+    // observers set later take their own height's table entries from here
+    if (refractivity_.size()) {
+      refractivity_host_.assign(p.refractivity, p.refractivity + p.table_size);
+      integrated_host_.assign(p.integrated_refractivity, p.integrated_refractivity + p.table_size);
+    }
+    config_.propagation.refractivity = refractivity_host_.data();
+    config_.propagation.integrated_refractivity = integrated_host_.data();
     std::size_t const observers = static_cast<std::size_t>(slots) * observers_per_slot;
     coreas_observers_.allocate(observers);
     zhs_observers_.allocate(observers);
@@ -95,7 +101,7 @@ void SlotRadio::set_slot(std::uint32_t slot, c8mi_radio_observer const* observer
   std::uint64_t const first = static_cast<std::uint64_t>(slot) * observers_per_slot_;
   auto fill = [&](bool potential, DeviceBuffer<ObserverDev>& device) {
     std::uint64_t total = 0, max_bins = 0;
-    auto made = make_observers(observers, count, limit, potential, total, max_bins);
+    auto made = make_observers(observers, count, limit, potential, config_.propagation, total, max_bins);
     for (std::uint64_t k = 0; k < count; ++k) {
       made[k].waveform_offset = (first + k) * bins_per_observer_;
       staging_[k] = made[k];
@@ -206,6 +212,8 @@ void SlotRadio::project(double const* tracks, std::uint64_t stride, std::uint64_
   L.item_count = item_count;
   L.slot_observer_counts = observer_counts_.data();
   L.slot_observers = observers_per_slot_;
+  L.group = 1;
+  L.block_threads = kProjectionBlock;
   check_project(count, chunk, max_segments);
   std::uint64_t const grid = grid_for(count, chunk, max_segments);
   std::array<hipEvent_t, 2> events{nullptr, nullptr};
@@ -215,13 +223,12 @@ void SlotRadio::project(double const* tracks, std::uint64_t stride, std::uint64_
     C8MI_HIP(hipEventRecord(events[0], stream_));
   }
   bool const exact = config_.exact_fp64 != 0;
-  auto const block = kProjectionBlock;
   auto const g = static_cast<std::uint32_t>(grid);
   if (fuse_) {
-    launch_pooled_projection(L, true, true, exact, block, g, stream_);
+    launch_pooled_projection(L, true, true, exact, g, stream_);
   } else {
-    if (config_.coreas_enabled) launch_pooled_projection(L, true, false, exact, block, g, stream_);
-    if (config_.zhs_enabled) launch_pooled_projection(L, false, true, exact, block, g, stream_);
+    if (config_.coreas_enabled) launch_pooled_projection(L, true, false, exact, g, stream_);
+    if (config_.zhs_enabled) launch_pooled_projection(L, false, true, exact, g, stream_);
   }
   if (timing_) {
     C8MI_HIP(hipEventRecord(events[1], stream_));

@@ -85,6 +85,7 @@ class SlotRadio {
   PropagationDev propagation_{};
   DeviceBuffer<double> refractivity_;
   DeviceBuffer<double> integrated_;
+  std::vector<double> refractivity_host_, integrated_host_;
   DeviceBuffer<ObserverDev> coreas_observers_;
   DeviceBuffer<ObserverDev> zhs_observers_;
   DeviceBuffer<std::uint32_t> observer_counts_;
