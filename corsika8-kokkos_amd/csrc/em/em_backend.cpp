@@ -869,7 +869,7 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
     launch_lepton_move(context_.data(), config_.profile_bins, f, stream_);
     mark(kKernLeptonTransport);
     bool const table = host_context_.moliere_polynomials != nullptr;
-    launch_lepton_moliere(context_.data(), table, f, stream_);
+    launch_lepton_moliere(context_.data(), table, host_context_.moliere.component_count, f, stream_);
     mark(kKernLeptonTransport);
     // the few open samples continue on the side stream while the other
     // sources finish and run their vertices here

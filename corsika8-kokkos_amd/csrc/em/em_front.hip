@@ -259,17 +259,34 @@ __global__ __launch_bounds__(kStepBlock, 3) void lepton_move_kernel(EmContext co
 // Molière scattering of the moved sources: the move record's end direction is
 // deflected in place; a failed sampling marks the source (kMovedMoliereFailed)
 // for the finish kernel; a sample not converged after the first Newton
-// iterations is listed for the tail kernel. A kernel of its own: the sampler's
+// iterations, or about to evaluate the large-x forms, is listed for the tail
+// kernel. One angle in two hundred gets there, so one wave in four held such a
+// lane and waited for its thousands of instructions per component and iteration
+// (pow and log per term) while most SIMDs were empty. A kernel of its own: the sampler's
 // registers do not weigh on the rest of the step. The context is read from
 // global memory (its snapshot and table pointers are uniform, scalar loads).
-template <bool Table>
+// One form per component count (N): a state of exactly the medium's components
+// stays in registers and runs no chain for an absent one, and the table's cubics
+// (four functions a component and iteration, a line of the L1 per lane each) are
+// read from LDS.
+template <bool Table, int N>
 __global__ __launch_bounds__(kStepBlock) void lepton_moliere_kernel(EmContext const* __restrict__ context,
-                                                                    FrontArgs f) {
+                                                                       FrontArgs f) {
+  __shared__ double rows[Table ? moliere::kIntervals * moliere::LdsTable::kRow : 1];
+  if constexpr (Table) {
+    for (int k = static_cast<int>(threadIdx.x); k < 16 * moliere::kIntervals; k += kStepBlock) {
+      int const cubic = k / 4, c = k % 4;  // cubic = function * kIntervals + interval
+      rows[(cubic % moliere::kIntervals) * moliere::LdsTable::kRow + 4 * (cubic / moliere::kIntervals) + c] =
+          context->moliere_polynomials[cubic].c[c];
+    }
+    __syncthreads();
+  }
   std::uint64_t const i = static_cast<std::uint64_t>(blockIdx.x) * kStepBlock + threadIdx.x;
   if (i >= f.count || f.moved[i] != kMovedOk) return;
   auto* mv = static_cast<phys::LeptonMove*>(f.moves) + i;
   phys::MoliereOpen open;
-  int const outcome = phys::moliere_scatter<Table>(*context, *mv, open);
+  moliere::LdsTable const table{rows, context->moliere_guess};
+  int const outcome = phys::moliere_scatter<Table, N>(*context, table, moliere::open_above<Table>(), *mv, open);
   if (outcome == phys::kMoliereFailed) {
     f.moved[i] = kMovedMoliereFailed;
   } else if (outcome == phys::kMoliereOpen) {
@@ -769,21 +786,33 @@ void launch_lepton_move(EmContext const* context, std::uint32_t bins, FrontArgs 
   C8MI_HIP(hipGetLastError());
 }
 
-void launch_lepton_moliere(EmContext const* context, bool table, FrontArgs const& f, hipStream_t stream) {
-  if (f.count == 0) return;
-  if (table)
-    lepton_moliere_kernel<true><<<grid_for(f.count, kStepBlock), kStepBlock, 0, stream>>>(context, f);
-  else
-    lepton_moliere_kernel<false><<<grid_for(f.count, kStepBlock), kStepBlock, 0, stream>>>(context, f);
+namespace {
+template <bool Table>
+void launch_moliere(EmContext const* context, std::uint32_t components, FrontArgs const& f, hipStream_t stream) {
+  unsigned const grid = grid_for(f.count, kStepBlock);
+  switch (components) {
+    case 1: lepton_moliere_kernel<Table, 1><<<grid, kStepBlock, 0, stream>>>(context, f); break;
+    case 2: lepton_moliere_kernel<Table, 2><<<grid, kStepBlock, 0, stream>>>(context, f); break;
+    case 3: lepton_moliere_kernel<Table, 3><<<grid, kStepBlock, 0, stream>>>(context, f); break;
+    default:
+      static_assert(moliere::kDeviceComponents == 4, "one form per component count");
+      lepton_moliere_kernel<Table, 4><<<grid, kStepBlock, 0, stream>>>(context, f);
+  }
   C8MI_HIP(hipGetLastError());
+}
+}  // namespace
+
+void launch_lepton_moliere(EmContext const* context, bool table, std::uint32_t components, FrontArgs const& f,
+                           hipStream_t stream) {
+  if (f.count == 0) return;
+  if (table) launch_moliere<true>(context, components, f, stream);
+  else launch_moliere<false>(context, components, f, stream);
 }
 
 void launch_lepton_open(EmContext const* context, std::uint32_t bins, bool table, FrontArgs const& f,
                         hipStream_t stream) {
   if (f.count == 0) return;
-  // the open samples are rare (~1e-5 of the steps): fixed grids of small
-  // workgroups that leave at once when there are none
-  constexpr unsigned kTailGrid = 256, kOpenGrid = 4;
+  constexpr unsigned kTailGrid = 1024, kOpenGrid = 16;
   if (table)
     lepton_moliere_tail_kernel<true><<<kTailGrid, moliere::kTailThreads, 0, stream>>>(context, f);
   else
@@ -792,7 +821,7 @@ void launch_lepton_open(EmContext const* context, std::uint32_t bins, bool table
   FrontArgs g = f;
   g.vertices = f.open_vertices;
   g.vertex_count = f.open_vertex_count;
-  lepton_vertex_kernel<<<1, kStepBlock, step_lds_bytes(bins), stream>>>(context, g);
+  lepton_vertex_kernel<<<4, kStepBlock, step_lds_bytes(bins), stream>>>(context, g);
   C8MI_HIP(hipGetLastError());
 }
 

@@ -128,8 +128,10 @@ void launch_radio_segments(FrontArgs const& f, std::uint32_t slots, unsigned lon
 
 // Molière scattering of the moved sources between the move and finish kernels
 // (the step kernel, then the tail kernel for samples still open);
-// table: the interpolation-view sampler (else the analytical functions).
-void launch_lepton_moliere(EmContext const* context, bool table, FrontArgs const& f, hipStream_t stream);
+// table: the interpolation-view sampler (else the analytical functions);
+// components: those of the Molière snapshot.
+void launch_lepton_moliere(EmContext const* context, bool table, std::uint32_t components, FrontArgs const& f,
+                           hipStream_t stream);
 // The open Molière samples on a stream of their own, overlapping the finish
 // and vertex kernels of the other sources: tail kernel, their finish, their
 // vertices (FrontArgs::open_vertices).

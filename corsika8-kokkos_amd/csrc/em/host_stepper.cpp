@@ -141,8 +141,10 @@ HostStep HostStepper::step(c8mi_particle_state const& particle, std::uint64_t fi
       bool failed = false;
       if (c.moliere_enabled && moliere) {
         phys::MoliereOpen open;
-        int const outcome = c.moliere_polynomials ? phys::moliere_scatter<true>(c, mv, open)
-                                                  : phys::moliere_scatter<false>(c, mv, open);
+        moliere::Table const table{c.moliere_polynomials, c.moliere_guess};
+        constexpr int n = moliere::kDeviceComponents;
+        int const outcome = c.moliere_polynomials ? phys::moliere_scatter<true, n>(c, table, __builtin_huge_val(), mv, open)
+                                                  : phys::moliere_scatter<false, n>(c, table, __builtin_huge_val(), mv, open);
         if (outcome == phys::kMoliereOpen) throw std::logic_error("em: host Moliere sample left open");
         failed = outcome == phys::kMoliereFailed;
       }

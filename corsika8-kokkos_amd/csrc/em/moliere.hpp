@@ -23,6 +23,12 @@
 
 namespace c8mi::em::moliere {
 
+// Math inline here: the Newton iterations call exp and erf per component, and a
+// call there cost the sampler 40% (263 -> 376 us a launch of 2.5e5 steps).
+using ::exp;
+using ::log;
+using ::pow;
+
 enum Status : int { kSuccess = 0, kNoDeflection = 1, kInvalidSnapshot = 2, kInvalidInput = 3,
                     kNonConvergent = 4, kNonFinite = 5 };
 
@@ -95,10 +101,29 @@ struct Quotients {
 struct Table {
   c8mi_moliere_cubic const* polynomials;
   double const* guess;
+  C8MI_HD double cubic(int f, std::uint32_t interval, double u) const;
 };
 
 inline constexpr double kTableUpper = 20.;
 inline constexpr int kIntervals = C8MI_MOLIERE_INTERVALS;
+
+C8MI_HD double Table::cubic(int f, std::uint32_t interval, double u) const {
+  double const* c = polynomials[f * kIntervals + interval].c;
+  return c[0] + u * (c[1] + u * (c[2] + u * c[3]));
+}
+
+// The view with its cubics in LDS, the four functions of an interval together:
+// 16 coefficients in a row of 18 words (rows of 16 would all start in the same
+// two banks).
+struct LdsTable {
+  static constexpr int kRow = 18;
+  double const* rows;
+  double const* guess;
+  C8MI_HD double cubic(int f, std::uint32_t interval, double u) const {
+    double const* c = rows + interval * kRow + 4 * f;
+    return c[0] + u * (c[1] + u * (c[2] + u * c[3]));
+  }
+};
 
 // The snapshot was validated when the backend was created.
 template <int Cap>
@@ -234,13 +259,13 @@ C8MI_HD void evaluate(c8mi_moliere_snapshot const& m, Quotients const& q, State<
 // evaluate_distribution with an interpolation view: the cubic of x's interval
 // for x <= 20 (the four functions share the interval), the large-x branches
 // above (x > 20 is past both branch points of the series).
-template <int N>
-C8MI_HD void evaluate_table(c8mi_moliere_snapshot const& m, Quotients const& q, Table const& t,
+template <class Tbl, int N>
+C8MI_HD void evaluate_table(c8mi_moliere_snapshot const& m, Quotients const& q, Tbl const& t,
                             State<N> const& st, double theta, double& density,
                             double& cumulative) {
   double const t2 = theta * theta;
   double dens = 0., cdf = 0.;
-#pragma unroll 1
+#pragma unroll
   for (int k = 0; k < N; ++k) {
     if (k >= static_cast<int>(m.component_count)) break;
     double const x = t2 * st.inverse_scale[k], ib = st.inverse_b[k], ib2 = ib * ib;
@@ -253,14 +278,10 @@ C8MI_HD void evaluate_table(c8mi_moliere_snapshot const& m, Quotients const& q, 
       auto interval = static_cast<std::uint32_t>(coordinate);
       if (interval >= static_cast<std::uint32_t>(kIntervals)) interval = kIntervals - 1;
       double const u = coordinate - static_cast<double>(interval);
-      auto cubic = [&](int f) {
-        double const* c = t.polynomials[f * kIntervals + interval].c;
-        return c[0] + u * (c[1] + u * (c[2] + u * c[3]));
-      };
-      f1v = cubic(0);
-      f2v = cubic(1);
-      i1v = cubic(2);
-      i2v = cubic(3);
+      f1v = t.cubic(0, interval, u);
+      f2v = t.cubic(1, interval, u);
+      i1v = t.cubic(2, interval, u);
+      i2v = t.cubic(3, interval, u);
     } else {
       f1v = f1_large(x);
       i1v = integral_f1_large(m, x);
@@ -312,15 +333,19 @@ C8MI_HD double improve_guess(double const* g, double reference_b, double beta2, 
 // Start of sample_one_dimensional: the invalid-input and median cases, else the
 // Newton start (the Gaussian quantile, corrected by the tabulated guess).
 inline constexpr int kStarted = -1;  // Newton iteration to follow
-template <bool Tab, int Cap>
-C8MI_HD int newton_start(c8mi_moliere_snapshot const& m, Table const& t, State<Cap> const& st,
+template <bool Tab, class Tbl, int Cap>
+C8MI_HD int newton_start(c8mi_moliere_snapshot const& m, Tbl const& t, State<Cap> const& st,
                          double u, double& current) {
   current = 0.;
   if (!isfinite(u) || !(u > 0.) || !(u < 1.)) return kInvalidInput;
   if (u == 0.5) return kSuccess;
   double const gaussian = normal_ppf(u) / kSqrt2;
   if constexpr (Tab) {
-    double const reference_b = 1. / st.inverse_b[m.maximum_weight_index];
+    double ib = st.inverse_b[0];  // without a dynamic index into registers
+#pragma unroll
+    for (int k = 1; k < Cap; ++k)
+      if (k == static_cast<int>(m.maximum_weight_index)) ib = st.inverse_b[k];
+    double const reference_b = 1. / ib;
     current = st.prefactor * improve_guess(t.guess, reference_b, st.beta_squared, gaussian);
   } else {
     current = st.prefactor * gaussian;
@@ -342,38 +367,51 @@ C8MI_HD int newton_update(double density, double cdf, double target, double& cur
 inline constexpr int kMaximumIterations = 100;
 inline constexpr int kPending = -2;  // not converged within the iterations allowed here
 
+// x above which the step kernel leaves an evaluation to the tail kernel: where the
+// large-x forms of f1 and its integral begin. Measured against never (and 42.25,
+// where those of f2 begin): a 100 GeV shower 113 -> 102.5 ms (105), 1 TeV with
+// the analytical functions 354 -> 296 (308; 301 at 20), a pool of 1000 showers
+// 437 -> 413 (410), 21 requests with radio 766 -> 654 (670), ice 754 -> 691 (691).
+template <bool Tab>
+C8MI_HD constexpr double open_above() {
+  return Tab ? kTableUpper : 12.;
+}
+
 // Newton iterations `first` .. `last` (1-based, at most 100) from `current`:
-// kSuccess, kNonFinite, kNonConvergent after iteration 100, or kPending after
-// `last` < 100.
-template <bool Tab, int Cap>
-C8MI_HD int newton_iterate(c8mi_moliere_snapshot const& m, Quotients const& q, Table const& t,
-                           State<Cap> const& st, double u, int first, int last,
-                           double& current) {
+// kSuccess, kNonFinite, kNonConvergent after iteration 100, or kPending: after
+// `last` < 100, or before an evaluation above `open_above` in any component's x.
+// `done`: the last iteration made.
+template <bool Tab, class Tbl, int Cap>
+C8MI_HD int newton_iterate(c8mi_moliere_snapshot const& m, Quotients const& q, Tbl const& t,
+                           State<Cap> const& st, double u, int first, int last, double open_above,
+                           double& current, int& done) {
   double const target = u - 0.5;
   for (int it = first; it <= last; ++it) {
+    double largest = 0.;
+#pragma unroll
+    for (int k = 0; k < Cap; ++k) {
+      double const x = current * current * st.inverse_scale[k];
+      largest = x > largest ? x : largest;
+    }
+    done = it - 1;
+    if (largest > open_above) return kPending;
     double density, cdf;
     if constexpr (Tab) evaluate_table(m, q, t, st, current, density, cdf);
     else evaluate(m, q, st, current, density, cdf);
     int const status = newton_update(density, cdf, target, current);
     if (status != kStarted) return status;
   }
+  done = last;
   return last >= kMaximumIterations ? kNonConvergent : kPending;
 }
 
-template <bool Tab, int Cap>
-C8MI_HD int one_dimensional(c8mi_moliere_snapshot const& m, Quotients const& q, Table const& t,
-                            State<Cap> const& st, double u, double& angle) {
-  int const status = newton_start<Tab>(m, t, st, u, angle);
-  if (status != kStarted) return status;
-  return newton_iterate<Tab>(m, q, t, st, u, 1, kMaximumIterations, angle);
-}
-
-// ---- the slow tail: one wavefront per sample that did not converge early ----
+// ---- the slow tail: one workgroup per sample that left the step kernel ----
 //
-// About one e+- step in 1e5 draws a far-tail quantile whose Newton iteration
-// runs to its limit of 100 through the large-x expansions (two dozen pow per
-// component and iteration). Serially that is ~1 ms of one lane, and the whole
-// launch waits for it. The step kernels therefore stop after a few iterations
+// About one e+- step in a hundred draws a quantile whose iterates reach the
+// large-x expansions (two dozen pow per component and iteration), one in 1e5 one
+// whose iteration runs through them to its limit of 100: serially ~1 ms of one
+// lane, and the whole launch waits for it. The step kernels therefore stop before
+// such an evaluation (open_above) or after a few iterations
 // (EmContext::moliere_fast_iterations); a sample still open continues here
 // with its iterate: each evaluation spreads the transcendental parts of every
 // component over a workgroup of kTailThreads (LDS `jobs`), then every thread
@@ -511,23 +549,6 @@ __device__ __forceinline__ int newton_iterate_wave(c8mi_moliere_snapshot const& 
     if (status != kStarted) return status;
   }
   return kNonConvergent;
-}
-
-// Space angle of two projected draws (sample_moliere_scattering_angle_2d).
-template <bool Tab, int Cap>
-C8MI_HD int angle_2d_for(c8mi_moliere_snapshot const& m, Quotients const& q, Table const& t,
-                         double grammage, double e_mev, double u1, double u2, double& angle) {
-  State<Cap> st;
-  angle = 0.;
-  int status = build(m, grammage, e_mev, st);
-  if (status != kSuccess) return status;
-  double a1, a2;
-  status = one_dimensional<Tab>(m, q, t, st, u1, a1);
-  if (status != kSuccess) return status;
-  status = one_dimensional<Tab>(m, q, t, st, u2, a2);
-  if (status != kSuccess) return status;
-  angle = sqrt(a1 * a1 + a2 * a2);
-  return isfinite(angle) ? kSuccess : kNonFinite;
 }
 
 // Media of up to kDeviceComponents components (air has three; the backend

@@ -568,14 +568,16 @@ C8MI_HD int moliere_apply(LeptonMove& mv, double a1, double a2, double ua) {
 
 // Up to the context's moliere_fast_iterations Newton iterations per sample; a
 // sample still open is described in `open` (kMoliereOpen) for
-// moliere_scatter_wave.
-template <bool Table>
-C8MI_HD int moliere_scatter(EmContext const& c, LeptonMove& mv, MoliereOpen& open) {
+// moliere_scatter_wave. N: at least the snapshot's components (a kernel for just
+// as many keeps the state in registers and evaluates no unused chain); Tbl: where
+// the interpolation view's cubics are read from.
+template <bool Table, int N, class Tbl>
+C8MI_HD int moliere_scatter(EmContext const& c, Tbl const& t, double open_above, LeptonMove& mv,
+                            MoliereOpen& open) {
   if (mv.particle_cut) return kMoliereDone;
   MoliereDraws const d = moliere_draws(c, mv.start);
   moliere::Quotients const q{c.moliere_i1, c.moliere_i2, c.moliere_i2_large, c.moliere_half_over};
-  moliere::Table const t{c.moliere_polynomials, c.moliere_guess};
-  moliere::State<moliere::kDeviceComponents> st;
+  moliere::State<N> st;
   int status = moliere::build(c.moliere, mv.step_grammage, mv.start.energy_gev * 1000., st);
   if (status == moliere::kNoDeflection) return kMoliereDone;
   if (status != moliere::kSuccess) return kMoliereFailed;
@@ -583,11 +585,12 @@ C8MI_HD int moliere_scatter(EmContext const& c, LeptonMove& mv, MoliereOpen& ope
   double const u[2] = {d.u1, d.u2};
   for (int k = 0; k < 2; ++k) {
     status = moliere::newton_start<Table>(c.moliere, t, st, u[k], a[k]);
-    int const fast = static_cast<int>(c.moliere_fast_iterations);
+    int done = 0;
     if (status == moliere::kStarted)
-      status = moliere::newton_iterate<Table>(c.moliere, q, t, st, u[k], 1, fast, a[k]);
+      status = moliere::newton_iterate<Table>(c.moliere, q, t, st, u[k], 1, static_cast<int>(c.moliere_fast_iterations),
+                                              open_above, a[k], done);
     if (status == moliere::kPending) {
-      open = {0u, static_cast<std::uint32_t>(k + 1), fast, 0u, a[k], k ? a[0] : 0.};
+      open = {0u, static_cast<std::uint32_t>(k + 1), done, 0u, a[k], k ? a[0] : 0.};
       return kMoliereOpen;
     }
     if (status != moliere::kSuccess) return kMoliereFailed;
