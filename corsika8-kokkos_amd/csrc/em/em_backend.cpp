@@ -205,7 +205,7 @@ EmBackend::EmBackend(c8mi_em_config const& config, c8mi_native_table_set const& 
   stats_.allocate(slots_ * static_cast<std::uint64_t>(kSlotStats));
   shower_totals_.allocate(static_cast<std::size_t>(kMaxShowerSlots) * kMaxRuns * kShowerFields);
   adjust_.allocate(slots_ * static_cast<std::uint64_t>(kMaxRuns) * 3u);
-  report_.allocate(kReportHeader + kReportPerSlot * static_cast<std::size_t>(slots_));
+  report_.allocate(kReportHeader);
   host_report_ = PinnedBuffer<unsigned long long>(kReportHeader + kReportPerSlot * static_cast<std::size_t>(slots_));
   control_dev_.allocate(slots_);
   control_host_ = PinnedBuffer<SlotControl>(slots_);
@@ -785,6 +785,7 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
   f.history = history_.data();
   f.stats = stats_.data();
   f.report = report_.data();
+  f.host_report = host_report_.data();
   f.vertices = vertices_.data();
   f.vertex_count = vertex_count_.data();
   f.moves = moves_.data();
@@ -871,17 +872,22 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
     bool const table = host_context_.moliere_polynomials != nullptr;
     launch_lepton_moliere(context_.data(), table, host_context_.moliere.component_count, f, stream_);
     mark(kKernLeptonTransport);
-    // the few open samples continue on the side stream while the other
-    // sources finish and run their vertices here
-    C8MI_HIP(hipEventRecord(open_ready_, stream_));
-    C8MI_HIP(hipStreamWaitEvent(side_stream_, open_ready_, 0));
-    launch_lepton_open(context_.data(), config_.profile_bins, table, f, side_stream_);
-    C8MI_HIP(hipEventRecord(open_done_, side_stream_));
+    bool const in_line = m <= kInlineTailSources;
+    if (in_line) {
+      launch_lepton_tail(context_.data(), table, f, stream_);
+    } else {
+      // the open samples continue on the side stream while the other sources
+      // finish and run their vertices here
+      C8MI_HIP(hipEventRecord(open_ready_, stream_));
+      C8MI_HIP(hipStreamWaitEvent(side_stream_, open_ready_, 0));
+      launch_lepton_open(context_.data(), config_.profile_bins, table, f, side_stream_);
+      C8MI_HIP(hipEventRecord(open_done_, side_stream_));
+    }
     launch_lepton_finish(context_.data(), config_.profile_bins, f, stream_);
     mark(kKernLeptonTransport);
     launch_lepton_vertex(context_.data(), config_.profile_bins, f, stream_);
     mark(kKernLeptonVertex);
-    C8MI_HIP(hipStreamWaitEvent(stream_, open_done_, 0));
+    if (!in_line) C8MI_HIP(hipStreamWaitEvent(stream_, open_done_, 0));
     mark(kKernLeptonTransport);  // what the open samples add beyond the overlap
     project_tracks();
   } else {
@@ -891,19 +897,20 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
     launch_lepton_vertex(context_.data(), config_.profile_bins, f, stream_);
     mark(kKernLeptonVertex);
   }
-  launch_count(f, stream_);
-  mark(kKernCount);
-  launch_scan(photon, f, stream_);
-  mark(kKernScan);
-  launch_scatter(f, next, other, count_[o], stream_);
-  mark(kKernScatter);
+  if (m <= kCompactSources) {
+    launch_compact(photon, f, next, other, count_[o], stream_);
+    mark(kKernScatter);
+  } else {
+    launch_count(f, stream_);
+    mark(kKernCount);
+    launch_scan(photon, f, stream_);
+    mark(kKernScan);
+    launch_scatter(f, next, other, count_[o], stream_);
+    mark(kKernScatter);
+  }
   // showers that sat this front out follow the continuing particles unchanged
   if (parked) launch_carry(front_in, m, n, next, report_.data(), stream_);
-  C8MI_HIP(hipMemcpyAsync(host_report_.data(), report_.data(),
-                          (kReportHeader + kReportPerSlot * static_cast<std::size_t>(active_range_)) *
-                              sizeof(unsigned long long),
-                          hipMemcpyDeviceToHost, stream_));
-  C8MI_HIP(hipStreamSynchronize(stream_));
+  C8MI_HIP(hipStreamSynchronize(stream_));  // the front's last kernels have written the pinned report
   FrontTotals t;
   std::memcpy(&t, host_report_.data(), sizeof t);
   totals_.device_to_host_bytes += (kReportHeader + kReportPerSlot * active_range_) * sizeof(unsigned long long);

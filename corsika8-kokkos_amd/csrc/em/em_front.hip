@@ -300,7 +300,7 @@ __global__ __launch_bounds__(kStepBlock) void lepton_moliere_kernel(EmContext co
 // The open samples, one workgroup each (grid-stride over the list).
 template <bool Table>
 __global__ __launch_bounds__(moliere::kTailThreads) void lepton_moliere_tail_kernel(
-    EmContext const* __restrict__ context, FrontArgs f) {
+    EmContext const* __restrict__ context, FrontArgs f, int in_line) {
   __shared__ double jobs[moliere::kDeviceComponents * moliere::kJobSlots];
   unsigned long long const n = *f.moliere_open_count;
   for (unsigned long long w = blockIdx.x; w < n; w += gridDim.x) {
@@ -310,14 +310,15 @@ __global__ __launch_bounds__(moliere::kTailThreads) void lepton_moliere_tail_ker
     if (threadIdx.x == 0) {
       // the outcome goes with the open record: the source stays kMovedOpen for
       // the finish kernel of the other sources, which may run meanwhile
+      // (in line, the finish kernel comes after and takes it as any other)
       auto* record = static_cast<phys::MoliereOpen*>(f.moliere_open) + w;
-      if (outcome == phys::kMoliereFailed) {
-        record->pad = kMovedMoliereFailed;
-      } else {
+      std::uint32_t const moved = outcome == phys::kMoliereFailed ? kMovedMoliereFailed : kMovedOk;
+      if (moved == kMovedOk) {
         auto* out = static_cast<phys::LeptonMove*>(f.moves) + open.source;
         for (int a = 0; a < 3; ++a) out->end.direction[a] = mv.end.direction[a];
-        record->pad = kMovedOk;
       }
+      if (in_line) f.moved[open.source] = moved;
+      else record->pad = moved;
     }
   }
 }
@@ -548,8 +549,17 @@ __global__ __launch_bounds__(kScanBlock) void scan_kernel(FrontArgs f, std::uint
     out.children = carry[2];
     out.steps = carry[3];
     out.interactions = carry[4];
-    *reinterpret_cast<FrontTotals*>(f.report) = out;
+    *reinterpret_cast<FrontTotals*>(f.report) = out;  // the carry kernel reads the new count
+    *reinterpret_cast<FrontTotals*>(f.host_report) = out;
   }
+}
+
+__device__ __forceinline__ void report_slot(FrontArgs const& f, std::uint32_t s, unsigned long long next,
+                                            unsigned long long other, unsigned long long children) {
+  unsigned long long* r = f.host_report + kReportHeader + kReportPerSlot * static_cast<std::uint64_t>(s);
+  r[0] = next;
+  r[1] = other;
+  r[2] = children;
 }
 
 // Per slot (a front is one run sorted by slot, so a global output rank is
@@ -582,9 +592,34 @@ __global__ __launch_bounds__(kStepBlock) void slot_update_kernel(FrontArgs f, in
   st[photon ? 0 : 1] += steps;
   st[photon ? 2 : 3] += interactions;
   st[4] += children;
-  f.report[kReportHeader + kReportPerSlot * static_cast<std::uint64_t>(s)] = next;
-  f.report[kReportHeader + kReportPerSlot * static_cast<std::uint64_t>(s) + 1] = other;
-  f.report[kReportHeader + kReportPerSlot * static_cast<std::uint64_t>(s) + 2] = children;
+  report_slot(f, s, next, other, children);
+}
+
+// The outputs of source `i` (its packed word) to their places; children take
+// the history IDs from `child_base` on.
+__device__ __forceinline__ void scatter_source(FrontArgs const& f, std::uint64_t i, std::uint32_t word,
+                                               ParticleQueue const& next_queue, std::uint64_t next_pos,
+                                               ParticleQueue const& other_queue, std::uint64_t other_pos,
+                                               std::uint64_t child_base) {
+  std::uint32_t const s = word >> kPackedSlotShift;
+  for (int k = 0; k < 2; ++k) {
+    std::uint32_t const kind = (word >> (6 + 2 * k)) & 3u;
+    if (kind == kSlotNone) continue;
+    c8mi_particle_state p = f.staging[2 * i + k];
+    if (kind != kSlotNextContinue) {
+      p.history_id = child_base + p.history_id;
+      // children of generation-zero parents only (a handful per shower)
+      if (p.generation == 1 && f.first_interactions)
+        phys::patch_first_interaction(f.first_interactions[s], f.first_candidates[s], p);
+    }
+    if (kind == kSlotOtherChild) {
+      store_particle(other_queue, other_pos, p);
+      other_queue.shower[other_pos++] = s | (kClassPending << kClassShift);
+    } else {
+      store_particle(next_queue, next_pos, p);
+      next_queue.shower[next_pos++] = s;
+    }
+  }
 }
 
 __global__ __launch_bounds__(kStepBlock) void scatter_kernel(FrontArgs f, ParticleQueue next_queue,
@@ -610,26 +645,80 @@ __global__ __launch_bounds__(kStepBlock) void scatter_kernel(FrontArgs f, Partic
     for (std::uint32_t w = 0; w < wave; ++w) before += wave_sums[w][k];
     pos[k] = f.offsets[3 * static_cast<std::uint64_t>(blockIdx.x) + k] + before + inc[k] - v[k] + adj[k];
   }
-  std::uint64_t next_pos = pos[0], other_pos = other_base + pos[1];
-  std::uint64_t const child_base = pos[2];
-  for (int k = 0; k < 2; ++k) {
-    std::uint32_t const kind = (word >> (6 + 2 * k)) & 3u;
-    if (kind == kSlotNone) continue;
-    c8mi_particle_state p = f.staging[2 * i + k];
-    if (kind != kSlotNextContinue) {
-      p.history_id = child_base + p.history_id;
-      // children of generation-zero parents only (a handful per shower)
-      if (p.generation == 1 && f.first_interactions)
-        phys::patch_first_interaction(f.first_interactions[s], f.first_candidates[s], p);
-    }
-    if (kind == kSlotOtherChild) {
-      store_particle(other_queue, other_pos, p);
-      other_queue.shower[other_pos++] = s | (kClassPending << kClassShift);
-    } else {
-      store_particle(next_queue, next_pos, p);
-      next_queue.shower[next_pos++] = s;
-    }
+  scatter_source(f, i, word, next_queue, pos[0], other_queue, other_base + pos[1], pos[2]);
+}
+
+// The four kernels above for a front of at most kCompactSources sources, in one
+// workgroup: a small front's time is its chain of launches (about 4 us each for a
+// few words of work), so the scan, the showers' history offsets and counts, the
+// scatter and the report are one. The prefix of a shower's first source, found
+// by a maximum scan over the segment starts, turns block ranks into its own.
+__global__ __launch_bounds__(kScanBlock) void compact_kernel(FrontArgs f, int photon, ParticleQueue next_queue,
+                                                             ParticleQueue other_queue, std::uint64_t other_base) {
+  __shared__ std::uint32_t wave_sums[kScanBlock / 64][kShowerFields];
+  __shared__ std::uint32_t wave_starts[kScanBlock / 64];
+  __shared__ std::uint32_t before_source[kShowerFields][kScanBlock];
+  __shared__ std::uint32_t slot_of[kScanBlock];
+  std::uint32_t const i = threadIdx.x, count = static_cast<std::uint32_t>(f.count);
+  std::uint32_t const wave = i / 64, lane = i % 64;
+  bool const active = i < count;
+  std::uint32_t const word = active ? f.packed[i] : 0u;
+  std::uint32_t const s = word >> kPackedSlotShift;
+  unsigned long long const history = active ? f.history[s] : 0ULL;  // before the shower's last source advances it
+  std::uint32_t const v[kShowerFields] = {word & 3u, (word >> 2) & 3u, (word >> 4) & 3u, (word >> 10) & 1u,
+                                          (word >> 11) & 1u};
+  slot_of[i] = active ? s : kNoKey;
+  std::uint32_t inc[kShowerFields];
+#pragma unroll
+  for (int k = 0; k < kShowerFields; ++k) inc[k] = wave_inclusive(v[k], lane);
+  if (lane == 63)
+    for (int k = 0; k < kShowerFields; ++k) wave_sums[wave][k] = inc[k];
+  __syncthreads();
+  std::uint32_t excl[kShowerFields];
+#pragma unroll
+  for (int k = 0; k < kShowerFields; ++k) {
+    std::uint32_t before = 0;
+    for (std::uint32_t w = 0; w < wave; ++w) before += wave_sums[w][k];
+    inc[k] += before;
+    excl[k] = inc[k] - v[k];
+    before_source[k][i] = excl[k];
   }
+  // the shower's first source: the last segment start at or before this one
+  std::uint32_t start = i == 0 || slot_of[i - 1] != slot_of[i] ? i : 0u;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    std::uint32_t const y = __shfl_up(start, d, 64);
+    if (static_cast<int>(lane) >= d) start = y > start ? y : start;
+  }
+  if (lane == 63) wave_starts[wave] = start;
+  __syncthreads();
+  for (std::uint32_t w = 0; w < wave; ++w) start = wave_starts[w] > start ? wave_starts[w] : start;
+  if (i == kScanBlock - 1) {  // absent sources add nothing: its inclusive sums are the front's totals
+    FrontTotals out{};
+    out.next = inc[0];
+    out.other = inc[1];
+    out.children = inc[2];
+    out.steps = inc[3];
+    out.interactions = inc[4];
+    *reinterpret_cast<FrontTotals*>(f.report) = out;  // the carry kernel reads the new count
+    *reinterpret_cast<FrontTotals*>(f.host_report) = out;
+    *f.vertex_count = 0;  // the vertex kernels of this front have finished
+    if (f.open_vertex_count) *f.open_vertex_count = 0;
+  }
+  if (!active) return;
+  if (i + 1 == count || slot_of[i + 1] != s) {  // the shower's last source
+    std::uint32_t t[kShowerFields];
+#pragma unroll
+    for (int k = 0; k < kShowerFields; ++k) t[k] = inc[k] - before_source[k][start];
+    f.history[s] = history + t[2];
+    unsigned long long* st = f.stats + static_cast<std::uint64_t>(s) * kSlotStats;
+    st[photon ? 0 : 1] += t[3];
+    st[photon ? 2 : 3] += t[4];
+    st[4] += t[2];
+    report_slot(f, s, t[0], t[1], t[2]);
+  }
+  scatter_source(f, i, word, next_queue, excl[0], other_queue, other_base + excl[1],
+                 history + excl[2] - before_source[2][start]);
 }
 
 // Per-shower radio: the (slot, run) segments of a lepton front's sources. A
@@ -809,14 +898,22 @@ void launch_lepton_moliere(EmContext const* context, bool table, std::uint32_t c
   else launch_moliere<false>(context, components, f, stream);
 }
 
+void launch_lepton_tail(EmContext const* context, bool table, FrontArgs const& f, hipStream_t stream) {
+  if (f.count == 0) return;
+  unsigned const grid = static_cast<unsigned>(std::max<std::uint64_t>(16, f.count / 32));
+  if (table) lepton_moliere_tail_kernel<true><<<grid, moliere::kTailThreads, 0, stream>>>(context, f, 1);
+  else lepton_moliere_tail_kernel<false><<<grid, moliere::kTailThreads, 0, stream>>>(context, f, 1);
+  C8MI_HIP(hipGetLastError());
+}
+
 void launch_lepton_open(EmContext const* context, std::uint32_t bins, bool table, FrontArgs const& f,
                         hipStream_t stream) {
   if (f.count == 0) return;
   constexpr unsigned kTailGrid = 1024, kOpenGrid = 16;
   if (table)
-    lepton_moliere_tail_kernel<true><<<kTailGrid, moliere::kTailThreads, 0, stream>>>(context, f);
+    lepton_moliere_tail_kernel<true><<<kTailGrid, moliere::kTailThreads, 0, stream>>>(context, f, 0);
   else
-    lepton_moliere_tail_kernel<false><<<kTailGrid, moliere::kTailThreads, 0, stream>>>(context, f);
+    lepton_moliere_tail_kernel<false><<<kTailGrid, moliere::kTailThreads, 0, stream>>>(context, f, 0);
   lepton_finish_open_kernel<<<kOpenGrid, kStepBlock, 0, stream>>>(context, f);
   FrontArgs g = f;
   g.vertices = f.open_vertices;
@@ -846,6 +943,17 @@ void launch_lepton_vertex(EmContext const* context, std::uint32_t bins, FrontArg
   if (f.count == 0) return;
   unsigned const grid = grid_for((f.count + kSourcesPerVertexBlock - 1) / kSourcesPerVertexBlock, 1);
   lepton_vertex_kernel<<<grid, kStepBlock, step_lds_bytes(bins), stream>>>(context, f);
+  C8MI_HIP(hipGetLastError());
+}
+
+void launch_compact(bool photon, FrontArgs const& f, ParticleQueue const& next_queue,
+                    ParticleQueue const& other_queue, std::uint64_t other_base, hipStream_t stream) {
+  static_assert(kCompactSources <= kScanBlock, "one source per thread");
+  if (f.count > kCompactSources) throw std::logic_error("em: front above the single-workgroup compaction");
+  if (f.slots > kMaxShowerSlots) throw std::length_error("em: more pool slots than the scan covers");
+  if (f.runs != 1) throw std::logic_error("em: a front's input must be one run sorted by slot");
+  if (f.count == 0) return;
+  compact_kernel<<<1, kScanBlock, 0, stream>>>(f, photon ? 1 : 0, next_queue, other_queue, other_base);
   C8MI_HIP(hipGetLastError());
 }
 
