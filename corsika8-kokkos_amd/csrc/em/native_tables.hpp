@@ -219,8 +219,12 @@ C8MI_HD double cubic(Tables const& t, c8mi_native_cubic const& s, double x) {
   return value;
 }
 
-C8MI_HD double cubic_derivative76(Tables const& t, c8mi_native_cubic const& s,
-                         double x) {
+// cubic() and its derivative from one pass over the coordinate and the coefficients.
+struct CubicSlope {
+  double value, derivative;
+};
+
+C8MI_HD CubicSlope cubic_slope76(Tables const& t, c8mi_native_cubic const& s, double x) {
   double const coordinate = axis_transform(s.axis, x);
   std::uint32_t const node = interval_node(coordinate, s.coefficient_count);
   double const fraction = coordinate - node;
@@ -234,8 +238,12 @@ C8MI_HD double cubic_derivative76(Tables const& t, c8mi_native_cubic const& s,
   double derivative = d[0] * t.cubic_values[off] + d[1] * t.cubic_values[off + 1] +
                       d[2] * t.cubic_node_derivatives[off] +
                       d[3] * t.cubic_node_derivatives[off + 1];
-  if (s.has_value_transform) derivative *= axis_back_derivative(s.value_transform, raw);
-  return derivative * axis_derivative(s.axis, x);
+  double value = raw;
+  if (s.has_value_transform) {
+    value = axis_back_transform(s.value_transform, raw);
+    derivative *= axis_back_derivative(s.value_transform, raw);
+  }
+  return {value, derivative * axis_derivative(s.axis, x)};
 }
 
 C8MI_HD int sgn(double x) { return (0. < x ? 1 : 0) - (x < 0. ? 1 : 0); }
@@ -246,9 +254,10 @@ struct NewtonResult {
   bool runtime_error;
 };
 
-// Boost 1.79 newton_raphson_iterate(f, guess, lower, upper, digits = 20).
-template <class F, class D>
-C8MI_HD NewtonResult newton76(F const& f, D const& df, double initial, double lower,
+// Boost 1.79 newton_raphson_iterate(f, guess, lower, upper, digits = 20);
+// fd(x) gives the value and the derivative.
+template <class F, class FD>
+C8MI_HD NewtonResult newton76(F const& f, FD const& fd, double initial, double lower,
                      double upper) {
   double residual = 0., last_residual = 0., result = initial, guess = initial;
   double delta = 1.7976931348623157e308, delta1 = delta, delta2 = delta;
@@ -259,8 +268,9 @@ C8MI_HD NewtonResult newton76(F const& f, D const& df, double initial, double lo
     last_residual = residual;
     delta2 = delta1;
     delta1 = delta;
-    residual = f(result);
-    double const derivative = df(result);
+    CubicSlope const at = fd(result);
+    residual = at.value;
+    double const derivative = at.derivative;
     ++it;
     if (!isfinite(residual) || !isfinite(derivative)) return {result, it, true};
     if (residual == 0.) break;
@@ -618,7 +628,10 @@ C8MI_HD QueryResult total_rate(Tables const& t, std::int32_t pid, double e) {
   return qr(C8MI_QUERY_SUCCESS, value < 0. ? 0. : value);
 }
 
-C8MI_HD QueryResult selection_total_rate(Tables const& t, std::int32_t pid, double e) {
+// The total selection rate; the rates of the first `kept` columns of the particle
+// are left in `rates`, for a caller that then walks the columns.
+C8MI_HD QueryResult selection_total_rate(Tables const& t, std::int32_t pid, double e,
+                                              double* rates = nullptr, std::uint32_t kept = 0) {
   using namespace detail;
   if (!valid_view(t)) return qr(C8MI_QUERY_INVALID_VIEW);
   double total = 0.;
@@ -627,10 +640,13 @@ C8MI_HD QueryResult selection_total_rate(Tables const& t, std::int32_t pid, doub
   for (std::uint32_t i = begin; i < end; ++i) {
     auto const* c = selection_dndx(t, i);
     if (!c || c->pdg_id != pid) return qr(C8MI_QUERY_INVALID_VIEW);
-    if (rate_below_threshold(*c, e)) continue;
-    QueryResult const r = rate_for_column(t, *c, e);
-    if (r.status != C8MI_QUERY_SUCCESS) return r;
-    total += r.value;
+    QueryResult r = qr(C8MI_QUERY_SUCCESS);
+    if (!rate_below_threshold(*c, e)) {
+      r = rate_for_column(t, *c, e);
+      if (r.status != C8MI_QUERY_SUCCESS) return r;
+      total += r.value;
+    }
+    if (i - begin < kept) rates[i - begin] = r.value;
   }
   if (begin == end) return qr(C8MI_QUERY_PARTICLE_NOT_FOUND);
   return qr(C8MI_QUERY_SUCCESS, total);
@@ -853,66 +869,108 @@ C8MI_HD QueryResult loss_fraction(Tables const& t, std::int32_t pid, std::int32_
   return qr(C8MI_QUERY_SUCCESS, physical, newton, bisection);
 }
 
-C8MI_HD QueryResult range(Tables const& t, std::int32_t pid, double e) {
-  using namespace detail;
-  auto const* c = find_utility(t, pid);
-  if (!c) return qr(C8MI_QUERY_PARTICLE_NOT_FOUND);
-  if (!isfinite(e)) return qr(C8MI_QUERY_NON_FINITE_INPUT);
-  if (e < c->lower_energy_limit_mev || e < c->spline.axis.low || e > c->spline.axis.high)
-    return qr(C8MI_QUERY_ENERGY_OUT_OF_RANGE);
-  double const upper = cubic(t, c->spline, e);
-  double const lower = cubic(t, c->spline, c->lower_energy_limit_mev);
-  double const value = c->reverse ? lower - upper : upper - lower;
-  if (!isfinite(value) || value < 0.) return qr(C8MI_QUERY_INVALID_VIEW);
-  return qr(C8MI_QUERY_SUCCESS, value);
+// A range query with the spline values it is the difference of, for the callers
+// that go on from the same energy.
+struct RangePoint {
+  QueryResult result;
+  double at_energy, at_limit;  // the spline at the energy and at the lower energy limit
+};
+
+C8MI_HD RangePoint range_between(c8mi_native_utility_column const& c, double at_energy, double at_limit) {
+  double const value = c.reverse ? at_limit - at_energy : at_energy - at_limit;
+  if (!isfinite(value) || value < 0.) return {qr(C8MI_QUERY_INVALID_VIEW), at_energy, at_limit};
+  return {qr(C8MI_QUERY_SUCCESS, value), at_energy, at_limit};
 }
 
-C8MI_HD QueryResult energy_after_loss(Tables const& t, std::int32_t pid, double e0,
-                             double grammage) {
+// The checks of a range query that come before its evaluation.
+C8MI_HD std::uint32_t range_status(c8mi_native_utility_column const* c, double e) {
+  if (!c) return C8MI_QUERY_PARTICLE_NOT_FOUND;
+  if (!isfinite(e)) return C8MI_QUERY_NON_FINITE_INPUT;
+  if (e < c->lower_energy_limit_mev || e < c->spline.axis.low || e > c->spline.axis.high)
+    return C8MI_QUERY_ENERGY_OUT_OF_RANGE;
+  return C8MI_QUERY_SUCCESS;
+}
+
+C8MI_HD RangePoint range_point(Tables const& t, c8mi_native_utility_column const* c, double e) {
+  std::uint32_t const status = range_status(c, e);
+  if (status != C8MI_QUERY_SUCCESS) return {qr(status), 0., 0.};
+  double const upper = detail::cubic(t, c->spline, e);
+  double const lower = detail::cubic(t, c->spline, c->lower_energy_limit_mev);
+  return range_between(*c, upper, lower);
+}
+
+// The range at another energy of a column whose value at the lower limit is known.
+C8MI_HD QueryResult range_beside(Tables const& t, c8mi_native_utility_column const* c, double e, RangePoint const& known) {
+  std::uint32_t const status = range_status(c, e);
+  if (status != C8MI_QUERY_SUCCESS) return qr(status);
+  return range_between(*c, detail::cubic(t, c->spline, e), known.at_limit).result;
+}
+
+C8MI_HD QueryResult range(Tables const& t, std::int32_t pid, double e) {
+  return range_point(t, detail::find_utility(t, pid), e).result;
+}
+
+// The energy after a loss, from the range at the initial energy. The spline values
+// at the two ends and at the last lower end of the bisection are kept: of 31
+// evaluations for a typical step of an e+- (with its range queries), 13 remain.
+C8MI_HD QueryResult energy_after_loss(Tables const& t, c8mi_native_utility_column const* c, double e0,
+                                      double grammage, RangePoint const& initial) {
   using namespace detail;
-  auto const* c = find_utility(t, pid);
   if (!c) return qr(C8MI_QUERY_PARTICLE_NOT_FOUND);
   if (!isfinite(e0) || !isfinite(grammage) || grammage < 0.) return qr(C8MI_QUERY_NON_FINITE_INPUT);
   if (e0 < c->lower_energy_limit_mev || e0 > c->spline.axis.high)
     return qr(C8MI_QUERY_ENERGY_OUT_OF_RANGE);
-  QueryResult const maximum = range(t, pid, e0);
+  QueryResult const& maximum = initial.result;
   if (maximum.status != C8MI_QUERY_SUCCESS) return maximum;
   if (grammage > maximum.value) return qr(C8MI_QUERY_ENERGY_OUT_OF_RANGE);
   if (grammage == maximum.value) return qr(C8MI_QUERY_SUCCESS, c->lower_energy_limit_mev);
   if (grammage == 0.) return qr(C8MI_QUERY_SUCCESS, e0);
   double const signed_grammage = c->reverse ? -grammage : grammage;
-  double const target = cubic(t, c->spline, e0) - signed_grammage;
+  double const target = initial.at_energy - signed_grammage;
   auto residual = [&](double e) { return cubic(t, c->spline, e) - target; };
-  auto slope = [&](double e) { return cubic_derivative76(t, c->spline, e); };
+  auto with_slope = [&](double e) {
+    CubicSlope const at = cubic_slope76(t, c->spline, e);
+    return CubicSlope{at.value - target, at.derivative};
+  };
+  // between the lower limit and e0
   auto bisect = [&](double accuracy, double& lower, double& upper, std::uint32_t& iterations) {
-    double const lv = residual(lower), uv = residual(upper);
-    if (!isfinite(lv) || !isfinite(uv) || lv * uv > 0.) return false;
+    lower = c->lower_energy_limit_mev;
+    upper = e0;
+    double at_lower = initial.at_limit - target;
+    double const at_upper = initial.at_energy - target;
+    if (!isfinite(at_lower) || !isfinite(at_upper) || at_lower * at_upper > 0.) return false;
     for (std::uint32_t it = 0; it <= 100; ++it) {
       double const center = (lower + upper) / 2.;
-      double const cv = residual(center);
-      double const clv = residual(lower);
-      if (!isfinite(cv) || !isfinite(clv)) return false;
-      if (sgn(cv) == sgn(clv)) lower = center;
-      else upper = center;
+      double const at_center = residual(center);
+      if (!isfinite(at_center)) return false;
+      if (sgn(at_center) == sgn(at_lower)) {
+        lower = center;
+        at_lower = at_center;
+      } else {
+        upper = center;
+      }
       ++iterations;
       if ((upper - lower) < accuracy) return true;
     }
     return true;
   };
-  double lower = c->lower_energy_limit_mev, upper = e0;
+  double lower, upper;
   std::uint32_t bisection = 0;
   double const coarse = (e0 - c->lower_energy_limit_mev) * 1.e-2;
   if (!bisect(coarse, lower, upper, bisection))
     return qr(C8MI_QUERY_ROOT_NOT_CONVERGED, 0., 0, bisection);
-  double const initial = upper == e0 ? e0 : (lower + upper) / 2.;
-  NewtonResult const n = newton76(residual, slope, initial, lower, upper);
+  double const start = upper == e0 ? e0 : (lower + upper) / 2.;
+  NewtonResult const n = newton76(residual, with_slope, start, lower, upper);
   if (!n.runtime_error && isfinite(n.value))
     return qr(C8MI_QUERY_SUCCESS, n.value, n.iterations, bisection);
-  lower = c->lower_energy_limit_mev;
-  upper = e0;
   if (!bisect(1.e-6, lower, upper, bisection))
     return qr(C8MI_QUERY_ROOT_NOT_CONVERGED, 0., n.iterations, bisection);
   return qr(C8MI_QUERY_SUCCESS, lower, n.iterations, bisection);
+}
+
+C8MI_HD QueryResult energy_after_loss(Tables const& t, std::int32_t pid, double e0, double grammage) {
+  auto const* c = detail::find_utility(t, pid);
+  return energy_after_loss(t, c, e0, grammage, range_point(t, c, e0));
 }
 
 C8MI_HD QueryResult energy_of_range(Tables const& t, std::int32_t pid, double r) {

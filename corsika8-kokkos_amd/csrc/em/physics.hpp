@@ -380,12 +380,14 @@ C8MI_HD Tq cq_minimum_energy(EmContext const& c, std::int32_t pid) {
   return {kTsSuccess, minimum};
 }
 
-C8MI_HD Tq cq_energy_after_loss(EmContext const& c, std::int32_t pid, double e0, double x) {
+// `initial` is the range at e0.
+C8MI_HD Tq cq_energy_after_loss(EmContext const& c, c8mi_native_utility_column const* u, double e0, double x,
+                                RangePoint const& initial) {
   if (!isfinite(x) || x < 0.) return {kTsNonFinite, 0.};
-  Tq const initial = native(range(c.tables, pid, e0), true);
-  if (initial.status != kTsSuccess) return initial;
-  if (x >= initial.value && x != 0.) return {kTsTransportCut, 0.};
-  return native(energy_after_loss(c.tables, pid, e0, x), true);
+  Tq const range = native(initial.result, true);
+  if (range.status != kTsSuccess) return range;
+  if (x >= range.value && x != 0.) return {kTsTransportCut, 0.};
+  return native(energy_after_loss(c.tables, u, e0, x, initial), true);
 }
 
 C8MI_HD bool pk_finite(double v) {
@@ -437,10 +439,16 @@ struct Selection {
   bool selected;
 };
 
+// The rates that the total was summed from are kept for the walk over the columns
+// (7 of photons in air, 5 of positrons): evaluating them a second time up to the selected one was
+// up to half of a selection. Columns beyond the kept ones are evaluated again.
+constexpr std::uint32_t kSelectionRates = 16;
+
 C8MI_HD Selection select_column(EmContext const& c, std::int32_t pid, double e, double u) {
   Selection r{kTsNonFinite, 0, 0, 0., false};
   if (!isfinite(u) || u < 0. || u >= 1.) return r;
-  Tq const total = native(selection_total_rate(c.tables, pid, e), false);
+  double rates[kSelectionRates];
+  Tq const total = native(selection_total_rate(c.tables, pid, e, rates, kSelectionRates), false);
   if (total.status != kTsSuccess) {
     r.status = total.status;
     return r;
@@ -457,7 +465,8 @@ C8MI_HD Selection select_column(EmContext const& c, std::int32_t pid, double e, 
       return r;
     }
     QueryResult rate{C8MI_QUERY_SUCCESS, 0, 0, 0.};
-    if (!detail::rate_below_threshold(*col, e)) rate = rate_for_column(c.tables, *col, e);
+    if (pos - begin < kSelectionRates) rate.value = rates[pos - begin];
+    else if (!detail::rate_below_threshold(*col, e)) rate = rate_for_column(c.tables, *col, e);
     Tq const rt = native(rate, false);
     if (rt.status != kTsSuccess) {
       r.status = rt.status;
@@ -533,6 +542,10 @@ struct Fallback {
   int reason;
 };
 
+// `Photon`: the queue's species (a photon queue holds photons, a lepton queue
+// charged leptons). Leptons select their column at the vertex; without the
+// photons' selection the move kernel needs 168 registers instead of 210.
+template <bool Photon>
 C8MI_HD void select_interaction(EmContext const& c, Particle const& p, Interaction& in,
                        Fallback& fb) {
   in.particle = p;
@@ -554,13 +567,12 @@ C8MI_HD void select_interaction(EmContext const& c, Particle const& p, Interacti
     in.interaction_grammage = __builtin_inf();
     return;
   }
-  bool const charged = is_charged_lepton(p.pid);
-  if (p.pid == 22 && e_mev < c.em_cut_mev) {
+  if (Photon && p.pid == 22 && e_mev < c.em_cut_mev) {
     in.status = kParticleCut;
     in.interaction_grammage = __builtin_inf();
     return;
   }
-  if (charged) {
+  if (!Photon && is_charged_lepton(p.pid)) {
     Tq const mass = cq_mass(c, p.pid);
     if (mass.status == kTsSuccess) in.particle_mass_gev = mass.value / 1000.;
     double const tm = 1000. * transport_mass(p.pid);
@@ -588,7 +600,7 @@ C8MI_HD void select_interaction(EmContext const& c, Particle const& p, Interacti
   double const ud = uniform(c, p, kDistanceProcess, 0);
   in.interaction_grammage = -log(ud) / total.value;
   in.process_uniform = uniform(c, p, kColumnProcess, 0);
-  if (charged) {
+  if constexpr (!Photon) {
     in.status = kDistanceSampled;
     return;
   }

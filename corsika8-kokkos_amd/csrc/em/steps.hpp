@@ -19,7 +19,7 @@ C8MI_HD void photon_step(EmContext const& c, Accumulator const& acc, Particle co
                 Outputs& o) {
   Interaction in;
   Fallback fb{false, 0};
-  select_interaction(c, p, in, fb);
+  select_interaction<true>(c, p, in, fb);
   if (fb.flag) {
     record_fallback(acc, p, fb.reason, in.process_id, kStageSelection);
     return;
@@ -317,7 +317,7 @@ C8MI_HD bool lepton_move(EmContext const& c, Accumulator const& acc, Particle co
                          LeptonMove& mv) {
   Interaction in;
   Fallback fb{false, 0};
-  select_interaction(c, p, in, fb);
+  select_interaction<false>(c, p, in, fb);
   if (fb.flag) {
     record_fallback(acc, p, fb.reason, in.process_id, kStageSelection);
     return false;
@@ -363,12 +363,15 @@ C8MI_HD bool lepton_move(EmContext const& c, Accumulator const& acc, Particle co
   if (!is_ee(start.pid)) return transport_fallback(kFrUnsupportedParticle);
   bool const particle_cut = in.status == kParticleCut || e0 - tm < tcut.value;
   double max_grammage = 0.;
+  c8mi_native_utility_column const* const utility = detail::find_utility(c.tables, start.pid);
+  RangePoint range0{};
   if (!particle_cut) {
-    Tq const r0 = native(range(c.tables, start.pid, e0), true);
+    range0 = range_point(c.tables, utility, e0);
+    Tq const r0 = native(range0.result, true);
     if (r0.status != kTsSuccess) return transport_fallback(fallback_reason(r0.status));
     double const rl = (1. - kMaxRelativeLoss) * e0;
     double const target = rl > minimum.value ? rl : minimum.value;
-    Tq const r1 = native(range(c.tables, start.pid, target), true);
+    Tq const r1 = native(range_beside(c.tables, utility, target, range0), true);
     if (r1.status != kTsSuccess) return transport_fallback(fallback_reason(r1.status));
     max_grammage = r0.value - r1.value;
     double const scale = r0.value > 1. ? r0.value : 1.;
@@ -449,7 +452,7 @@ C8MI_HD bool lepton_move(EmContext const& c, Accumulator const& acc, Particle co
     if (cg.status != env::kSuccess) return transport_fallback(kFrGrammage);
     traversed = cg.value;
     step_grammage = traversed;
-    Tq const fe = cq_energy_after_loss(c, start.pid, e0, traversed);
+    Tq const fe = cq_energy_after_loss(c, utility, e0, traversed, range0);
     double final_mev;
     bool cut_reached = false;
     if (fe.status == kTsSuccess) {

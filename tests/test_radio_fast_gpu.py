@@ -98,3 +98,32 @@ def test_large_increments():
         want = ref[name + "_fixed"].astype(np.float64)
         assert np.abs(want).max() > 2.0 ** 52
         assert np.linalg.norm(got[k] - want) <= 1e-6 * np.linalg.norm(want)
+
+
+# The launch gives a workgroup more observers the more there are; 64-bin windows leave room
+# for eight of them. Each observer has its own height, rate, bins and window here.
+@pytest.mark.parametrize("observers,count", [(17, 9000), (33, 700), (65, 3001), (100, 9000), (66, 40000), (61, 40000)])
+@pytest.mark.parametrize("mode", ["both", "coreas", "zhs"])
+def test_groups_of_observers_and_their_remainders(observers, count, mode):
+    rng = np.random.default_rng(observers)
+    tracks = mixed(count, 100 + observers, 0.1)
+    positions = np.stack([rng.uniform(-60, 60, observers), rng.uniform(-60, 60, observers), rng.uniform(0.0, 40.0, observers)], 1)
+    obs = window_observers(tracks, [tuple(p) for p in positions], 1.0e9, 64)
+    obs["sample_rate_hz"] = rng.choice((2.5e8, 5.0e8, 1.0e9), observers)
+    obs["number_of_bins"] = rng.integers(2, 65, observers)
+    obs["duration_s"] = (obs["number_of_bins"] - 1.0) / obs["sample_rate_hz"]
+    prop = exponential_table()
+    modes = dict(coreas=mode != "zhs", zhs=mode != "coreas")
+    ref = oracle_lib.radio_project(prop, obs, tracks, limit=LIMIT, threads=4)
+    got = gpu_project(tracks, obs, prop, exact=False, limit=LIMIT, **modes)
+    ends = np.cumsum(obs["number_of_bins"].astype(np.int64))
+    for fixed, name in ((got[0], "coreas"), (got[1], "zhs")):
+        if not modes[name]:
+            continue
+        field = oracle_lib.radio_decode(fixed, obs, limit=LIMIT, potential=name == "zhs")
+        want = ref[name + "_float"]
+        for k, end in enumerate(ends):
+            part = slice(int(end) - int(obs["number_of_bins"][k]), int(end))
+            error = np.linalg.norm(field[:, part] - want[:, part])
+            assert error <= 1e-6 * np.linalg.norm(want[:, part]), (name, k)
+        assert got[2][name + "_contributions"] == ref["counters"][name + "_contributions"]
