@@ -586,8 +586,16 @@ C8MI_HD QueryResult cumulative_rate(Tables const& t, c8mi_native_dndx_column con
   return cumulative_rate(t, c, e, loss, [&] { return detail::bicubic76(t, c.spline, e, loss); });
 }
 
+// The powers of a Sauter rate that no column enters, for the caller that
+// evaluates several columns at one energy (a pow is ~270 dependent instructions,
+// a Sauter rate was five of them).
+struct SauterPowers {
+  bool known;
+  double alpha4, energy5;
+};
+
 C8MI_HD QueryResult rate_for_column(Tables const& t, c8mi_native_dndx_column const& c,
-                                    double e) {
+                                    double e, SauterPowers& powers) {
   using namespace detail;
   if (!valid_view(t)) return qr(C8MI_QUERY_INVALID_VIEW);
   if (rate_below_threshold(c, e)) return qr(C8MI_QUERY_SUCCESS);
@@ -610,7 +618,8 @@ C8MI_HD QueryResult rate_for_column(Tables const& t, c8mi_native_dndx_column con
     double const gamma = 1. + (e - ionization) / me;
     double const gamma_beta = sqrt(gamma * gamma - 1.);
     double const sigma_t = 8. * pi * re * re / 3.;
-    double const sigma = 1.5 * sigma_t * pow(z, 5.) * pow(alpha, 4.) * pow(me / e, 5.) *
+    if (!powers.known) powers = {true, pow(alpha, 4.), pow(me / e, 5.)};
+    double const sigma = 1.5 * sigma_t * pow(z, 5.) * powers.alpha4 * powers.energy5 *
                          pow(gamma_beta, 3.) *
                          (4. / 3. + gamma * (gamma - 2.) / (gamma + 1.) *
                                         (1. - log(gamma + gamma_beta) / (gamma * gamma_beta)));
@@ -660,6 +669,11 @@ C8MI_HD QueryResult rate_for_column(Tables const& t, c8mi_native_dndx_column con
   return cumulative_rate(t, c, e, 1.);
 }
 
+C8MI_HD QueryResult rate_for_column(Tables const& t, c8mi_native_dndx_column const& c, double e) {
+  SauterPowers powers{};
+  return rate_for_column(t, c, e, powers);
+}
+
 C8MI_HD QueryResult query_rate(Tables const& t, std::int32_t pid, std::int32_t process,
                       std::uint64_t component, double e) {
   using namespace detail;
@@ -692,12 +706,13 @@ C8MI_HD QueryResult selection_total_rate(Tables const& t, std::int32_t pid, doub
   double total = 0.;
   std::uint32_t begin, end;
   dndx_range(t, pid, begin, end);
+  SauterPowers powers{};
   for (std::uint32_t i = begin; i < end; ++i) {
     auto const* c = selection_dndx(t, i);
     if (!c || c->pdg_id != pid) return qr(C8MI_QUERY_INVALID_VIEW);
     QueryResult r = qr(C8MI_QUERY_SUCCESS);
     if (!rate_below_threshold(*c, e)) {
-      r = rate_for_column(t, *c, e);
+      r = rate_for_column(t, *c, e, powers);
       if (r.status != C8MI_QUERY_SUCCESS) return r;
       total += r.value;
     }

@@ -417,17 +417,21 @@ C8MI_HD bool encode_pair_split(double e, double rho, double& s) {
   return pk_finite(s) && s >= 0. && s <= 1.;
 }
 
+// The loss fraction of the native pair split as the final state takes it.
+C8MI_HD Tq pair_split(QueryResult const& split, double e) {
+  Tq const r = native(split, false);
+  if (r.status != kTsSuccess) return r;
+  double s = 0.;
+  if (!encode_pair_split(e / 1000., r.value, s)) return {kTsInverseCdf, 0.};
+  return {kTsSuccess, s};
+}
+
 C8MI_HD Tq dq_loss_fraction(EmContext const& c, std::int32_t pid, std::int32_t process,
                    std::uint64_t comp, double e, double q) {
   if (process == kPhotonMuPairFinalState && pid == 22)
     return native(loss_fraction(c.tables, pid, kPhotonMuPair, comp, e, q, true), false);
-  if (process == kPhotonPairFinalState && pid == 22) {
-    Tq r = native(loss_fraction(c.tables, pid, kPhotonPair, comp, e, q, true), false);
-    if (r.status != kTsSuccess) return r;
-    double s = 0.;
-    if (!encode_pair_split(e / 1000., r.value, s)) return {kTsInverseCdf, 0.};
-    return {kTsSuccess, s};
-  }
+  if (process == kPhotonPairFinalState && pid == 22)
+    return pair_split(loss_fraction(c.tables, pid, kPhotonPair, comp, e, q, true), e);
   return native(loss_fraction(c.tables, pid, process, comp, e, q, false), false);
 }
 
@@ -535,6 +539,8 @@ struct Interaction {
   double energy_fraction;
   double process_uniform;
   double loss_quantile;
+  bool pair_split_drawn;  // a selected pair: its split, drawn with the selection
+  Tq pair_split;
 };
 
 struct Fallback {
@@ -561,6 +567,8 @@ C8MI_HD void select_interaction(EmContext const& c, Particle const& p, Interacti
   in.energy_fraction = 0.;
   in.process_uniform = 0.;
   in.loss_quantile = 0.;
+  in.pair_split_drawn = false;
+  in.pair_split = {kTsSuccess, 0.};
   double const e_mev = p.energy_gev * 1000.;
   if (native_muon_pair_cut(p) || p.time_s > kCutTime) {
     in.status = kParticleCut;
@@ -621,7 +629,28 @@ C8MI_HD void select_interaction(EmContext const& c, Particle const& p, Interacti
     in.deferred_reason = kFrSelectionReplay;
     return;
   }
-  Tq const loss = dq_loss_fraction(c, p.pid, s.process, s.component, e_mev, s.quantile);
+  // A pair takes all the energy: its loss fraction is 1 without a query, and its
+  // split, which the final state needs, is drawn here instead, in the same query
+  // as the other photons' losses. Two queries of a wave one after the other were a
+  // third of the photon kernel (45 and 39 of 125 us); the split of a photon that
+  // does not reach its vertex is not used.
+  bool pair = p.pid == 22 && s.process == kPhotonPair;
+  if (pair) {
+    auto const* column = detail::find_dndx(c.tables, p.pid, s.process, s.component);
+    pair = column && column->kinematic_model == C8MI_KIN_PHOTON_PAIR_FULL_LOSS;
+  }
+  double const quantile = pair ? uniform(c, p, kPhotonPair, 1) : s.quantile;
+  bool const muon_split = s.process == kPhotonMuPairFinalState && p.pid == 22;
+  bool const split = s.process == kPhotonPairFinalState && p.pid == 22;
+  QueryResult const query = loss_fraction(
+      c.tables, p.pid, muon_split ? std::int32_t{kPhotonMuPair} : split ? std::int32_t{kPhotonPair} : s.process, s.component, e_mev, quantile,
+      pair || muon_split || split);
+  Tq loss = split ? pair_split(query, e_mev) : native(query, false);
+  if (pair) {
+    in.pair_split = pair_split(query, e_mev);
+    in.pair_split_drawn = true;
+    loss = {kTsSuccess, 1.};
+  }
   if (loss.status != kTsSuccess) {
     int const reason = fallback_reason(loss.status);
     if (requires_selected_loss(reason)) {

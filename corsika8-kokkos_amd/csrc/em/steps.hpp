@@ -233,9 +233,11 @@ C8MI_HD void photon_step(EmContext const& c, Accumulator const& acc, Particle co
   if (!isfinite(parent.energy_gev) || parent.energy_gev < 2. * kElectronMassGeV ||
       parent.generation == 0xffffffffU || parent.step_id == 0xffffffffffffffffULL)
     return final_fallback(kFrInvalidFinalState);
-  double const su = uniform(c, parent, kPhotonPair, 1);
-  Tq const split = dq_loss_fraction(c, parent.pid, kPhotonPairFinalState, in.component_hash,
-                                    parent.energy_gev * 1000., su);
+  Tq split = in.pair_split;
+  if (!in.pair_split_drawn) {
+    double const su = uniform(c, parent, kPhotonPair, 1);
+    split = dq_loss_fraction(c, parent.pid, kPhotonPairFinalState, in.component_hash, parent.energy_gev * 1000., su);
+  }
   if (split.status != kTsSuccess) return final_fallback(fallback_reason(split.status));
   double rho = 0.;
   if (!decode_pair_split(parent.energy_gev, split.value, rho)) return final_fallback(kFrInvalidFinalState);
