@@ -15,6 +15,11 @@
 //              accumulate in workgroup-private LDS copies (one for the shower
 //              of the workgroup's first source, one for its last) that are
 //              added to the showers' device totals once per workgroup.
+//              With Moliere scattering the transport part is split into move,
+//              moliere, tail (the few samples that need long series) and finish.
+//              The step kernels read the context and the small tables from LDS.
+//   compact    fronts of at most kCompactSources sources: the four kernels
+//              below in one workgroup.
 //   count      per-workgroup output counts and per-(slot, run) output totals
 //              from the packed words.
 //   scan       one workgroup: exclusive scan of the per-workgroup counts, and

@@ -134,8 +134,10 @@ void launch_radio_segments(FrontArgs const& f, std::uint32_t slots, unsigned lon
 void launch_lepton_moliere(EmContext const* context, bool table, std::uint32_t components, FrontArgs const& f,
                            hipStream_t stream);
 // Fronts of at most so many e+- run the tail kernel in line: its sources then go
-// through the finish and vertex kernels with the others. Above, one of the rare
-// samples of 100 iterations (~150 us) would hold up the front too often.
+// through the finish and vertex kernels with the others. Above, its few samples
+// overlap the finish and vertices of the others (all in line: pool of 1000 showers
+// 340 -> 342 ms, serving stream 519 -> 530, 10 TeV in ice 542 -> 549; a small front
+// gains more from the two launches and events it saves).
 inline constexpr std::uint64_t kInlineTailSources = 8192;
 void launch_lepton_tail(EmContext const* context, bool table, FrontArgs const& f, hipStream_t stream);
 // The open Molière samples on a stream of their own, overlapping the finish

@@ -409,8 +409,8 @@ C8MI_HD int newton_iterate(c8mi_moliere_snapshot const& m, Quotients const& q, T
 //
 // About one e+- step in a hundred draws a quantile whose iterates reach the
 // large-x expansions (two dozen pow per component and iteration), one in 1e5 one
-// whose iteration runs through them to its limit of 100: serially ~1 ms of one
-// lane, and the whole launch waits for it. The step kernels therefore stop before
+// whose iteration never converges (newton_iterate_wave): serially up to ~1 ms of
+// one lane, and the whole launch waits for it. The step kernels therefore stop before
 // such an evaluation (open_above) or after a few iterations
 // (EmContext::moliere_fast_iterations); a sample still open continues here
 // with its iterate: each evaluation spreads the transcendental parts of every
@@ -537,16 +537,34 @@ __device__ __forceinline__ void evaluate_wave(c8mi_moliere_snapshot const& m, Qu
 }
 
 // newton_iterate with the workgroup evaluation (every thread the same iterates).
+//
+// The samples that run to the limit of 100 iterations are those whose target lies
+// in a step of the CDF where two of its forms meet: the iterates fall into a cycle
+// of two, one on either side, further apart than the convergence test allows. Once
+// three iterates in a row repeat the one before last to 1e-10 while neighbours
+// differ by twice the tolerance or more, the iteration has contracted onto such a
+// cycle and the outcome is the one of iteration 100 (its value is not used): of
+// 1.16e7 draws in air and ice, table and analytic, 6620 ran to the limit, 6594 were
+// recognised after 8 iterations (table) or 13 on average, and none of them would
+// have converged. The tail kernel of a pool of 512 showers took 216 us on average.
 template <bool Tab, int Cap>
 __device__ __forceinline__ int newton_iterate_wave(c8mi_moliere_snapshot const& m, Quotients const& q,
                                                    Table const& t, State<Cap> const& st, double u, int first,
                                                    double* jobs, double& current) {
   double const target = u - 0.5;
+  double previous = __builtin_nan("");  // the iterate before `current`
+  int repeats = 0;
   for (int it = first; it <= kMaximumIterations; ++it) {
+    double const before = previous;
+    previous = current;
     double density, cdf;
     evaluate_wave<Tab>(m, q, t, st, current, jobs, density, cdf);
     int const status = newton_update(density, cdf, target, current);
     if (status != kStarted) return status;
+    bool const repeated = fabs(current - before) <= 1.e-10 * fabs(current) &&
+                          fabs(current - previous) >= 1.e-4 * fabs(current);
+    repeats = repeated ? repeats + 1 : 0;
+    if (repeats == 3) return kNonConvergent;
   }
   return kNonConvergent;
 }
