@@ -872,9 +872,11 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
     bool const table = host_context_.moliere_polynomials != nullptr;
     launch_lepton_moliere(context_.data(), table, host_context_.moliere.component_count, f, stream_);
     mark(kKernLeptonTransport);
-    bool const in_line = m <= kInlineTailSources;
-    if (in_line) {
+    if (m <= kInlineTailSources) {
       launch_lepton_tail(context_.data(), table, f, stream_);
+      mark(kKernLeptonTransport);
+      launch_lepton_finish_vertex(context_.data(), config_.profile_bins, f, stream_);
+      mark(kKernLeptonVertex);
     } else {
       // the open samples continue on the side stream while the other sources
       // finish and run their vertices here
@@ -882,12 +884,12 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
       C8MI_HIP(hipStreamWaitEvent(side_stream_, open_ready_, 0));
       launch_lepton_open(context_.data(), config_.profile_bins, table, f, side_stream_);
       C8MI_HIP(hipEventRecord(open_done_, side_stream_));
+      launch_lepton_finish(context_.data(), config_.profile_bins, f, stream_);
+      mark(kKernLeptonTransport);
+      launch_lepton_vertex(context_.data(), config_.profile_bins, f, stream_);
+      mark(kKernLeptonVertex);
+      C8MI_HIP(hipStreamWaitEvent(stream_, open_done_, 0));
     }
-    launch_lepton_finish(context_.data(), config_.profile_bins, f, stream_);
-    mark(kKernLeptonTransport);
-    launch_lepton_vertex(context_.data(), config_.profile_bins, f, stream_);
-    mark(kKernLeptonVertex);
-    if (!in_line) C8MI_HIP(hipStreamWaitEvent(stream_, open_done_, 0));
     mark(kKernLeptonTransport);  // what the open samples add beyond the overlap
     project_tracks();
   } else {

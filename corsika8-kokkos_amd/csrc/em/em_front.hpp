@@ -133,12 +133,13 @@ void launch_radio_segments(FrontArgs const& f, std::uint32_t slots, unsigned lon
 // components: those of the Molière snapshot.
 void launch_lepton_moliere(EmContext const* context, bool table, std::uint32_t components, FrontArgs const& f,
                            hipStream_t stream);
-// Fronts of at most so many e+- run the tail kernel in line: its sources then go
-// through the finish and vertex kernels with the others. Above, its few samples
-// overlap the finish and vertices of the others (all in line: pool of 1000 showers
-// 340 -> 342 ms, serving stream 519 -> 530, 10 TeV in ice 542 -> 549; a small front
-// gains more from the two launches and events it saves).
-inline constexpr std::uint64_t kInlineTailSources = 8192;
+// Fronts of at most so many e+- run the tail kernel in line and finish and
+// vertices in one kernel (launch_lepton_finish_vertex). Above, finish and vertex
+// are kernels of their own, and the tail's few samples overlap them. Measured at
+// limits of 8192, 65536, 131072 and none: 10 TeV in ice 495, 478, 471 and 468 ms,
+// pool of 1000 showers in 512 slots 339.7, 339.3, 337.4 and 352.6, pool of 3000
+// in 3000 slots 946, 949, 946 and 987.
+inline constexpr std::uint64_t kInlineTailSources = 131072;
 void launch_lepton_tail(EmContext const* context, bool table, FrontArgs const& f, hipStream_t stream);
 // The open Molière samples on a stream of their own, overlapping the finish
 // and vertex kernels of the other sources: tail kernel, their finish, their
@@ -146,6 +147,8 @@ void launch_lepton_tail(EmContext const* context, bool table, FrontArgs const& f
 void launch_lepton_open(EmContext const* context, std::uint32_t bins, bool table, FrontArgs const& f,
                         hipStream_t stream);
 void launch_lepton_finish(EmContext const* context, std::uint32_t bins, FrontArgs const& f, hipStream_t stream);
+// Both for a front whose tail ran in line.
+void launch_lepton_finish_vertex(EmContext const* context, std::uint32_t bins, FrontArgs const& f, hipStream_t stream);
 void launch_lepton_vertex(EmContext const* context, std::uint32_t bins, FrontArgs const& f, hipStream_t stream);
 // Fronts of at most so many sources are compacted by one workgroup
 // (launch_compact) instead of the count, scan, slot update and scatter kernels:
