@@ -1043,8 +1043,7 @@ def main():
     kernel_avg_ms = kernel_total_ms / max(launches, 1)
     achieved = FLOPS_PER_UPDATE[kind] * updates / (kernel_avg_ms * 1e-3) / 1e12
     labels = {"coreas_zhs": (1, 1), "coreas": (1, 0), "zhs": (0, 1)}
-    kernel_name = "radio_project_kernel<coreas=%d,zhs=%d,fixed=1,exact=%d>" % (
-        labels[kind] + (int(args.exact),))
+    kernel_name = "radio_%s_kernel<coreas=%d,zhs=%d>" % (("exact" if args.exact else "fast",) + labels[kind])
     result = {
         "metric": METRIC,
         "value": value,
@@ -1057,7 +1056,7 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f64",
-        "precision": "exact FP64 order" if args.exact else "FP64, hardware reciprocal/rsqrt + Newton",
+        "precision": "exact FP64 order" if args.exact else "FP64, hardware reciprocal/rsqrt + third-order Newton",
         "data": "synthetic",
         "config": {
             "workload": f"radio standalone: {n} tracks x {observers.size} antennas, "

@@ -142,9 +142,9 @@ class RadioAccumulator {
 
   std::uint64_t chunk_tracks_ = 0;     // 0: automatic
   std::uint32_t tile_bins_limit_ = 0;  // 0: automatic
-  // Defaults measured on MI355X for 2^20 tracks x 160 antennas x 2048 bins:
-  // separate CoREAS and ZHS launches (48 KiB LDS each, three workgroups per
-  // CU), 512 threads, about 8192 workgroups per launch.
+  // Separate CoREAS and ZHS launches; about 8192 workgroups for the exact
+  // projection (48 KiB window tiles, 512 threads), measured on MI355X for 2^20
+  // tracks x 160 antennas x 2048 bins. The fast one's shape is estimated per launch.
   std::uint32_t target_workgroups_ = 8192;
   std::uint32_t block_threads_ = 0;  // 0: by the launch's shape
   bool split_ = true;

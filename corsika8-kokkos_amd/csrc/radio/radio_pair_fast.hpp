@@ -208,7 +208,7 @@ __device__ __forceinline__ double doppler(double index, V3 beta, V3 emit, double
 }
 
 // Per-thread tallies. The 32-bit counts cannot wrap: a workgroup takes at most
-// 2^30 tracks (kMaxChunkTracks), a thread 2^22 of them.
+// 2^27 tracks (kMaxChunkTracks) of 8 observers (kMaxGroup), a thread 2^22 of the pairs.
 struct Tally {
   std::uint32_t coreas = 0, single_subtracks = 0, valid = 0;
   unsigned long long zhs = 0, subtracks = 0, overflow = 0;
