@@ -11,8 +11,6 @@
 //    multiply-adds instead of two cross products;
 //  * the fixed-point scale rides on the amplitude, so a sample's components are
 //    its increments; the three range checks are one comparison of their sum;
-//  * a ZHS segment's arrival times are its midpoint's -+ (half duration)
-//    |1 - n e.b|; in one bin the denominator cancels (no reciprocal);
 //  * the first, middle and last bins of a ZHS segment share their difference-array
 //    entries (four per component instead of six).
 // Arrival times stay at FP64 accuracy: a sample is a spike in one bin, and a delay
@@ -378,18 +376,26 @@ __device__ __forceinline__ void add_segment_row(long long* row, std::int32_t bin
   add(l2 + 1, 0ull - l);
 }
 
-// Arrival of a ZHS segment in bins of the observer: centre -+ spread.
+// Arrival of a ZHS segment at the observer, in seconds and bins, in the
+// reference's order: near the Cherenkov angle the difference of the two times is
+// the rounding of each, divided by 1 - n e.b, and a mathematically equal form
+// (midpoint -+ half the spread, or the duration in one bin) rounds differently:
+// 1e-8 to 1e-7 of the field of an in-ice track list against 1e-9 to 9e-9.
 struct Arrival {
-  double x1, x2, b1, b2, den;
+  double d1, d2, x1, x2, b1, b2, den;
 };
 __device__ __forceinline__ Arrival segment_arrival(Path const& path, double index, double beta_emit,
-                                                   double middle_time, double half_duration, View const& o) {
+                                                   double time1, double time2, View const& o) {
   Arrival a;
-  a.den = fma(-index, beta_emit, 1.);
-  double const spread = half_duration * fabs(a.den);
-  double const centre = middle_time + path.time;
-  a.x1 = ((centre - spread) - o.start) * o.rate;
-  a.x2 = ((centre + spread) - o.start) * o.rate;
+  double const slope = index * beta_emit;
+  a.den = 1. - slope;
+  double const middle = (time1 + time2) * 0.5;
+  double const first = time1 + path.time - slope * (time1 - middle);
+  double const second = time2 + path.time - slope * (time2 - middle);
+  a.d1 = first > second ? second : first;
+  a.d2 = first > second ? first : second;
+  a.x1 = (a.d1 - o.start) * o.rate;
+  a.x2 = (a.d2 - o.start) * o.rate;
   a.b1 = nearest_bin(a.x1);
   a.b2 = nearest_bin(a.x2);
   return a;
@@ -397,8 +403,7 @@ __device__ __forceinline__ Arrival segment_arrival(Path const& path, double inde
 
 // A segment over one bin or two neighbouring ones, as the difference array's
 // entries at the first bin and the two after it. u: e x (b x e) times the
-// amplitude over the distance; in one bin the denominator cancels and the
-// potential is u times the duration.
+// amplitude over the distance.
 __device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival const& a, View const& o,
                                                   long long* tile, std::uint32_t stride, Tally& tally) {
   bool const two = a.b1 != a.b2;
@@ -407,7 +412,8 @@ __device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival
   std::int32_t const at = static_cast<std::int32_t>(a.b1 - o.tile_begin);  // -1 .. bins - 1
   bool const has_first = at >= 0, has_last = two && at + 1 < bins;
   // a part without its bin in this tile takes no part in the sums
-  double const first = !has_first ? 0. : two ? (a.b1 + 0.5 - a.x1) * k : duration * o.rate;
+  double const whole = fabs(a.den) > 1.e-15 ? fabs(a.d2 * o.rate - a.d1 * o.rate) * k : duration * o.rate;
+  double const first = !has_first ? 0. : two ? (a.b1 + 0.5 - a.x1) * k : whole;
   double const last = has_last ? (a.x2 + 0.5 - a.b2) * k : 0.;
   double const bound = (fabs(u.x) + fabs(u.y) + fabs(u.z)) * (fabs(first) + fabs(last));
   std::uint32_t const base = at > 0 ? static_cast<std::uint32_t>(at) : 0u;
@@ -460,15 +466,15 @@ __device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival
 
 // One ZHS segment of any length. `subdivided` keeps the reference's sign of the
 // middle bins.
-__device__ __forceinline__ void zhs_segment(Path const& path, double index, double beta_emit, double middle_time,
-                                            double half_duration, Track const& t, View const& o,
+__device__ __forceinline__ void zhs_segment(Path const& path, double index, double beta_emit, double time1,
+                                            double time2, Track const& t, View const& o,
                                             long long* tile, std::uint32_t stride, Tally& tally,
                                             bool subdivided) {
-  Arrival const a = segment_arrival(path, index, beta_emit, middle_time, half_duration, o);
+  Arrival const a = segment_arrival(path, index, beta_emit, time1, time2, o);
   if (!(a.b2 >= o.tile_begin && a.b1 < o.tile_end)) return;
   V3 const u = transverse(path.emit, t.beta, beta_emit, -(t.amplitude * path.inv_distance * o.scale));
   if (a.b2 - a.b1 <= 1.) {
-    add_short_segment(u, 2. * half_duration, a, o, tile, stride, tally);
+    add_short_segment(u, time2 - time1, a, o, tile, stride, tally);
     return;
   }
   std::int32_t const bins = static_cast<std::int32_t>(o.tile_end - o.tile_begin);
@@ -517,7 +523,7 @@ __device__ __forceinline__ void zhs_update(Track const& t, Source const& middle,
   double const measure = fraunhofer(mp, bm, t.duration, length2, o);
   if (!(measure > 1.) && refinement <= 1u) {
     if (count_subtracks) ++tally.single_subtracks;
-    zhs_segment(mp, middle.index, bm, (t.t0 + t.t1) * 0.5, t.duration * 0.5, t, o, tile, stride, tally, false);
+    zhs_segment(mp, middle.index, bm, t.t0, t.t1, t, o, tile, stride, tally, false);
     return;
   }
   double divisor = 1.;
@@ -544,8 +550,7 @@ __device__ __forceinline__ void zhs_update(Track const& t, Source const& middle,
     Source const part =
         make_source<Homogeneous>(p, {(p1.x + p2.x) * 0.5, (p1.y + p2.y) * 0.5, (p1.z + p2.z) * 0.5}, part_kind);
     Path const path = propagate<Homogeneous>(p, o, part, part_kind);
-    zhs_segment(path, part.index, dot(t.beta, path.emit), (time1 + time2) * 0.5, (time2 - time1) * 0.5, t, o, tile,
-                stride, tally, true);
+    zhs_segment(path, part.index, dot(t.beta, path.emit), time1, time2, t, o, tile, stride, tally, true);
     p1 = p2;
     time1 = time2;
   }
