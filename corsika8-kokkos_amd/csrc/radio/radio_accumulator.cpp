@@ -213,7 +213,7 @@ void RadioAccumulator::check_accumulate(std::uint64_t count) const {
   if (sealed_) throw std::logic_error("radio endpoint already committed; reset before new tracks");
   // the launch shapes project() will build (they throw on oversized batches)
   bool const coreas = !coreas_host_.empty(), zhs = !zhs_host_.empty();
-  if (fuse_ && !split_) {
+  if (one_launch()) {
     (void)base_launch(true, true, static_cast<std::uint32_t>(coreas_host_.size()),
                       std::max(coreas_max_bins_, zhs_max_bins_), count);
     return;
@@ -280,7 +280,7 @@ void RadioAccumulator::project(double const* tracks, std::uint64_t stride, std::
     statistics_.track_observer_pairs += count * observers * (std::uint64_t(coreas) + zhs);
     if (coreas && zhs) statistics_.fused_track_observer_pairs += count * observers;
   };
-  if (fuse_ && !split_) {
+  if (one_launch()) {
     run(true, true, true);
   } else {
     bool first = true;

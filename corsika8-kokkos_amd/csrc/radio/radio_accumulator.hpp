@@ -92,6 +92,8 @@ class RadioAccumulator {
  private:
   void project(double const* tracks, std::uint64_t stride, std::uint64_t count);
   void project_batch();
+  // CoREAS and ZHS in one kernel: fusable, asked for, and not the exact form.
+  bool one_launch() const noexcept { return fuse_ && !split_ && !(config_.deterministic && config_.exact_fp64); }
   void ensure_track_capacity(std::uint64_t count);
   ProjectionLaunch base_launch(bool coreas, bool zhs, std::uint32_t observers,
                                std::uint64_t max_bins, std::uint64_t count) const;

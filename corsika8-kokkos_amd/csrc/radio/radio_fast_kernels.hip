@@ -56,7 +56,8 @@ constexpr std::uint32_t kForwardBit = 1u << 31;
 constexpr std::uint32_t kMemberShift = 27;  // track in the chunk below, observer of the group above
 static_assert(kMaxChunkTracks <= (std::uint64_t{1} << kMemberShift), "list entries hold a chunk's tracks");
 static_assert(kMaxGroup <= 16, "list entries hold four bits of observer");
-static_assert(kPairListBytesPerThread * 64 == kListEntries * sizeof(std::uint32_t), "LDS budget of the lists");
+static_assert(kPairListBytesPerThread * 64 == kListEntries * sizeof(std::uint32_t), "LDS of the lists");
+static_assert(kBudgetBytesPerObserver == kRanges * sizeof(Budget), "LDS of the budgets");
 
 // Appends the lanes' entries where `listed`; true when a full wave of them is
 // due (take_pair).
@@ -83,7 +84,8 @@ __device__ __forceinline__ void project_chunk(ProjectionLaunch const& L, Observe
                                               ObserverDev const* zhs_observers, std::uint32_t members,
                                               std::uint32_t tile_begin, std::uint64_t chunk_begin,
                                               std::uint64_t chunk_end, long long* tiles, bool count_valid,
-                                              std::uint32_t* entries, fast::Tally& tally) {
+                                              std::uint32_t* entries, std::uint32_t first, Budget* budgets,
+                                              fast::Tally& tally) {
   PropagationDev const& prop = L.propagation;
   std::uint32_t const W = L.tile_bins;
   std::uint32_t const words = (Coreas ? 3 * W : 0) + (Zhs ? 3 * (W + 1) : 0);  // tile words of a member
@@ -95,7 +97,7 @@ __device__ __forceinline__ void project_chunk(ProjectionLaunch const& L, Observe
     fast::Track t;
     (void)fast::load_track(chunk, L.stride, entry & ((1u << kMemberShift) - 1u), t);
     fast::coreas_near<Homogeneous>(t, prop, make_view(coreas_observers[member], tile_begin, W), tiles + member * words,
-                                   W, tally, (entry & kForwardBit) != 0);
+                                   W, {first + member, nullptr}, tally, (entry & kForwardBit) != 0);
   };
   for (std::uint32_t i = 0; i < count; i += Block) {
     fast::Track t;
@@ -122,14 +124,15 @@ __device__ __forceinline__ void project_chunk(ProjectionLaunch const& L, Observe
         if (active) {
           fast::View const v = make_view(*(ObserverConst*)(zhs_observers + k), tile_begin, W);
           fast::zhs_update<Homogeneous>(t, middle, middle_kind, length2, prop, L.zhs_refinement, v,
-                                        tile + (Coreas ? 3 * W : 0), W + 1, tally, tile_begin == 0);
+                                        tile + (Coreas ? 3 * W : 0), W + 1, {first + k, budgets + k * kRanges}, tally, tile_begin == 0);
         }
       }
       if constexpr (Coreas) {
         bool near = false, forward = false;
         if (active) {
           fast::View const v = make_view(*(ObserverConst*)(coreas_observers + k), tile_begin, W);
-          near = fast::coreas_far<Homogeneous>(t, start, start_kind, end, end_kind, prop, v, tile, W, tally, forward);
+          near = fast::coreas_far<Homogeneous>(t, start, start_kind, end, end_kind, prop, v, tile, W,
+                                                {first + k, nullptr}, tally, forward);
         }
         std::uint32_t const entry =
             (i + threadIdx.x) | (k << kMemberShift) | (forward ? kForwardBit : 0u);
@@ -150,6 +153,8 @@ __global__ void __launch_bounds__(Block, Block == 256 ? 3 : 4) radio_fast_kernel
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ long long scan_scratch[Zhs ? Block / 64 : 1];
   __shared__ BlockTallies block;
+  constexpr std::uint32_t kBudgets = Zhs ? most_observers(Block) * kRanges : 1;
+  __shared__ Budget budgets[kBudgets];
   __shared__ std::uint32_t lists[Coreas ? Block / 64 : 1][Coreas ? kListEntries : 1];
 
   // the workgroup's chunk, observers [first, first + members) and window tile
@@ -177,13 +182,14 @@ __global__ void __launch_bounds__(Block, Block == 256 ? 3 : 4) radio_fast_kernel
     chunk_begin = seg.begin + chunk * L.chunk_size;
     chunk_end = chunk_begin + L.chunk_size < seg.end ? chunk_begin + L.chunk_size : seg.end;
     counters = L.counters + seg.slot;
-    count_valid = within == 0;
+    count_valid = L.count_valid && within == 0;
   }
   std::uint32_t const W = L.tile_bins;
   std::uint32_t const tile_begin = within % L.bin_tiles * W;  // below 2^31 bins (checked on the host)
   std::uint32_t const words = (Coreas ? 3 * W : 0) + (Zhs ? 3 * (W + 1) : 0);
   long long* const tiles = reinterpret_cast<long long*>(lds_raw);
   for (std::uint32_t i = threadIdx.x; i < members * words; i += Block) tiles[i] = 0;
+  if (threadIdx.x < kBudgets) budgets[threadIdx.x] = 0.;
   clear_tallies(block);
   __syncthreads();
 
@@ -192,11 +198,10 @@ __global__ void __launch_bounds__(Block, Block == 256 ? 3 : 4) radio_fast_kernel
   std::uint32_t* const entries = lists[Coreas ? threadIdx.x / 64 : 0];
   fast::Tally tally;
   project_chunk<Coreas, Zhs, Homogeneous, Block>(L, coreas_observers, zhs_observers, members, tile_begin, chunk_begin,
-                                                 chunk_end, tiles, count_valid, entries, tally);
+                                                 chunk_end, tiles, count_valid, entries, first, budgets, tally);
   unsigned long long const counts[5] = {tally.coreas, tally.zhs, tally.subtracks + tally.single_subtracks, tally.valid,
                                         tally.overflow};
-  double const abs_sums[2] = {tally.coreas_abs, tally.zhs_abs};
-  add_tallies<Coreas, Zhs>(block, counts, abs_sums);
+  add_tallies<Coreas, Zhs>(block, counts);
   __syncthreads();
 
   unsigned long long overflows = 0;
@@ -226,9 +231,10 @@ void launch_typed(ProjectionLaunch const& launch, std::uint32_t grid, hipStream_
   static bool attribute_set = false;
   if (!attribute_set) {
     C8MI_HIP(hipFuncSetAttribute(reinterpret_cast<void const*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 static_cast<int>(fast_dynamic_lds_limit(Coreas, Block))));
+                                 static_cast<int>(fast_dynamic_lds_limit(Coreas, Zhs, Block))));
     attribute_set = true;
   }
+  if (launch.group > most_observers(Block)) throw std::logic_error("radio: more observers than the workgroup takes");
   std::size_t const lds = launch.group * projection_lds_bytes(Coreas, Zhs, launch.tile_bins);
   hipLaunchKernelGGL(kernel, dim3(grid), dim3(Block), lds, stream, launch);
   C8MI_HIP(hipGetLastError());

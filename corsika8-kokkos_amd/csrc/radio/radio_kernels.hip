@@ -41,7 +41,6 @@ constexpr double kPi = 3.141592653589793238462643383279502884;
 constexpr double kEmConstant = 1. / (4. * kPi * kEps0 * kC);
 constexpr double kChargeEm = kE * kEmConstant;
 constexpr double kCoreasThreshold = 1.e-3;
-constexpr double kIntLimit = 9223372036854775808.;  // 2^63
 
 struct V3 {
   double x, y, z;
@@ -183,7 +182,7 @@ __device__ __forceinline__ Path propagate(PropagationDev const& p, V3 source, Ob
 // Per-thread tallies, folded into the block and then the global counters.
 struct Tally {
   unsigned long long coreas = 0, zhs = 0, subtracks = 0, valid = 0, overflow = 0;
-  double abs_sum = 0.;  // sum of |increments|: bounds every LDS partial sum
+  double abs_sum = 0.;  // sum of |increments|, for kThreadLimit
 };
 
 // LDS accumulator for one mode: `Fixed` selects int64 fixed point (the
@@ -195,25 +194,14 @@ struct Tile {
   std::uint32_t stride;  // bins per component row
   std::int32_t begin;    // first global bin of this tile
   std::int32_t bins;     // bins owned by this tile
+  std::uint32_t observer;  // what contributions past the thread's limit need
+  Budget* budgets;       // ZHS: of its ranges
 };
 
-// add_radio_fixed_point on an LDS cell; returns false on a non-representable
-// contribution (the reference's overflow case), in which case nothing is added.
-// Below 2^51 the round-to-nearest-even integer comes from adding 1.5 * 2^52
-// and reading the low mantissa bits: the same value as (long long) rint().
-__device__ __forceinline__ bool fixed_increment(double value, double scale, long long& inc,
-                                                double& abs_sum) {
-  double const scaled = value * scale;
-  double const magnitude = fabs(scaled);
-  if (magnitude < 2251799813685248.) {  // 2^51
-    double const shifted = scaled + 6755399441055744.;  // 1.5 * 2^52
-    inc = __double_as_longlong(shifted) - 0x4338000000000000LL;
-  } else {
-    if (!isfinite(scaled) || magnitude >= kIntLimit) return false;
-    inc = static_cast<long long>(rint(scaled));
-  }
-  abs_sum += magnitude;
-  return true;
+// Below 2^51 (kThreadLimit) the round-to-nearest-even integer comes from adding
+// 1.5 * 2^52 and reading the low mantissa bits: the same value as (long long) rint().
+__device__ __forceinline__ long long fixed_increment(double scaled) {
+  return __double_as_longlong(scaled + 6755399441055744.) - 0x4338000000000000LL;
 }
 
 template <class T>
@@ -243,20 +231,32 @@ __device__ __forceinline__ void add_field_sample(Obs const& o, double scale,
   std::int32_t const local = bin - tile.begin;
   if (local < 0 || local >= tile.bins) return;
   if constexpr (Fixed) {
-    long long ix = 0, iy = 0, iz = 0;
-    bool const vx = fixed_increment(c.x, scale, ix, tally.abs_sum);
-    bool const vy = fixed_increment(c.y, scale, iy, tally.abs_sum);
-    bool const vz = fixed_increment(c.z, scale, iz, tally.abs_sum);
-    if (vx) lds_add(tile.data + local, ix);
-    if (vy) lds_add(tile.data + tile.stride + local, iy);
-    if (vz) lds_add(tile.data + 2 * tile.stride + local, iz);
-    // Counter updates are value selects: a branch between two tally fields
-    // can become a store through a selected pointer, which pins the tally to
-    // scratch memory.
-    bool const valid = vx && vy && vz;
-    tally.overflow += valid ? 0ull : 1ull;
-    tally.coreas += valid ? 1ull : 0ull;
-    return;
+    V3 const v = vmul(c, scale);
+    double const magnitude = fabs(v.x) + fabs(v.y) + fabs(v.z);
+    tally.abs_sum += magnitude;
+    if (__builtin_expect(tally.abs_sum < kThreadLimit, 1)) {
+      lds_add(tile.data + local, fixed_increment(v.x));
+      lds_add(tile.data + tile.stride + local, fixed_increment(v.y));
+      lds_add(tile.data + 2 * tile.stride + local, fixed_increment(v.z));
+    } else {
+      Rows const waves = waveform_rows<false>(tile.observer);
+      double const vs[3] = {v.x, v.y, v.z};
+      bool valid = true;
+      unsigned long long overflows = 0;
+      for (int k = 0; k < 3; ++k) {
+        long long value = 0;
+        if (!round_increment(vs[k], value)) valid = false;
+        else if (magnitude < kThreadLimit)
+          overflows += add_watched(tile.data + k * tile.stride + local, waves.row + k * waves.stride + bin, value);
+        else overflows += checked_add(waves.row + k * waves.stride + bin, value);
+      }
+      // Counter updates are value selects: a branch between two tally fields
+      // can become a store through a selected pointer, which pins the tally to
+      // scratch memory.
+      tally.overflow += overflows + (valid ? 0ull : 1ull);
+      tally.coreas += valid ? 1ull : 0ull;
+      return;
+    }
   } else {
     lds_add(tile.data + local, c.x);
     lds_add(tile.data + tile.stride + local, c.y);
@@ -280,23 +280,36 @@ __device__ __forceinline__ std::int32_t add_potential_range(double scale,
   valid = true;
   if (lo >= hi) return 0;
   if constexpr (Fixed) {
-    long long ix = 0, iy = 0, iz = 0;
-    bool const vx = fixed_increment(c.x, scale, ix, tally.abs_sum);
-    bool const vy = fixed_increment(c.y, scale, iy, tally.abs_sum);
-    bool const vz = fixed_increment(c.z, scale, iz, tally.abs_sum);
-    if (vx) {
-      lds_add(tile.data + lo, ix);
-      lds_add(tile.data + hi, -ix);
+    V3 const v = vmul(c, scale);
+    double const magnitude = fabs(v.x) + fabs(v.y) + fabs(v.z);
+    tally.abs_sum += magnitude;
+    double const vs[3] = {v.x, v.y, v.z};
+    if (__builtin_expect(tally.abs_sum < kThreadLimit, 1)) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        long long const value = fixed_increment(vs[k]);
+        lds_add(tile.data + k * tile.stride + lo, value);
+        lds_add(tile.data + k * tile.stride + hi, -value);
+      }
+    } else {
+      bool const in_tile = tile_takes(tile.budgets, static_cast<std::uint32_t>(lo), static_cast<std::uint32_t>(hi - 1),
+                                      static_cast<std::uint32_t>(tile.bins), magnitude);
+      Rows const waves = waveform_rows<true>(tile.observer);
+      unsigned long long overflows = 0;
+      for (int k = 0; k < 3; ++k) {
+        long long value = 0;
+        if (!round_increment(vs[k], value)) {
+          valid = false;
+        } else if (in_tile) {
+          lds_add(tile.data + k * tile.stride + lo, value);
+          lds_add(tile.data + k * tile.stride + hi, -value);
+        } else {
+          long long* const wave = waves.row + k * waves.stride + tile.begin;
+          for (std::int32_t b = lo; b < hi; ++b) overflows += checked_add(wave + b, value);
+        }
+      }
+      tally.overflow += overflows;
     }
-    if (vy) {
-      lds_add(tile.data + tile.stride + lo, iy);
-      lds_add(tile.data + tile.stride + hi, -iy);
-    }
-    if (vz) {
-      lds_add(tile.data + 2 * tile.stride + lo, iz);
-      lds_add(tile.data + 2 * tile.stride + hi, -iz);
-    }
-    valid = vx && vy && vz;
   } else {
     lds_add(tile.data + lo, c.x);
     lds_add(tile.data + hi, -c.x);
@@ -432,8 +445,8 @@ __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double t
   double const end_bin = floor((d2 - o.start) * o.rate + 0.5);
   V3 const bperp = vcross(path.emit, vcross(t.beta, path.emit));
   double const den = 1. - n_source * bk;
+  V3 potential;  // of the last bin
   if (start_bin == end_bin) {
-    V3 potential;
     if (fabs(den) > 1.e-15) {
       double const fraction = fabs(d2 * o.rate - d1 * o.rate);
       potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
@@ -441,40 +454,38 @@ __device__ __forceinline__ void zhs_segment(V3 p1, V3 p2, double time1, double t
       double const fraction = (time2 - time1) * o.rate;
       potential = vmul(bperp, sign * t.constant * fraction / path.distance);
     }
-    add_potential_sample(o, scale, tile, d2, potential, tally);
-    return;
-  }
-  int const nb = static_cast<int>(end_bin - start_bin);
-  double fraction = fabs(start_bin + 0.5 - x1);
-  V3 potential;
-  potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
-  add_potential_sample(o, scale, tile, d1, potential, tally);
-  if (nb > 1) {
-    V3 const middle = vmul(bperp, (subdivided ? 1. : sign) * t.constant / (den * path.distance));
-    // Bins of the first and last middle sample, exactly as the per-bin loop
-    // computes them; in between the bins are consecutive.
-    double const b_first = nearest_bin((d1 + 1. / o.rate - o.start) * o.rate);
-    double const b_last = nearest_bin((d1 + static_cast<double>(nb - 1) / o.rate - o.start) * o.rate);
-    if (b_last - b_first == static_cast<double>(nb - 2)) {
-      double const lo = b_first < 0. ? 0. : b_first;
-      double const hi = b_last < o.nbins_d - 1. ? b_last : o.nbins_d - 1.;
-      if (lo <= hi) {
-        bool valid = true;
-        std::int32_t const added =
-            add_potential_range(scale, tile, static_cast<std::int32_t>(lo),
-                                static_cast<std::int32_t>(hi), middle, tally, valid);
-        unsigned long long const n = static_cast<unsigned long long>(added);
-        tally.zhs += valid ? n : 0ull;
-        tally.overflow += valid ? 0ull : n;
+  } else {
+    int const nb = static_cast<int>(end_bin - start_bin);
+    double fraction = fabs(start_bin + 0.5 - x1);
+    potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
+    add_potential_sample(o, scale, tile, d1, potential, tally);
+    if (nb > 1) {
+      V3 const middle = vmul(bperp, (subdivided ? 1. : sign) * t.constant / (den * path.distance));
+      // Bins of the first and last middle sample, exactly as the per-bin loop
+      // computes them; in between the bins are consecutive.
+      double const b_first = nearest_bin((d1 + 1. / o.rate - o.start) * o.rate);
+      double const b_last = nearest_bin((d1 + static_cast<double>(nb - 1) / o.rate - o.start) * o.rate);
+      if (b_last - b_first == static_cast<double>(nb - 2)) {
+        double const lo = b_first < 0. ? 0. : b_first;
+        double const hi = b_last < o.nbins_d - 1. ? b_last : o.nbins_d - 1.;
+        if (lo <= hi) {
+          bool valid = true;
+          std::int32_t const added =
+              add_potential_range(scale, tile, static_cast<std::int32_t>(lo),
+                                  static_cast<std::int32_t>(hi), middle, tally, valid);
+          unsigned long long const n = static_cast<unsigned long long>(added);
+          tally.zhs += valid ? n : 0ull;
+          tally.overflow += valid ? 0ull : n;
+        }
+      } else {
+        for (int index = 1; index < nb; ++index)
+          add_potential_sample(o, scale, tile, d1 + static_cast<double>(index) / o.rate, middle,
+                               tally);
       }
-    } else {
-      for (int index = 1; index < nb; ++index)
-        add_potential_sample(o, scale, tile, d1 + static_cast<double>(index) / o.rate, middle,
-                             tally);
     }
+    fraction = fabs((d2 - o.start) * o.rate + 0.5 - end_bin);
+    potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
   }
-  fraction = fabs((d2 - o.start) * o.rate + 0.5 - end_bin);
-  potential = vmul(bperp, sign * t.constant * fraction / (den * path.distance));
   add_potential_sample(o, scale, tile, d2, potential, tally);
 }
 
@@ -563,6 +574,7 @@ __global__ void __launch_bounds__(Block, 4) radio_exact_kernel(ProjectionLaunch 
   extern __shared__ __align__(16) unsigned char lds_raw[];
   __shared__ Acc scan_scratch[Zhs ? Block / 64 : 1];
   __shared__ BlockTallies block;
+  __shared__ Budget budgets[kRanges];
 
   std::uint32_t observer, bin_tile, within;
   std::uint64_t chunk_begin, chunk_end;
@@ -586,7 +598,7 @@ __global__ void __launch_bounds__(Block, 4) radio_exact_kernel(ProjectionLaunch 
     chunk_begin = seg.begin + chunk * L.chunk_size;
     chunk_end = chunk_begin + L.chunk_size < seg.end ? chunk_begin + L.chunk_size : seg.end;
     counters = L.counters + seg.slot;
-    first_observer_tile = within == 0;
+    first_observer_tile = L.count_valid && within == 0;
   }
 
   std::uint32_t const W = L.tile_bins;
@@ -594,6 +606,7 @@ __global__ void __launch_bounds__(Block, 4) radio_exact_kernel(ProjectionLaunch 
   Acc* const zhs_lds = coreas_lds + (Coreas ? 3 * W : 0);
   std::uint32_t const lds_count = (Coreas ? 3 * W : 0) + (Zhs ? 3 * (W + 1) : 0);
   for (std::uint32_t i = threadIdx.x; i < lds_count; i += blockDim.x) coreas_lds[i] = 0;
+  if (threadIdx.x < kRanges) budgets[threadIdx.x] = 0.;
   clear_tallies(block);
   __syncthreads();
 
@@ -610,9 +623,9 @@ __global__ void __launch_bounds__(Block, 4) radio_exact_kernel(ProjectionLaunch 
       tile_begin < nbins ? static_cast<std::uint32_t>(nbins - tile_begin < W ? nbins - tile_begin : W)
                          : 0u;
   Tile<Fixed> const ctile{coreas_lds, W, static_cast<std::int32_t>(tile_begin),
-                          static_cast<std::int32_t>(tile_bins)};
+                          static_cast<std::int32_t>(tile_bins), observer, budgets};
   Tile<Fixed> const ztile{zhs_lds, W + 1, static_cast<std::int32_t>(tile_begin),
-                          static_cast<std::int32_t>(tile_bins)};
+                          static_cast<std::int32_t>(tile_bins), observer, budgets};
 
   Tally ctally, ztally;
   for (std::uint64_t i = chunk_begin + threadIdx.x; i < chunk_end; i += blockDim.x) {
@@ -628,8 +641,7 @@ __global__ void __launch_bounds__(Block, 4) radio_exact_kernel(ProjectionLaunch 
   }
   unsigned long long const counts[5] = {ctally.coreas, ztally.zhs, ztally.subtracks, ctally.valid,
                                         ctally.overflow + ztally.overflow};
-  double const abs_sums[2] = {ctally.abs_sum, ztally.abs_sum};
-  add_tallies<Coreas, Zhs>(block, counts, abs_sums);
+  add_tallies<Coreas, Zhs>(block, counts);
   __syncthreads();
 
   if constexpr (Zhs) {
@@ -695,12 +707,22 @@ void launch_block(ProjectionLaunch const& launch, std::uint32_t block, hipStream
   }
 }
 
+// CoREAS and ZHS in one exact kernel need more registers than four waves a SIMD
+// leave, and a 2048-bin window two tiles: 6.1 ms against 3.3 for 5e5 tracks on 100
+// antennas. So there is none.
+template <bool Coreas, bool Zhs>
+void launch_exact(ProjectionLaunch const& launch, std::uint32_t block, hipStream_t stream, std::size_t lds,
+                  std::uint32_t grid) {
+  if constexpr (Coreas && Zhs) throw std::logic_error("radio: an exact projection takes its algorithms one by one");
+  else launch_block<Coreas, Zhs, true>(launch, block, stream, lds, grid);
+}
+
 template <bool Coreas, bool Zhs>
 void launch_modes(ProjectionLaunch const& launch, bool fixed, bool exact, std::uint32_t block,
                   hipStream_t stream, std::size_t lds, std::uint32_t grid) {
   // FP64 (non-deterministic) accumulation is offered in the exact form only.
   if (!fixed) launch_block<Coreas, Zhs, false>(launch, block, stream, lds, grid);
-  else if (exact) launch_block<Coreas, Zhs, true>(launch, block, stream, lds, grid);
+  else if (exact) launch_exact<Coreas, Zhs>(launch, block, stream, lds, grid);
   else launch_fast(launch, Coreas, Zhs, block, grid, stream);
 }
 

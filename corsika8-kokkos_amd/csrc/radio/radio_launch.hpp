@@ -25,19 +25,24 @@ inline constexpr std::size_t kPreferredWorkgroupLdsBytes = 53 * 1024;
 // Upper bound of a projection kernel's static LDS beside the pair lists: the
 // wave totals of the ZHS scan (16 x 8 B for 1024 threads), counters and sums.
 inline constexpr std::size_t kProjectionStaticLdsBytes = 256;
-// Pair lists of the fast CoREAS kernels, bytes per thread (512 per wave).
+// Pair lists of the fast CoREAS kernels, bytes per thread (512 per wave); budgets
+// of the fast ZHS kernels, bytes per observer.
 inline constexpr std::size_t kPairListBytesPerThread = 8;
+inline constexpr std::size_t kBudgetBytesPerObserver = 128;
+// Most observers of a group, and of a workgroup of so many threads: only one of
+// 1024 takes several.
+inline constexpr std::uint32_t kMaxGroup = 8;
+inline constexpr std::uint32_t most_observers(std::uint32_t threads) { return threads == 1024 ? kMaxGroup : 1; }
 // LDS of a CU; what a fast workgroup holds beside its window tiles, and the most
 // its tiles may take.
 inline constexpr std::size_t kCuLdsBytes = 160 * 1024;
-inline constexpr std::size_t fast_static_lds(bool coreas, std::uint32_t threads) {
-  return kProjectionStaticLdsBytes + (coreas ? kPairListBytesPerThread * threads : 0u);
+inline constexpr std::size_t fast_static_lds(bool coreas, bool zhs, std::uint32_t threads) {
+  return kProjectionStaticLdsBytes + (coreas ? kPairListBytesPerThread * threads : 0u) +
+         (zhs ? kBudgetBytesPerObserver * most_observers(threads) : 0u);
 }
-inline constexpr std::size_t fast_dynamic_lds_limit(bool coreas, std::uint32_t threads) {
-  return kCuLdsBytes - fast_static_lds(coreas, threads);
+inline constexpr std::size_t fast_dynamic_lds_limit(bool coreas, bool zhs, std::uint32_t threads) {
+  return kCuLdsBytes - fast_static_lds(coreas, zhs, threads);
 }
-// Most observers of a group.
-inline constexpr std::uint32_t kMaxGroup = 8;
 // Most tracks a workgroup takes (its tallies and lists use 32-bit words).
 inline constexpr std::uint64_t kMaxChunkTracks = std::uint64_t{1} << 27;
 // Tracks per workgroup the default chunking gives a batch large enough for

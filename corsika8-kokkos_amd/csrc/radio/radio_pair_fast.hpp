@@ -10,7 +10,7 @@
 //  * e x (e x b) = e (e.b) - b with the e.b of the Doppler factor, three fused
 //    multiply-adds instead of two cross products;
 //  * the fixed-point scale rides on the amplitude, so a sample's components are
-//    its increments; the three range checks are one comparison of their sum;
+//    its increments; their range checks are one comparison of the thread's sum;
 //  * the first, middle and last bins of a ZHS segment share their difference-array
 //    entries (four per component instead of six).
 // Arrival times stay at FP64 accuracy: a sample is a spike in one bin, and a delay
@@ -21,6 +21,7 @@
 
 #include <cstdint>
 
+#include "radio_block.hpp"
 #include "radio_device.hpp"
 
 namespace c8mi::radio::fast {
@@ -30,8 +31,6 @@ inline constexpr double kInvC = 1. / 299792458.;
 inline constexpr double kPi = 3.141592653589793238462643383279502884;
 inline constexpr double kChargeEm = 1.6021766208e-19 * (1. / (4. * kPi * 8.8541878128e-12 * kC));
 inline constexpr double kCoreasThreshold = 1.e-3;
-inline constexpr double kIntLimit = 9223372036854775808.;      // 2^63
-inline constexpr double kShiftLimit = 2251799813685248.;       // 2^51
 inline constexpr double kShift = 6755399441055744.;            // 1.5 * 2^52
 inline constexpr long long kShiftBits = 0x4338000000000000LL;  // its bit pattern
 
@@ -210,9 +209,16 @@ __device__ __forceinline__ double doppler(double index, V3 beta, V3 emit, double
 struct Tally {
   std::uint32_t coreas = 0, single_subtracks = 0, valid = 0;
   unsigned long long zhs = 0, subtracks = 0, overflow = 0;
-  double coreas_abs = 0., zhs_abs = 0.;  // sums of |increments|: bound every LDS partial sum
+  double coreas_abs = 0., zhs_abs = 0.;  // sums of |increments|, for kThreadLimit
 };
 
+// What an observer's contributions past the thread's limit need.
+struct Excess {
+  std::uint32_t observer;
+  Budget* budgets;  // ZHS: of the observer's ranges
+};
+
+// Round to nearest even below 2^51 (kThreadLimit): the same as rint.
 __device__ __forceinline__ long long increment(double scaled) {
   return __double_as_longlong(scaled + kShift) - kShiftBits;
 }
@@ -220,45 +226,35 @@ __device__ __forceinline__ void lds_add(long long* address, long long value) {
   atomicAdd(reinterpret_cast<unsigned long long*>(address), static_cast<unsigned long long>(value));
 }
 
-// A component beyond the shift form: rounded by rint below 2^63, else refused.
-__device__ __forceinline__ bool checked_increment(double scaled, long long& inc, double& abs_sum) {
-  double const magnitude = fabs(scaled);
-  if (magnitude < kShiftLimit) {
-    inc = increment(scaled);
-  } else {
-    if (!(magnitude < kIntLimit)) return false;
-    inc = static_cast<long long>(rint(scaled));
-  }
-  abs_sum += magnitude;
-  return true;
-}
-
 // One CoREAS sample: scaled components c at arrival `time` (no sample outside
 // the window or the tile).
 __device__ __forceinline__ void add_field(View const& o, long long* tile, std::uint32_t stride, double time,
-                                          V3 c, Tally& tally) {
+                                          V3 c, Excess const& excess, Tally& tally) {
   if (!(time >= o.start && time <= o.end)) return;
   double const bin = floor(fma(time - o.start, o.rate, 0.5));
   if (!(bin >= o.tile_begin && bin < o.tile_end)) return;
   std::uint32_t const at = static_cast<std::uint32_t>(bin - o.tile_begin);
   double const magnitude = fabs(c.x) + fabs(c.y) + fabs(c.z);
-  if (magnitude < kShiftLimit) {
-    tally.coreas_abs += magnitude;
+  tally.coreas_abs += magnitude;
+  if (__builtin_expect(tally.coreas_abs < kThreadLimit, 1)) {
     lds_add(tile + at, increment(c.x));
     lds_add(tile + stride + at, increment(c.y));
     lds_add(tile + 2 * stride + at, increment(c.z));
     ++tally.coreas;
     return;
   }
-  long long ix = 0, iy = 0, iz = 0;
-  bool const vx = checked_increment(c.x, ix, tally.coreas_abs);
-  bool const vy = checked_increment(c.y, iy, tally.coreas_abs);
-  bool const vz = checked_increment(c.z, iz, tally.coreas_abs);
-  if (vx) lds_add(tile + at, ix);
-  if (vy) lds_add(tile + stride + at, iy);
-  if (vz) lds_add(tile + 2 * stride + at, iz);
-  bool const valid = vx && vy && vz;
-  tally.overflow += valid ? 0ull : 1ull;
+  Rows const waves = waveform_rows<false>(excess.observer);
+  long long* const wave = waves.row + static_cast<std::uint64_t>(bin);
+  double const cs[3] = {c.x, c.y, c.z};
+  bool valid = true;
+  unsigned long long overflows = 0;
+  for (int k = 0; k < 3; ++k) {
+    long long value = 0;
+    if (!round_increment(cs[k], value)) valid = false;
+    else if (magnitude < kThreadLimit) overflows += add_watched(tile + k * stride + at, wave + k * waves.stride, value);
+    else overflows += checked_add(wave + k * waves.stride, value);
+  }
+  tally.overflow += overflows + (valid ? 0ull : 1ull);
   tally.coreas += valid ? 1u : 0u;
 }
 
@@ -300,8 +296,8 @@ __device__ __forceinline__ V3 transverse(V3 emit, V3 beta, double beta_emit, dou
 template <bool Homogeneous>
 __device__ __forceinline__ bool coreas_far(Track const& t, Source const& start, std::uint32_t start_kind,
                                            Source const& end, std::uint32_t end_kind, PropagationDev const& p,
-                                           View const& o, long long* tile, std::uint32_t stride, Tally& tally,
-                                           bool& forward) {
+                                           View const& o, long long* tile, std::uint32_t stride,
+                                           Excess const& excess, Tally& tally, bool& forward) {
   Path const ps = propagate<Homogeneous>(p, o, start, start_kind);
   Path const pe = propagate<Homogeneous>(p, o, end, end_kind);
   double const bs = dot(t.beta, ps.emit), be = dot(t.beta, pe.emit);
@@ -326,15 +322,16 @@ __device__ __forceinline__ bool coreas_far(Track const& t, Source const& start, 
       separate_same_bin(start_receive, end_receive, o, false);
     }
   }
-  add_field(o, tile, stride, start_receive, fs, tally);
-  add_field(o, tile, stride, end_receive, fe, tally);
+  add_field(o, tile, stride, start_receive, fs, excess, tally);
+  add_field(o, tile, stride, end_receive, fe, excess, tally);
   return false;
 }
 
 // The CoREAS update near the Cherenkov angle: both samples from the midpoint.
 template <bool Homogeneous>
 __device__ __forceinline__ void coreas_near(Track const& t, PropagationDev const& p, View const& o,
-                                            long long* tile, std::uint32_t stride, Tally& tally, bool forward) {
+                                            long long* tile, std::uint32_t stride, Excess const& excess,
+                                            Tally& tally, bool forward) {
   std::uint32_t kind;
   Source const middle = make_source<Homogeneous>(p, midpoint(t), kind);
   Path const pm = propagate<Homogeneous>(p, o, middle, kind);
@@ -350,8 +347,8 @@ __device__ __forceinline__ void coreas_near(Track const& t, PropagationDev const
     f = scaled(f, fabs(delta * o.rate));
     separate_same_bin(start_receive, end_receive, o, true);
   }
-  add_field(o, tile, stride, start_receive, f, tally);
-  add_field(o, tile, stride, end_receive, {-f.x, -f.y, -f.z}, tally);
+  add_field(o, tile, stride, start_receive, f, excess, tally);
+  add_field(o, tile, stride, end_receive, {-f.x, -f.y, -f.z}, excess, tally);
 }
 
 // One component row of a ZHS segment over bins l1 (first), l1 + 1 .. l2 - 1
@@ -405,7 +402,8 @@ __device__ __forceinline__ Arrival segment_arrival(Path const& path, double inde
 // entries at the first bin and the two after it. u: e x (b x e) times the
 // amplitude over the distance.
 __device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival const& a, View const& o,
-                                                  long long* tile, std::uint32_t stride, Tally& tally) {
+                                                  long long* tile, std::uint32_t stride, Excess const& excess,
+                                                  Tally& tally) {
   bool const two = a.b1 != a.b2;
   double const k = reciprocal(fabs(a.den));
   std::int32_t const bins = static_cast<std::int32_t>(o.tile_end - o.tile_begin);
@@ -418,9 +416,9 @@ __device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival
   double const bound = (fabs(u.x) + fabs(u.y) + fabs(u.z)) * (fabs(first) + fabs(last));
   std::uint32_t const base = at > 0 ? static_cast<std::uint32_t>(at) : 0u;
   std::uint32_t const n = (has_first ? 1u : 0u) + (has_last ? 1u : 0u);
-  if (bound < kShiftLimit) {
-    tally.zhs_abs += bound;
-    double const us[3] = {u.x, u.y, u.z};
+  tally.zhs_abs += bound;
+  double const us[3] = {u.x, u.y, u.z};
+  if (__builtin_expect(tally.zhs_abs < kThreadLimit, 1)) {
 #pragma unroll
     for (int c = 0; c < 3; ++c) {
       long long* const row = tile + c * stride + base;
@@ -437,44 +435,47 @@ __device__ __forceinline__ void add_short_segment(V3 u, double duration, Arrival
     tally.zhs += n;
     return;
   }
-  double const us[3] = {u.x, u.y, u.z};
+  // the bins of the parts that are there (n of them, from `base` or the next on)
+  std::uint32_t const from = has_first ? base : static_cast<std::uint32_t>(at + 1);
+  bool const in_tile = n != 0 && tile_takes(excess.budgets, from, from + n - 1, static_cast<std::uint32_t>(bins), bound);
+  Rows const waves = waveform_rows<true>(excess.observer);
+  std::int64_t const bin = static_cast<std::int64_t>(o.tile_begin) + at;
   bool vf = true, vl = true;
+  unsigned long long overflows = 0;
   for (int c = 0; c < 3; ++c) {
     long long* const row = tile + c * stride;
-    long long f = 0, l = 0;
-    if (has_first) {
-      bool const ok = checked_increment(us[c] * first, f, tally.zhs_abs);
-      vf = vf && ok;
-      if (ok) {
-        lds_add(row + at, f);
-        lds_add(row + at + 1, -f);
+    long long* const wave = waves.row + c * waves.stride + bin;
+    auto add = [&](bool has, int ahead, double value, bool& valid) {
+      long long v = 0;
+      if (!has) return;
+      if (!round_increment(value, v)) {
+        valid = false;
+      } else if (in_tile) {
+        lds_add(row + at + ahead, v);
+        lds_add(row + at + ahead + 1, -v);
+      } else {
+        overflows += checked_add(wave + ahead, v);
       }
-    }
-    if (has_last) {
-      bool const ok = checked_increment(us[c] * last, l, tally.zhs_abs);
-      vl = vl && ok;
-      if (ok) {
-        lds_add(row + at + 1, l);
-        lds_add(row + at + 2, -l);
-      }
-    }
+    };
+    add(has_first, 0, us[c] * first, vf);
+    add(has_last, 1, us[c] * last, vl);
   }
   unsigned long long const nf = has_first ? 1ull : 0ull, nl = has_last ? 1ull : 0ull;
   tally.zhs += (vf ? nf : 0ull) + (vl ? nl : 0ull);
-  tally.overflow += (vf ? 0ull : nf) + (vl ? 0ull : nl);
+  tally.overflow += overflows + (vf ? 0ull : nf) + (vl ? 0ull : nl);
 }
 
 // One ZHS segment of any length. `subdivided` keeps the reference's sign of the
 // middle bins.
 __device__ __forceinline__ void zhs_segment(Path const& path, double index, double beta_emit, double time1,
                                             double time2, Track const& t, View const& o,
-                                            long long* tile, std::uint32_t stride, Tally& tally,
+                                            long long* tile, std::uint32_t stride, Excess const& excess, Tally& tally,
                                             bool subdivided) {
   Arrival const a = segment_arrival(path, index, beta_emit, time1, time2, o);
   if (!(a.b2 >= o.tile_begin && a.b1 < o.tile_end)) return;
   V3 const u = transverse(path.emit, t.beta, beta_emit, -(t.amplitude * path.inv_distance * o.scale));
   if (a.b2 - a.b1 <= 1.) {
-    add_short_segment(u, time2 - time1, a, o, tile, stride, tally);
+    add_short_segment(u, time2 - time1, a, o, tile, stride, excess, tally);
     return;
   }
   std::int32_t const bins = static_cast<std::int32_t>(o.tile_end - o.tile_begin);
@@ -482,26 +483,44 @@ __device__ __forceinline__ void zhs_segment(Path const& path, double index, doub
   std::int32_t const l1 = static_cast<std::int32_t>(fmax(a.b1 - o.tile_begin, -2.));
   std::int32_t const l2 = static_cast<std::int32_t>(fmin(a.b2 - o.tile_begin, static_cast<double>(bins) + 1.));
   V3 const edge = scaled(u, reciprocal(fabs(a.den)));
-  double const first = fabs(a.b1 + 0.5 - a.x1), last = fabs(a.x2 + 0.5 - a.b2);
-  double const sign = subdivided && a.den < 0. ? -1. : 1.;
   bool const has_first = l1 >= 0, has_last = l2 < bins;
   std::int32_t const middle_bins = (l2 < bins ? l2 : bins) - (l1 + 1 > 0 ? l1 + 1 : 0);
   bool const has_middle = l2 - l1 > 1 && middle_bins > 0;
-  double const es[3] = {edge.x, edge.y, edge.z};
-  bool vf = true, vm = true, vl = true;
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    // a part without bins in this tile takes no part in the sums
-    long long f = 0, m = 0, l = 0;
-    if (has_first && !checked_increment(es[c] * first, f, tally.zhs_abs)) vf = false;
-    if (has_middle && !checked_increment(es[c] * sign, m, tally.zhs_abs)) vm = false;
-    if (has_last && !checked_increment(es[c] * last, l, tally.zhs_abs)) vl = false;
-    add_segment_row(tile + c * stride, bins, l1, l2, f, m, l);
-  }
+  // a part without bins in this tile takes no part in the sums
+  double const first = has_first ? fabs(a.b1 + 0.5 - a.x1) : 0.;
+  double const middle = has_middle ? (subdivided && a.den < 0. ? -1. : 1.) : 0.;
+  double const last = has_last ? fabs(a.x2 + 0.5 - a.b2) : 0.;
   unsigned long long const nm = has_middle ? static_cast<unsigned long long>(middle_bins) : 0ull;
   unsigned long long const nf = has_first ? 1ull : 0ull, nl = has_last ? 1ull : 0ull;
+  double const bound = (fabs(edge.x) + fabs(edge.y) + fabs(edge.z)) * (first + fabs(middle) + last);
+  tally.zhs_abs += bound;
+  double const es[3] = {edge.x, edge.y, edge.z};
+  if (__builtin_expect(tally.zhs_abs < kThreadLimit, 1)) {
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+      add_segment_row(tile + c * stride, bins, l1, l2, increment(es[c] * first), increment(es[c] * middle),
+                      increment(es[c] * last));
+    tally.zhs += nf + nm + nl;
+    return;
+  }
+  std::int32_t const from = l1 > 0 ? l1 : 0, to = l2 < bins ? l2 : bins - 1;
+  Rows const waves = waveform_rows<true>(excess.observer);
+  std::int64_t const begin = static_cast<std::int64_t>(o.tile_begin);
+  bool vf = true, vm = true, vl = true;
+  unsigned long long overflows = 0;
+  for (int c = 0; c < 3; ++c) {
+    long long f = 0, m = 0, l = 0;
+    vf = round_increment(es[c] * first, f) && vf;
+    vm = round_increment(es[c] * middle, m) && vm;
+    vl = round_increment(es[c] * last, l) && vl;
+    long long* const wave = waves.row + c * waves.stride + begin;
+    for (std::int32_t b = from; b <= to; ++b) {
+      long long const v = b == l1 ? f : b == l2 ? l : m;
+      if (v != 0) overflows += checked_add(wave + b, v);
+    }
+  }
   tally.zhs += (vf ? nf : 0ull) + (vm ? nm : 0ull) + (vl ? nl : 0ull);
-  tally.overflow += (vf ? 0ull : nf) + (vm ? 0ull : nm) + (vl ? 0ull : nl);
+  tally.overflow += overflows + (vf ? 0ull : nf) + (vm ? 0ull : nm) + (vl ? 0ull : nl);
 }
 
 // The Fraunhofer measure of a track (RadioProjection.inl:482-529): above one it
@@ -516,14 +535,14 @@ __device__ __forceinline__ double fraunhofer(Path const& path, double beta_emit,
 template <bool Homogeneous>
 __device__ __forceinline__ void zhs_update(Track const& t, Source const& middle, std::uint32_t kind, double length2,
                                            PropagationDev const& p, std::uint32_t refinement, View const& o,
-                                           long long* tile, std::uint32_t stride, Tally& tally,
-                                           bool count_subtracks) {
+                                           long long* tile, std::uint32_t stride, Excess const& excess,
+                                           Tally& tally, bool count_subtracks) {
   Path const mp = propagate<Homogeneous>(p, o, middle, kind);
   double const bm = dot(t.beta, mp.emit);
   double const measure = fraunhofer(mp, bm, t.duration, length2, o);
   if (!(measure > 1.) && refinement <= 1u) {
     if (count_subtracks) ++tally.single_subtracks;
-    zhs_segment(mp, middle.index, bm, t.t0, t.t1, t, o, tile, stride, tally, false);
+    zhs_segment(mp, middle.index, bm, t.t0, t.t1, t, o, tile, stride, excess, tally, false);
     return;
   }
   double divisor = 1.;
@@ -550,7 +569,7 @@ __device__ __forceinline__ void zhs_update(Track const& t, Source const& middle,
     Source const part =
         make_source<Homogeneous>(p, {(p1.x + p2.x) * 0.5, (p1.y + p2.y) * 0.5, (p1.z + p2.z) * 0.5}, part_kind);
     Path const path = propagate<Homogeneous>(p, o, part, part_kind);
-    zhs_segment(path, part.index, dot(t.beta, path.emit), time1, time2, t, o, tile, stride, tally, true);
+    zhs_segment(path, part.index, dot(t.beta, path.emit), time1, time2, t, o, tile, stride, excess, tally, true);
     p1 = p2;
     time1 = time2;
   }

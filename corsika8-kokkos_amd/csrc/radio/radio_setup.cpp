@@ -160,7 +160,7 @@ void shape_fast(ProjectionLaunch& L, bool coreas, bool zhs, std::uint64_t observ
                 std::uint64_t count) {
   auto const tile_bytes = [&](std::uint64_t tile) { return projection_lds_bytes(coreas, zhs, static_cast<std::uint32_t>(tile)); };
   std::size_t const per_bin = (coreas ? 3u : 0u) + (zhs ? 3u : 0u);
-  std::size_t const most_lds = fast_dynamic_lds_limit(coreas, 1024);
+  std::size_t const most_lds = fast_dynamic_lds_limit(coreas, zhs, 1024);
   std::uint64_t const capacity = (most_lds / sizeof(long long) - (zhs ? 3u : 0u)) / per_bin;
   std::uint64_t const preferred = default_tile_capacity(per_bin, zhs);
   std::uint64_t const last_tiles = (bins + preferred - 1) / preferred;
@@ -187,7 +187,7 @@ void shape_fast(ProjectionLaunch& L, bool coreas, bool zhs, std::uint64_t observ
             L.bin_tiles = static_cast<std::uint32_t>(used);
             L.group = group;
             // two workgroups of one tile each share a CU; a large tile or a group takes it alone
-            L.block_threads = group == 1 && 2 * (tile_bytes(tile) + fast_static_lds(coreas, 512)) <= kCuLdsBytes ? 512u : 1024u;
+            L.block_threads = group == 1 && 2 * (tile_bytes(tile) + fast_static_lds(coreas, zhs, 512)) <= kCuLdsBytes ? 512u : 1024u;
             L.chunk_size = chunk;
           }
         }
@@ -210,7 +210,7 @@ void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std
       max_bins != 0 && count != 0) {
     shape_fast(L, coreas, zhs, observers, max_bins, count);
   } else {
-    std::size_t const words = (fast ? std::min(kMaxDynamicLdsBytes, fast_dynamic_lds_limit(coreas, L.block_threads))
+    std::size_t const words = (fast ? std::min(kMaxDynamicLdsBytes, fast_dynamic_lds_limit(coreas, zhs, L.block_threads))
                                     : kMaxDynamicLdsBytes) / sizeof(long long);
     std::size_t const per_bin = (coreas ? 3u : 0u) + (zhs ? 3u : 0u);
     std::uint64_t capacity = default_tile_capacity(per_bin, zhs);

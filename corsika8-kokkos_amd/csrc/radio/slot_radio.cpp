@@ -26,9 +26,9 @@ SlotRadio::SlotRadio(c8mi_radio_config const& config, std::uint32_t slots, std::
   config_.coreas_observers = config_.zhs_observers = nullptr;
   config_.coreas_observer_count = config_.zhs_observer_count = 0;
   total_bins_ = static_cast<std::uint64_t>(slots) * observers_per_slot * bins_per_observer;
-  // Both algorithms share every observer, so they share one launch.
-  fuse_ = config.coreas_enabled && config.zhs_enabled;
-  std::size_t const per_bin = (config.coreas_enabled ? 3u : 0u) + (config.zhs_enabled ? 3u : 0u);
+  // Both algorithms share every observer, so they share one launch (but for the exact form, which has none for both).
+  fuse_ = config.coreas_enabled && config.zhs_enabled && !config.exact_fp64;
+  std::size_t const per_bin = fuse_ ? 6u : 3u;
   std::uint64_t const capacity = default_tile_capacity(per_bin, config.zhs_enabled != 0);
   std::uint64_t const tiles = (bins_per_observer + capacity - 1) / capacity;
   tile_bins_ = static_cast<std::uint32_t>((bins_per_observer + tiles - 1) / tiles);
@@ -224,10 +224,14 @@ void SlotRadio::project(double const* tracks, std::uint64_t stride, std::uint64_
   }
   bool const exact = config_.exact_fp64 != 0;
   auto const g = static_cast<std::uint32_t>(grid);
+  L.count_valid = 1;  // in the first launch
   if (fuse_) {
     launch_pooled_projection(L, true, true, exact, g, stream_);
   } else {
-    if (config_.coreas_enabled) launch_pooled_projection(L, true, false, exact, g, stream_);
+    if (config_.coreas_enabled) {
+      launch_pooled_projection(L, true, false, exact, g, stream_);
+      L.count_valid = 0;
+    }
     if (config_.zhs_enabled) launch_pooled_projection(L, false, true, exact, g, stream_);
   }
   if (timing_) {
