@@ -231,12 +231,7 @@ ProjectionLaunch RadioAccumulator::base_launch(bool coreas, bool zhs, std::uint3
   L.zhs_refinement = config_.zhs_subtrack_refinement;
   L.propagation = propagation_;
   L.counters = counters_.data();
-  LaunchTuning tuning;
-  tuning.chunk_tracks = chunk_tracks_;
-  tuning.tile_bins_limit = tile_bins_limit_;
-  tuning.target_workgroups = target_workgroups_;
-  tuning.block_threads = block_threads_;
-  shape_projection(L, coreas, zhs, config_.deterministic && !config_.exact_fp64, observers, max_bins, count, tuning);
+  shape_projection(L, coreas, zhs, config_.deterministic && !config_.exact_fp64, observers, max_bins, count, tuning_);
   return L;
 }
 
@@ -375,15 +370,7 @@ void RadioAccumulator::download_fixed(std::int64_t* coreas, std::int64_t* zhs,
 void RadioAccumulator::set_tuning(std::uint64_t chunk_tracks, std::uint32_t tile_bins,
                                   std::uint32_t target_workgroups, std::uint32_t block_threads,
                                   bool split) {
-  std::uint32_t const block = block_threads == 0 ? kProjectionBlock : block_threads;
-  if (block != 256 && block != 512 && block != 1024)
-    throw std::invalid_argument("radio workgroup size must be 256, 512 or 1024");
-  if (chunk_tracks % block != 0)
-    throw std::invalid_argument("radio chunk size must be a multiple of the workgroup size");
-  chunk_tracks_ = chunk_tracks;
-  tile_bins_limit_ = tile_bins;
-  if (target_workgroups != 0) target_workgroups_ = target_workgroups;
-  block_threads_ = block;
+  tuning_ = make_tuning(chunk_tracks, tile_bins, target_workgroups, block_threads);
   split_ = split;
 }
 

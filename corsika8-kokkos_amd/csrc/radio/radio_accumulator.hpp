@@ -18,6 +18,7 @@
 #include "c8mi/c8mi_types.h"
 #include "../runtime.hpp"
 #include "radio_device.hpp"
+#include "radio_launch.hpp"
 
 namespace c8mi::radio {
 
@@ -142,13 +143,7 @@ class RadioAccumulator {
   PinnedBuffer<c8mi_lepton_transport_record> host_batch_;
   std::size_t host_count_ = 0;
 
-  std::uint64_t chunk_tracks_ = 0;     // 0: automatic
-  std::uint32_t tile_bins_limit_ = 0;  // 0: automatic
-  // Separate CoREAS and ZHS launches; about 8192 workgroups for the exact
-  // projection (48 KiB window tiles, 512 threads), measured on MI355X for 2^20
-  // tracks x 160 antennas x 2048 bins. The fast one's shape is estimated per launch.
-  std::uint32_t target_workgroups_ = 8192;
-  std::uint32_t block_threads_ = 0;  // 0: by the launch's shape
+  LaunchTuning tuning_;
   bool split_ = true;
 
   bool timing_ = false;

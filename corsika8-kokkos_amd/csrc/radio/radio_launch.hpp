@@ -11,7 +11,7 @@
 
 namespace c8mi::radio {
 
-// Default threads per projection workgroup (one observer x one track chunk);
+// Threads per workgroup of the pooled projection, and the least a workgroup has:
 // 256, 512 and 1024 are instantiated.
 inline constexpr std::uint32_t kProjectionBlock = 256;
 // Dynamic LDS a projection workgroup may request (gfx950: 160 KiB per CU).
@@ -60,19 +60,30 @@ inline std::uint64_t default_tile_capacity(std::size_t per_bin, bool zhs) {
   return preferred < most ? preferred : most;
 }
 
-// Launch-shape knobs of a projection (set_tuning): tracks per workgroup
-// (0 = automatic), window tile limit in bins (0 = automatic), target
-// workgroups per launch and threads per workgroup.
+// Launch-shape knobs of a projection (set_tuning), 0 = automatic: tracks per
+// workgroup, window tile limit in bins, target workgroups per launch and threads
+// per workgroup.
 struct LaunchTuning {
   std::uint64_t chunk_tracks = 0;
   std::uint32_t tile_bins_limit = 0;
-  std::uint32_t target_workgroups = 8192;
-  std::uint32_t block_threads = 0;  // 0: by the launch's shape
+  std::uint32_t target_workgroups = 0;
+  std::uint32_t block_threads = 0;
+  bool automatic() const noexcept {
+    return chunk_tracks == 0 && tile_bins_limit == 0 && target_workgroups == 0 && block_threads == 0;
+  }
 };
+// The knobs as a caller gives them; throws invalid_argument.
+LaunchTuning make_tuning(std::uint64_t chunk_tracks, std::uint32_t tile_bins, std::uint32_t target_workgroups,
+                         std::uint32_t block_threads);
+// What an automatic knob stands for where the shape isn't estimated (the exact
+// form, the fast one of both algorithms or with another knob given): about 8192 workgroups of 512
+// threads, measured for 2^20 tracks on 160 antennas with 2048 bins.
+inline constexpr std::uint32_t kDefaultWorkgroups = 8192, kDefaultThreads = 512;
 
 // Fills the shape fields of `L` (tile_bins, bin_tiles, chunk_size, chunks, group,
 // block_threads) for `count` tracks on `observers` observers whose longest window
-// has `max_bins` bins; `fast`: the fast kernels (groups of observers). Throws
+// has `max_bins` bins; `fast`: the fast kernels (an estimate gives their shape, with
+// groups of observers, for one algorithm while every knob is automatic). Throws
 // length_error when the grid exceeds 2^32 workgroups.
 void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std::uint32_t observers,
                       std::uint64_t max_bins, std::uint64_t count, LaunchTuning const& tuning);

@@ -156,10 +156,11 @@ constexpr double kRoundNs = 6000., kFlushNsPerBin = 4.;
 constexpr std::uint64_t kCus = 256;
 constexpr std::uint64_t kMaxRounds = 16;  // chunk counts tried: up to so many workgroups a CU
 
-void shape_fast(ProjectionLaunch& L, bool coreas, bool zhs, std::uint64_t observers, std::uint64_t bins,
+void shape_fast(ProjectionLaunch& L, bool zhs, std::uint64_t observers, std::uint64_t bins,
                 std::uint64_t count) {
+  bool const coreas = !zhs;
   auto const tile_bytes = [&](std::uint64_t tile) { return projection_lds_bytes(coreas, zhs, static_cast<std::uint32_t>(tile)); };
-  std::size_t const per_bin = (coreas ? 3u : 0u) + (zhs ? 3u : 0u);
+  constexpr std::size_t per_bin = 3;
   std::size_t const most_lds = fast_dynamic_lds_limit(coreas, zhs, 1024);
   std::uint64_t const capacity = (most_lds / sizeof(long long) - (zhs ? 3u : 0u)) / per_bin;
   std::uint64_t const preferred = default_tile_capacity(per_bin, zhs);
@@ -174,8 +175,8 @@ void shape_fast(ProjectionLaunch& L, bool coreas, bool zhs, std::uint64_t observ
     for (std::uint32_t group = 1; group <= kMaxGroup && group <= observers; ++group) {
       if (group * tile_bytes(tile) > most_lds) break;
       std::uint64_t const per_chunk = (observers + group - 1) / group * used;
-      double const update = (coreas ? kCoreasNs * kCoreasShare[group - 1] : 0.) + (zhs ? kZhsNs * kZhsShare[group - 1] : 0.);
-      double const round = kRoundNs + kFlushNsPerBin * static_cast<double>(group * tile * ((coreas ? 1u : 0u) + (zhs ? 1u : 0u)));
+      double const update = zhs ? kZhsNs * kZhsShare[group - 1] : kCoreasNs * kCoreasShare[group - 1];
+      double const round = kRoundNs + kFlushNsPerBin * static_cast<double>(group * tile);
       for (std::uint64_t chunks = kXcdCount;; chunks += kXcdCount) {
         std::uint64_t const chunk = (count + chunks - 1) / chunks;
         std::uint64_t const rounds = (per_chunk * chunks + kCus - 1) / kCus;
@@ -199,16 +200,29 @@ void shape_fast(ProjectionLaunch& L, bool coreas, bool zhs, std::uint64_t observ
 
 }  // namespace
 
+LaunchTuning make_tuning(std::uint64_t chunk_tracks, std::uint32_t tile_bins, std::uint32_t target_workgroups,
+                         std::uint32_t block_threads) {
+  if (block_threads != 0 && block_threads != 256 && block_threads != 512 && block_threads != 1024)
+    throw std::invalid_argument("radio workgroup size must be 256, 512 or 1024");
+  if (chunk_tracks % (block_threads ? block_threads : kProjectionBlock) != 0)
+    throw std::invalid_argument("radio chunk size must be a multiple of the workgroup size");
+  return {chunk_tracks, tile_bins, target_workgroups, block_threads};
+}
+
 void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std::uint32_t observers,
                       std::uint64_t max_bins, std::uint64_t count, LaunchTuning const& tuning) {
   // Window tile: the whole waveform when it fits the preferred LDS size, else
   // equal tiles of at most that size (a tuning limit may ask for others up to
   // the LDS budget).
-  L.block_threads = tuning.block_threads ? tuning.block_threads : 512;
+  // The fast form of both algorithms needs more than the 128 registers that 512
+  // threads leave: 256 (three waves a SIMD). Measured with 3e4 tracks on 160 antennas
+  // and 1024 bins, 262144 on 64 and 400, 5e5 on 100 and 2048: 0.20, 0.56 and 3.1 ms,
+  // in the estimated shape of 512 or 1024 threads 0.24, 0.43 and 3.5.
+  bool const fused = coreas && zhs;
+  L.block_threads = tuning.block_threads ? tuning.block_threads : fast && fused ? 256u : kDefaultThreads;
   L.group = 1;
-  if (fast && tuning.block_threads == 0 && tuning.chunk_tracks == 0 && tuning.tile_bins_limit == 0 && observers != 0 &&
-      max_bins != 0 && count != 0) {
-    shape_fast(L, coreas, zhs, observers, max_bins, count);
+  if (fast && !fused && tuning.automatic() && observers != 0 && max_bins != 0 && count != 0) {
+    shape_fast(L, zhs, observers, max_bins, count);
   } else {
     std::size_t const words = (fast ? std::min(kMaxDynamicLdsBytes, fast_dynamic_lds_limit(coreas, zhs, L.block_threads))
                                     : kMaxDynamicLdsBytes) / sizeof(long long);
@@ -228,7 +242,8 @@ void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std
     std::uint64_t chunk = tuning.chunk_tracks;
     if (chunk == 0) {
       std::uint64_t const per_chunk = std::max<std::uint64_t>(1, std::uint64_t(observers) * L.bin_tiles);
-      std::uint64_t const chunks_wanted = std::max<std::uint64_t>(1, tuning.target_workgroups / per_chunk);
+      std::uint64_t const target = tuning.target_workgroups ? tuning.target_workgroups : kDefaultWorkgroups;
+      std::uint64_t const chunks_wanted = std::max<std::uint64_t>(1, target / per_chunk);
       // a workgroup clears and flushes a whole window tile, so chunks of tens
       // of thousands of tracks pay (2^20 tracks on 160 antennas: 32768-track
       // chunks 1.2x faster than 16384, as fast as 65536)

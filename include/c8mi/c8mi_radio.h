@@ -90,14 +90,15 @@ int c8mi_radio_zhs_electric_field(const c8mi_radio_observer* observers, uint64_t
                                   const double* potential, double* field, double* times);
 
 /* TuningParameters (track/observer tiles, team size; TuningParameters.hpp)
- * analogue: tracks per workgroup (multiple of the workgroup size,
- * 0 = automatic), LDS window tile in bins (0 = automatic), target workgroups
- * per launch (0 = default 8192; used where the tracks per workgroup are
- * automatic), threads per workgroup (256, 512 or 1024; 0 = automatic) and
+ * analogue: tracks per workgroup (a multiple of the workgroup size), LDS window
+ * tile in bins, target workgroups per launch (used while the tracks per workgroup
+ * are automatic) and threads per workgroup (256, 512 or 1024), 0 = automatic each;
  * split: 1 runs fusable CoREAS+ZHS work as two launches (the default), 0 as one
- * fused launch (the exact fixed-point form has none and takes two). The fast
- * projection takes its whole shape (tile, observers and tracks per workgroup,
- * threads) from an estimate while tracks, tile and threads are automatic. Results do not depend on any of these. */
+ * fused launch (the exact fixed-point form has none and takes two). While all four
+ * are automatic, the fast projection of one algorithm takes its shape (tile,
+ * observers and tracks per workgroup, threads) from an estimate; elsewhere an
+ * automatic target is 8192 workgroups, and automatic threads are 512 (256 in the
+ * fast fused launch). Results do not depend on any of these. */
 int c8mi_radio_set_tuning(c8mi_radio* radio, uint64_t chunk_tracks, uint32_t tile_bins,
                           uint32_t target_workgroups, uint32_t block_threads, int split);
 
