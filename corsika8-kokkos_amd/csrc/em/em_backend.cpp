@@ -735,6 +735,32 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
     if (slot_radio_) slot_radio_->check_project(m, slot_radio_->chunk_for(m), active_range_ * kMaxRuns);
   }
   resize_scratch(m);
+  int const track_buffer = track_parity_;
+  // An attached accumulator alone gathers the fronts' tracks into its own
+  // batches (a front's 1e2 to 1e5 tracks leave the projection's workgroups with a
+  // window to clear and flush for few tracks each, and its launches hold up the
+  // next front's kernels: 10 TeV with 160 antennas 0.36 -> 0.30 s, whose groups of
+  // observers launched front by front took 0.31 where one observer a workgroup took 0.28).
+  bool const batched = radio_ && !slot_radio_ && !photon;
+  double* tracks = nullptr;
+  std::uint64_t track_stride = 0;
+  if (batched) {
+    tracks = radio_->reserve_tracks(m, track_stride);
+  } else if ((radio_ || slot_radio_) && !photon) {
+    // tracks [9][n]
+    std::uint64_t& capacity = track_capacity_[track_buffer];
+    if (capacity < m) {
+      if (track_busy_[track_buffer]) C8MI_HIP(hipEventSynchronize(track_done_[track_buffer]));
+      if (slot_busy_[track_buffer]) C8MI_HIP(hipEventSynchronize(slot_done_[track_buffer]));
+      track_busy_[track_buffer] = slot_busy_[track_buffer] = false;
+      std::uint64_t const grown = std::max<std::uint64_t>(m, 2 * capacity);
+      capacity = 0;
+      tracks_[track_buffer].allocate(C8MI_RADIO_TRACK_FIELDS * grown);
+      capacity = grown;
+    }
+    tracks = tracks_[track_buffer].data();
+    track_stride = m;
+  }
   commit();
   ParticleQueue const cur = queues_[s][current_[s]]->view();
   ParticleQueue const alt = queues_[s][1 - current_[s]]->view();
@@ -796,29 +822,14 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
   f.open_vertex_count = open_vertex_count_.data();
   f.first_interactions = first_interactions_.data();
   f.first_candidates = first_candidates_.data();
-  int const track_buffer = track_parity_;
-  // An attached accumulator alone gathers the fronts' tracks into its own
-  // batches (a front's 1e2 to 1e5 tracks leave the projection's workgroups with a
-  // window to clear and flush for few tracks each, and its launches hold up the
-  // next front's kernels: 10 TeV with 160 antennas 0.36 -> 0.30 s, whose groups of
-  // observers launched front by front took 0.31 where one observer a workgroup took 0.28).
-  bool const batched = radio_ && !slot_radio_ && !photon;
+  f.tracks = tracks;
+  f.track_stride = track_stride;
+  // the buffer's previous projections must be done first
   if (batched) {
-    f.tracks = radio_->reserve_tracks(m, f.track_stride, stream_);
-  } else if ((radio_ || slot_radio_) && !photon) {
-    // tracks [9][n]; the buffer's previous projections must be done first
-    std::uint64_t& capacity = track_capacity_[track_buffer];
-    if (capacity < m) {
-      if (track_busy_[track_buffer]) C8MI_HIP(hipEventSynchronize(track_done_[track_buffer]));
-      if (slot_busy_[track_buffer]) C8MI_HIP(hipEventSynchronize(slot_done_[track_buffer]));
-      track_busy_[track_buffer] = slot_busy_[track_buffer] = false;
-      capacity = std::max<std::uint64_t>(m, 2 * capacity);
-      tracks_[track_buffer].allocate(C8MI_RADIO_TRACK_FIELDS * capacity);
-    }
+    radio_->await_reserved(stream_);
+  } else if (tracks) {
     if (track_busy_[track_buffer]) C8MI_HIP(hipStreamWaitEvent(stream_, track_done_[track_buffer], 0));
     if (slot_busy_[track_buffer]) C8MI_HIP(hipStreamWaitEvent(stream_, slot_done_[track_buffer], 0));
-    f.tracks = tracks_[track_buffer].data();
-    f.track_stride = m;
   }
   // Projects this front's tracks on the accumulators' streams once the step kernel is done.
   auto project_tracks = [&] {

@@ -98,7 +98,7 @@ RadioAccumulator::~RadioAccumulator() {
 void RadioAccumulator::reset() {
   if (host_count_ != 0)
     throw std::logic_error("cannot reset radio with uncommitted host tracks");
-  for (auto& b : batches_) b.count = 0;  // their waveforms would be cleared here
+  for (auto& b : batches_) b.count = b.done = 0;  // their waveforms would be cleared here
   if (coreas_fixed_.size())
     C8MI_HIP(hipMemsetAsync(coreas_fixed_.data(), 0, coreas_fixed_.bytes(), stream_));
   if (zhs_fixed_.size())
@@ -173,7 +173,7 @@ void RadioAccumulator::accumulate_tracks(double const* device_tracks, std::uint6
   project(device_tracks, stride, count);
 }
 
-double* RadioAccumulator::reserve_tracks(std::uint64_t count, std::uint64_t& stride, hipStream_t producer) {
+double* RadioAccumulator::reserve_tracks(std::uint64_t count, std::uint64_t& stride) {
   if (sealed_) throw std::logic_error("radio endpoint already committed; reset before new tracks");
   if (batches_[batch_].count + count > batches_[batch_].capacity) {
     project_batch();
@@ -182,14 +182,19 @@ double* RadioAccumulator::reserve_tracks(std::uint64_t count, std::uint64_t& str
   TrackBatch& b = batches_[batch_];
   if (b.capacity < count) {
     if (b.recorded) C8MI_HIP(hipEventSynchronize(b.projected));
+    std::uint64_t const capacity = std::max({count, 2 * b.capacity, kBatchTracks});
     b.capacity = 0;
-    b.tracks.allocate(C8MI_RADIO_TRACK_FIELDS * std::max(count, kBatchTracks));
-    b.capacity = std::max(count, kBatchTracks);
+    b.tracks.allocate(C8MI_RADIO_TRACK_FIELDS * capacity);
+    b.capacity = capacity;
   }
   if (!b.projected) C8MI_HIP(hipEventCreateWithFlags(&b.projected, hipEventDisableTiming));
-  if (b.recorded) C8MI_HIP(hipStreamWaitEvent(producer, b.projected, 0));
   stride = b.capacity;
   return b.tracks.data() + b.count;
+}
+
+void RadioAccumulator::await_reserved(hipStream_t producer) const {
+  TrackBatch const& b = batches_[batch_];
+  if (b.recorded) C8MI_HIP(hipStreamWaitEvent(producer, b.projected, 0));
 }
 
 void RadioAccumulator::commit_tracks(std::uint64_t count, hipEvent_t written) {
@@ -201,9 +206,13 @@ void RadioAccumulator::commit_tracks(std::uint64_t count, hipEvent_t written) {
 void RadioAccumulator::project_batch() {
   TrackBatch& b = batches_[batch_];
   if (b.count == 0) return;
-  std::uint64_t const count = b.count;
-  b.count = 0;
-  project(b.tracks.data(), b.capacity, count);
+  // In as many launches as its size asks for: each front was small enough for one.
+  while (b.done < b.count) {
+    std::uint64_t const n = launchable(b.count - b.done, [this](std::uint64_t tracks) { check_shapes(tracks); });
+    project(b.tracks.data() + b.done, b.capacity, n);
+    b.done += n;
+  }
+  b.count = b.done = 0;
   C8MI_HIP(hipEventRecord(b.projected, stream_));
   b.recorded = true;
 }
@@ -211,7 +220,10 @@ void RadioAccumulator::project_batch() {
 void RadioAccumulator::check_accumulate(std::uint64_t count) const {
   if (count == 0) return;
   if (sealed_) throw std::logic_error("radio endpoint already committed; reset before new tracks");
-  // the launch shapes project() will build (they throw on oversized batches)
+  check_shapes(count);
+}
+
+void RadioAccumulator::check_shapes(std::uint64_t count) const {
   bool const coreas = !coreas_host_.empty(), zhs = !zhs_host_.empty();
   if (one_launch()) {
     (void)base_launch(true, true, static_cast<std::uint32_t>(coreas_host_.size()),
@@ -370,7 +382,9 @@ void RadioAccumulator::download_fixed(std::int64_t* coreas, std::int64_t* zhs,
 void RadioAccumulator::set_tuning(std::uint64_t chunk_tracks, std::uint32_t tile_bins,
                                   std::uint32_t target_workgroups, std::uint32_t block_threads,
                                   bool split) {
-  tuning_ = make_tuning(chunk_tracks, tile_bins, target_workgroups, block_threads);
+  LaunchTuning const tuning = make_tuning(chunk_tracks, tile_bins, target_workgroups, block_threads);
+  project_batch();  // in the shape its tracks were accepted for
+  tuning_ = tuning;
   split_ = split;
 }
 

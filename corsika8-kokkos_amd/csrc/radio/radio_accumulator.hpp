@@ -58,12 +58,15 @@ class RadioAccumulator {
   // launching anything (callers check before work that cannot be undone).
   void check_accumulate(std::uint64_t count) const;
   // Tracks of a producer on another stream, gathered into batches large enough to
-  // fill the chip: room for `count` tracks in the accumulator's own buffer
-  // ([9][stride], valid until the next reserve or download), which `producer`
-  // then writes and commits with an event recorded behind its writes. A full
-  // batch is projected at once, the last by download, download_fixed or
-  // kernel_time_ms.
-  double* reserve_tracks(std::uint64_t count, std::uint64_t& stride, hipStream_t producer);
+  // fill the chip: room for `count` tracks (which check_accumulate has passed) in
+  // the accumulator's own buffer ([9][stride], valid until the next reserve or
+  // download). The producer waits for the buffer (await_reserved), writes and
+  // commits with an event recorded behind its writes. A full batch is projected by
+  // the reserve that finds it so, the last by download, download_fixed, set_tuning
+  // or kernel_time_ms. What the projection or the buffer's allocation throws,
+  // reserve throws before the producer has done anything; no track is lost by it.
+  double* reserve_tracks(std::uint64_t count, std::uint64_t& stride);
+  void await_reserved(hipStream_t producer) const;
   void commit_tracks(std::uint64_t count, hipEvent_t written);
 
   // Decoded waveforms, [3][total_bins] per algorithm (x, y, z blocks). Either
@@ -93,6 +96,8 @@ class RadioAccumulator {
  private:
   void project(double const* tracks, std::uint64_t stride, std::uint64_t count);
   void project_batch();
+  // Throws length_error if the launches of so many tracks would be too large.
+  void check_shapes(std::uint64_t count) const;
   // CoREAS and ZHS in one kernel: fusable, asked for, and not the exact form.
   bool one_launch() const noexcept { return fuse_ && !split_ && !(config_.deterministic && config_.exact_fp64); }
   void ensure_track_capacity(std::uint64_t count);
@@ -133,7 +138,7 @@ class RadioAccumulator {
   static constexpr std::uint64_t kBatchTracks = std::uint64_t{1} << 20;
   struct TrackBatch {
     DeviceBuffer<double> tracks;
-    std::uint64_t capacity = 0, count = 0;
+    std::uint64_t capacity = 0, count = 0, done = 0;  // done: projected (more than one launch)
     hipEvent_t projected = nullptr;
     bool recorded = false;
   };

@@ -5,6 +5,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <stdexcept>
 
 #include "c8mi/c8mi_types.h"
 #include "radio_device.hpp"
@@ -87,6 +88,20 @@ inline constexpr std::uint32_t kDefaultWorkgroups = 8192, kDefaultThreads = 512;
 // length_error when the grid exceeds 2^32 workgroups.
 void shape_projection(ProjectionLaunch& L, bool coreas, bool zhs, bool fast, std::uint32_t observers,
                       std::uint64_t max_bins, std::uint64_t count, LaunchTuning const& tuning);
+
+// `count` tracks, or the first of its halves, quarters, ... for which `check` (a
+// shape_projection of so many) does not throw length_error.
+template <class Check>
+std::uint64_t launchable(std::uint64_t count, Check const& check) {
+  for (;; count = (count + 1) / 2) {
+    try {
+      check(count);
+      return count;
+    } catch (std::length_error const&) {
+      if (count <= 1) throw;
+    }
+  }
+}
 
 // LDS bytes for one workgroup holding `tile_bins` bins of each enabled mode.
 std::size_t projection_lds_bytes(bool coreas, bool zhs, std::uint32_t tile_bins);

@@ -33,6 +33,15 @@ extern "C" int shape(int coreas, int zhs, int fast, unsigned observers, unsigned
     return 2;
   }
 }
+// the tracks of `count` that a tuned CoREAS launch takes
+extern "C" unsigned long taken(unsigned observers, unsigned long bins, unsigned long count, unsigned long chunk,
+                               unsigned tile) {
+  LaunchTuning const tuning = make_tuning(chunk, tile, 0, 0);
+  return launchable(count, [&](std::uint64_t tracks) {
+    ProjectionLaunch L{};
+    shape_projection(L, true, false, true, observers, bins, tracks, tuning);
+  });
+}
 """
 
 
@@ -57,6 +66,7 @@ def shape(tmp_path_factory):
             return status
         return dict(zip(("tile_bins", "bin_tiles", "group", "threads", "chunk", "chunks"), out))
 
+    call.library = lib
     return call
 
 
@@ -99,3 +109,16 @@ def test_refused_knobs(shape):
     assert shape(True, 10, 100, 1000, tuning=dict(chunk_tracks=100)) == 1
     assert shape(True, 10, 100, 1000, tuning=dict(chunk_tracks=512, block_threads=1024)) == 1
     assert shape(True, 4096, 1 << 20, 1 << 24, tuning=dict(chunk_tracks=256, tile_bins=1)) == 2
+
+
+def test_a_list_too_large_for_one_launch(shape):
+    """A batch of fronts is projected in launches that 2^32 workgroups hold."""
+    taken = shape.library.taken
+    taken.restype = ctypes.c_ulong
+    n = lambda count, tile: taken(ctypes.c_uint(160), ctypes.c_ulong(65536), ctypes.c_ulong(count), ctypes.c_ulong(256),
+                                  ctypes.c_uint(tile))
+    per_chunk = 160 * 65536
+    got = n(1 << 20, 1)
+    assert got == 1 << 16 and got // 256 * per_chunk < 1 << 32 <= 2 * got // 256 * per_chunk
+    assert n(100000, 1) == 100000
+    assert n(1 << 20, 1000) == 1 << 20
