@@ -969,6 +969,7 @@ bool EmBackend::front(bool photon, c8mi_em_run_result& out) {
 void EmBackend::run(std::uint64_t maximum_rounds, c8mi_em_run_result& out) {
   std::memset(&out, 0, sizeof out);
   run_rounds_loop(maximum_rounds, out);
+  project_gathered_tracks();
   std::vector<unsigned long long> records(2u * slots_);
   C8MI_HIP(hipMemcpy(records.data(), record_counts_.data(), records.size() * sizeof(unsigned long long),
                      hipMemcpyDeviceToHost));
@@ -978,6 +979,12 @@ void EmBackend::run(std::uint64_t maximum_rounds, c8mi_em_run_result& out) {
   }
   pending(out.pending_photons, out.pending_leptons);
   out.next_history_id = slot_host_[0].call.counter;
+}
+
+// The call that makes the tracks projects them: none are left to the download. (Held
+// back to the end of a host handoff's many calls instead, 10 TeV took 208 ms against 194.)
+void EmBackend::project_gathered_tracks() {
+  if (radio_ && !slot_radio_) radio_->project_gathered();
 }
 
 // Rounds of the schedule: every shower's photon front (if its call runs one
@@ -1048,6 +1055,7 @@ void EmBackend::run_call(bool photon, c8mi_particle_state const* particles, std:
     throw;
   }
   c.resident = true;
+  project_gathered_tracks();
   out.wavefronts = c.call_fronts;
   out.transport_records = photon ? acc.photon_steps : acc.lepton_steps;
   out.interactions = photon ? acc.photon_interactions : acc.lepton_interactions;
@@ -1403,6 +1411,7 @@ void EmBackend::serve(c8mi_em_request const* requests, std::uint64_t count, c8mi
     }
     update_active_range();
   }
+  project_gathered_tracks();
   C8MI_HIP(hipStreamSynchronize(stream_));  // nothing may read `axes` after it is freed
 }
 

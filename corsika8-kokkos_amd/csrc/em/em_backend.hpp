@@ -171,6 +171,7 @@ class EmBackend {
   bool settle(CallState& c, std::uint64_t const n[2], c8mi_em_run_result& out) const;
   void reserve_call(CallState& c, int species, std::uint64_t n, c8mi_em_run_result& out) const;
   void run_rounds_loop(std::uint64_t maximum_rounds, c8mi_em_run_result& out);
+  void project_gathered_tracks();
   void flush_staged(int species);
   void add_medium(std::int32_t medium);
   std::uint32_t active_slot_count() const;

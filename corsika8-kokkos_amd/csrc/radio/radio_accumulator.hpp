@@ -62,12 +62,14 @@ class RadioAccumulator {
   // the accumulator's own buffer ([9][stride], valid until the next reserve or
   // download). The producer waits for the buffer (await_reserved), writes and
   // commits with an event recorded behind its writes. A full batch is projected by
-  // the reserve that finds it so, the last by download, download_fixed, set_tuning
-  // or kernel_time_ms. What the projection or the buffer's allocation throws,
-  // reserve throws before the producer has done anything; no track is lost by it.
+  // the reserve that finds it so, the last by project_gathered when the producer's
+  // run ends (after a run that failed by download, download_fixed, set_tuning or
+  // kernel_time_ms). What the projection or the buffer's allocation throws, reserve
+  // throws before the producer has done anything; no track is lost by it.
   double* reserve_tracks(std::uint64_t count, std::uint64_t& stride);
   void await_reserved(hipStream_t producer) const;
   void commit_tracks(std::uint64_t count, hipEvent_t written);
+  void project_gathered() { project_batch(); }
 
   // Decoded waveforms, [3][total_bins] per algorithm (x, y, z blocks). Either
   // output may be null. Throws OverflowError when the fixed-point range was

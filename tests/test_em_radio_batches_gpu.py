@@ -3,6 +3,8 @@ tracks each; the two buffers take turns), against per-shower radio, which projec
 front by itself: the increments of a track don't depend on the launch, and integers add up in
 any order, so the waveforms are equal bit for bit.
 """
+import time
+
 import numpy as np
 import pytest
 
@@ -148,3 +150,35 @@ def test_tuning_after_the_tracks(tables):
     assert downloads[0][2]["valid_tracks"] > 0 and downloads[0][0].any()
     assert downloads[0][2] == downloads[1][2]
     assert np.array_equal(downloads[0][0], downloads[1][0])
+
+
+@pytest.mark.parametrize("call", ["run", "run_lepton_wavefront"])
+def test_a_run_projects_its_tracks(tables, call):
+    """The download reads waveforms back; the projection (here many times longer than that,
+    64 segments a track) belongs to the run."""
+    atm = em.Atmosphere()
+    cfg = em.make_config(airtables, seed=7, atmosphere=atm, moliere=True, moliere_table=True)
+    observers, prop = np.concatenate([antennas(START, 128)] * 18)[:160], propagation()
+    dev = em.EmBackend(cfg, tables, atm)
+    radio = c8mi.RadioAccumulator(observers, prop, coreas=False, zhs_refinement=64, exact=True)
+    radio.enable_kernel_timing(True)
+    dev.attach_radio(radio)
+    if call == "run":
+        dev.begin_shower(11, 2)
+        dev.enqueue(em.particle(11, 100.0, START, DOWN, history_id=1))
+        dev.run()
+    else:
+        prim = electrons(3000)
+        prim["position_m"] = START
+        dev.begin_shower(11, 3001)
+        dev.run_lepton_wavefront(prim, 3001, 1 << 40, maximum_wavefronts=2)
+    time.sleep(1.0)
+    begin = time.perf_counter()
+    _, _, counters = radio.download_fixed()
+    seconds = time.perf_counter() - begin
+    ms, launches = radio.kernel_time()["zhs"]
+    dev.close()
+    radio.close()
+    print(f"{call}: {counters['valid_tracks']} tracks, projection {ms:.1f} ms, download {1e3 * seconds:.2f} ms", flush=True)
+    assert counters["valid_tracks"] > 2000 and ms > 10.0
+    assert 1e3 * seconds < 0.5 * ms
