@@ -160,16 +160,16 @@ __device__ __forceinline__ Path propagate(PropagationDev const& p, View const& o
   double const r2 = dot(d, d);
   r.inv_distance = reciprocal_sqrt(r2);
   r.emit = {d.x * r.inv_distance, d.y * r.inv_distance, d.z * r.inv_distance};
-  double const flight = (r2 * r.inv_distance) * kInvC;
+  double const distance = r2 * r.inv_distance;
   if constexpr (Homogeneous) {
-    r.time = s.index * flight;
+    r.time = s.index * distance * kInvC;  // the reference's order: see segment_arrival
     return r;
   }
   double const cells = s.height - o.destination_index;
   double const span = cells == 0. ? 1. : cells * p.step;
   double mean = fma(s.integrated - o.integrated_destination, reciprocal(span), 1.);
   if (kind != kInside) mean = edge_mean_index(o, s, kind);
-  r.time = mean * flight;
+  r.time = mean * (distance * kInvC);
   return r;
 }
 

@@ -161,41 +161,42 @@ def test_groups_of_observers_with_several_tiles(observers, bins, mode, index):
     assert got[2][mode + "_contributions"] == ref["counters"][mode + "_contributions"]
 
 
-@pytest.mark.parametrize("seed", [1, 2, 3])
-def test_arrival_times_round_as_the_oracles(seed):
+def test_arrival_times_round_as_the_oracles():
     """ZHS in ice, 1 km away: the two arrival times of a segment of 0.1 mm to 1 cm differ by 1e-16 s
     to 1e-12 s and are rounded to 8.5e-22 s each (2^-53 of 6e-6 s, half a unit), so a contribution
     carries a relative rounding of up to 1e-5. Evaluated in the oracle's order, fast times round
     as the oracle's unless the path's time, one square root apart, falls on the other side of a
     rounding boundary, and the contribution agrees to the errors of its other factors (ten operations
-    of 1.1e-16, below 1e-12 over 1 - n e.b of more than 1e-3): 81% of the bins do, 61% with a form that is equal in
-    exact arithmetic only (midpoint and spread; 5e-10 in the median). One segment a nanosecond, so
-    each has bins of its own."""
-    rng = np.random.default_rng(seed)
+    of 1.1e-16, below 1e-12 over 1 - n e.b of more than 1e-3): 83.7% of the bins do. With the index
+    multiplied after the division by c it was 81.5%, and 61% with a form that is equal in exact
+    arithmetic only (midpoint and spread). One segment a nanosecond, so each has bins of its own."""
     count, rate = 400, 1.0e10
-    tilt = rng.normal(0.0, 0.25, (2, count))
-    d = np.stack([tilt[0], tilt[1], -np.ones(count)])
-    d /= np.linalg.norm(d, axis=0)
-    length = 10.0 ** rng.uniform(-4.0, -2.0, count)
-    tracks = np.empty((9, count))
-    tracks[0:3] = rng.normal(0.0, 0.003, (3, count)) + [[0.0], [0.0], [-104.0]]
-    tracks[3:6] = tracks[0:3] + length * d
-    tracks[6] = 1.0e-9 * np.arange(count)
-    tracks[7] = tracks[6] + length / (rng.uniform(0.9, 1.0, count) * C)
-    tracks[8] = np.where(rng.random(count) < 0.6, -1.0, 1.0)
     obs = workloads.cherenkov_ring_observers(np.array([0.0, 0.0, -104.0]), (0.0, 0.0, -1.0), 1000.0, 1.78, count=8,
                                              sample_rate_hz=rate, number_of_bins=4096, pretrigger_s=2.0e-9)
     prop = c8mi.Propagation(homogeneous_index=1.78)
-    ref = oracle_lib.radio_project(prop, obs, tracks, coreas=False, threads=4)
-    want = ref["zhs_float"].reshape(3, obs.size, 4096)
-    limit = 1.0e3 * rate * np.abs(want).max()  # the int64 quantum is 2e-16 of the largest contribution
-    got = gpu_project(tracks, obs, prop, coreas=False, exact=False, limit=limit)
-    field = oracle_lib.radio_decode(got[1], obs, limit=limit, potential=True).reshape(want.shape)
-    size = np.linalg.norm(want, axis=0)
-    filled = size > 1e-6 * size.max()
-    assert filled.sum() > 0.8 * count * obs.size
-    error = np.linalg.norm(field - want, axis=0)[filled] / size[filled]
+    errors = []
+    for seed in (1, 2, 3):
+        rng = np.random.default_rng(seed)
+        tilt = rng.normal(0.0, 0.25, (2, count))
+        d = np.stack([tilt[0], tilt[1], -np.ones(count)])
+        d /= np.linalg.norm(d, axis=0)
+        length = 10.0 ** rng.uniform(-4.0, -2.0, count)
+        tracks = np.empty((9, count))
+        tracks[0:3] = rng.normal(0.0, 0.003, (3, count)) + [[0.0], [0.0], [-104.0]]
+        tracks[3:6] = tracks[0:3] + length * d
+        tracks[6] = 1.0e-9 * np.arange(count)
+        tracks[7] = tracks[6] + length / (rng.uniform(0.9, 1.0, count) * C)
+        tracks[8] = np.where(rng.random(count) < 0.6, -1.0, 1.0)
+        ref = oracle_lib.radio_project(prop, obs, tracks, coreas=False, threads=4)
+        want = ref["zhs_float"].reshape(3, obs.size, 4096)
+        limit = 1.0e3 * rate * np.abs(want).max()  # the int64 quantum is 2e-16 of the largest contribution
+        got = gpu_project(tracks, obs, prop, coreas=False, exact=False, limit=limit)
+        field = oracle_lib.radio_decode(got[1], obs, limit=limit, potential=True).reshape(want.shape)
+        size = np.linalg.norm(want, axis=0)
+        filled = size > 1e-6 * size.max()
+        assert filled.sum() > 0.8 * count * obs.size
+        errors.append(np.linalg.norm(field - want, axis=0)[filled] / size[filled])
+    error = np.concatenate(errors)
     alike = float(np.mean(error <= 1e-12))
-    print(f"seed {seed}: {alike:.3f} of {error.size} bins alike, median error {np.median(error):.1e}, largest {error.max():.1e}",
-          flush=True)
-    assert alike > 0.75
+    print(f"{alike:.4f} of {error.size} bins alike, median error {np.median(error):.1e}, largest {error.max():.1e}", flush=True)
+    assert alike > 0.828
