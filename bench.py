@@ -393,13 +393,15 @@ def em_section(showers, plain_showers, slots, cpu_seconds, no_cpu_baseline, ener
     # algorithmic bytes of all device particle-steps over the summed step-kernel time
     hbm_achieved = device_steps * EM_BYTES_PER_STEP / (step_kernel_ms * 1e-3) / 1e9
     # the "lepton_transport" timing covers the fused kernel, or with Molière its
-    # move, Molière, tail and finish kernels
+    # move, Molière, tail and finish kernels; "lepton_vertex" the vertex kernel, with
+    # Molière also the one that finishes and runs the vertices of small fronts
     tag = "true" if moliere_table else "false"
     transport_kernels = (["lepton_move_kernel", f"lepton_moliere_kernel<{tag}>", f"lepton_moliere_tail_kernel<{tag}>",
                           "lepton_finish_kernel", "lepton_finish_open_kernel"] if moliere
                          else ["lepton_transport_kernel"])
-    kernel_names = {"photon_step": ["photon_step_kernel"], "lepton_transport": transport_kernels,
-                    "lepton_vertex": ["lepton_vertex_kernel"]}[kind]
+    group_kernels = {"photon_step": ["photon_step_kernel"], "lepton_transport": transport_kernels,
+                     "lepton_vertex": ["lepton_vertex_kernel"] + (["lepton_finish_vertex_kernel"] if moliere else [])}
+    kernel_names = group_kernels[kind]
     kernel_name = "+".join(kernel_names)
     # The step kernels are bound by VALU issue (FP64 arithmetic with divergent
     # loops), not HBM: the roofline is the VALU issue rate of the dominant
@@ -409,8 +411,7 @@ def em_section(showers, plain_showers, slots, cpu_seconds, no_cpu_baseline, ener
     units = {"photon_step": totals["photon_steps"], "lepton_transport": totals["lepton_steps"],
              "lepton_vertex": totals["lepton_interactions"]}
     group_valu = {k: (sum(valu[n] for n in names) if all(n in valu for n in names) else None)
-                  for k, names in (("photon_step", ["photon_step_kernel"]), ("lepton_transport", transport_kernels),
-                                   ("lepton_vertex", ["lepton_vertex_kernel"]))}
+                  for k, names in group_kernels.items()}
     achieved = (group_valu[kind] * units[kind] / (timing[kind][0] * 1e-3) / 1e9
                 if group_valu[kind] is not None and timing[kind][0] > 0 else None)
     chip_valu = (sum(group_valu[k] * units[k] for k in step_kinds) / elapsed / 1e9

@@ -100,7 +100,7 @@ __device__ __forceinline__ EmContext const* stage_context(EmContext const* __res
 // before it reaches its coefficients, one dependent read after the other, and a
 // launch starts with cold caches (about 0.5 us a read): from LDS the walk costs a
 // tenth (100 GeV shower 79.3 -> 76.7 ms, pool of 1000 376 -> 366 ms). Arrays that don't fit the budget are read where they are.
-inline constexpr std::uint32_t kTableWords = 768;  // 6 KB: air takes 5.6, ice 3.4
+inline constexpr std::uint32_t kTableWords = 768;  // 6 KB: air takes 5.3, ice 3.6
 
 struct TableStage {
   long long* at;

@@ -145,9 +145,12 @@ __device__ __forceinline__ void project_chunk(ProjectionLaunch const& L, Observe
   }
 }
 
-// Four waves per SIMD (128 VGPRs); the pooled 256-thread form three (its two
-// tiles of an observer leave room for three workgroups a CU, and it holds the
-// endpoints and the midpoint of a track).
+// Four waves per SIMD (128 VGPRs); the 256-thread forms three (the pooled one's two
+// tiles of an observer leave room for three workgroups a CU up to 1090 bins, and it
+// holds the endpoints and the midpoint of a track: 168 VGPRs). Three such waves fill
+// a SIMD's registers, so the front kernels on other streams wait: the benchmark's
+// serving stream spends 1.1 s in scan and 0.53 s in scatter (0.37 and 0.34 beside
+// a 128-register kernel) while it gained 1.2x as a whole.
 template <bool Coreas, bool Zhs, bool Homogeneous, int Block>
 __global__ void __launch_bounds__(Block, Block == 256 ? 3 : 4) radio_fast_kernel(ProjectionLaunch L) {
   extern __shared__ __align__(16) unsigned char lds_raw[];

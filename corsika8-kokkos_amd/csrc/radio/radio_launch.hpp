@@ -17,14 +17,18 @@ namespace c8mi::radio {
 inline constexpr std::uint32_t kProjectionBlock = 256;
 // Dynamic LDS a projection workgroup may request (gfx950: 160 KiB per CU).
 inline constexpr std::size_t kMaxDynamicLdsBytes = 144 * 1024;
-// Default window tile: its dynamic LDS plus the kernel's static LDS stay within
-// this budget, so three workgroups share a CU (160 KiB). A 4096-bin ZHS window
-// in one 96 KiB tile (one workgroup per CU) measured 2x slower than two
-// 2048-bin tiles; a 1024-bin CoREAS+ZHS window (48 KiB of bins) and a 2048-bin
-// ZHS window keep one tile.
+// Default window tile: its dynamic LDS and kProjectionStaticLdsBytes stay within
+// this budget, so three workgroups of the exact kernels share a CU (160 KiB). A
+// 4096-bin ZHS window in one 96 KiB tile (one workgroup per CU) measured 2x slower
+// than two 2048-bin tiles; a 1024-bin CoREAS+ZHS window (48 KiB of bins) and a
+// 2048-bin ZHS window keep one tile. The fused pooled kernel has 2 KiB more static
+// LDS: with tiles of 1091 to 1124 bins two of its workgroups share a CU, which made
+// no difference (twelve served showers with windows of 1080 and 1110 bins 341 and
+// 340 ms, 2170 and 2230 353 and 353), where a second tile would evaluate every
+// update twice.
 inline constexpr std::size_t kPreferredWorkgroupLdsBytes = 53 * 1024;
-// Upper bound of a projection kernel's static LDS beside the pair lists: the
-// wave totals of the ZHS scan (16 x 8 B for 1024 threads), counters and sums.
+// Upper bound of a projection kernel's static LDS beside the pair lists and
+// budgets: the wave totals of the ZHS scan (16 x 8 B for 1024 threads) and counters.
 inline constexpr std::size_t kProjectionStaticLdsBytes = 256;
 // Pair lists of the fast CoREAS kernels, bytes per thread (512 per wave); budgets
 // of the fast ZHS kernels, bytes per observer.
