@@ -322,7 +322,8 @@ __global__ __launch_bounds__(kStepBlock, 3) void lepton_move_kernel(EmContext co
 // registers do not weigh on the rest of the step. The context is read from
 // global memory (its snapshot and table pointers are uniform, scalar loads).
 // One form per component count (N): a state of exactly the medium's components
-// stays in registers and runs no chain for an absent one, and the table's cubics
+// needs fewer registers (three with the table still take 96 B of scratch, four 128,
+// as all four always did) and runs no chain for an absent one, and the table's cubics
 // (four functions a component and iteration, a line of the L1 per lane each) are
 // read from LDS.
 template <bool Table, int N>
